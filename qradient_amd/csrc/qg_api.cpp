@@ -37,7 +37,7 @@ hipError_t simple_term_expec(int dtype, const void* v, int n, const PTerm* t, in
 hipError_t simple_sample_basis(int dtype, const void* v, int n, const int32_t* order, const double* u, int shots,
                                int32_t* idx, double* mass, hipStream_t st);
 constexpr int kDotBlocks = 512;
-hipError_t launch_fused(const void* descs, int batch, int n, hipStream_t st);
+hipError_t launch_fused(const void* descs, int batch, int n, int mode, int lut_w, hipStream_t st);
 hipError_t set_fused_attributes();
 size_t fused_desc_size();
 hipError_t noalloc_scratch_init(int device);
@@ -46,21 +46,26 @@ void* noalloc_scratch(int device);
 
 // Mirror of the device-side FusedDesc in qg_fused.hip (same layout).
 struct FusedDescH {
-  int32_t n, L, kind, ent;
+  int32_t n, L, ent;
   const int32_t* gtype;
-  const double* gcs;
-  const double* params;
+  const double* gab;
+  const double* gamma;
   const DTerm* dterms;
   int32_t ndterms;
   const DTerm* xy;
   int32_t nxy;
+  int32_t lut_w;
   uint32_t lad1, lad2;
+  uint32_t inv1, inv2;
   const double* init_tab;
   double* out;
   int32_t grad;
   int32_t psi_c64;
   void* psi_out;
 };
+// and of its FusedMode
+enum FusedMode : int32_t { FM_MCCLEAN = 0, FM_QAOA_LUT = 1, FM_QAOA_SINCOS = 2, FM_QAOA_LARGE = 3 };
+constexpr double kSincosMax = 67108864.0;  // phase angles below this take the reduced sincos (qg_math.hpp)
 }  // namespace qg
 
 using namespace qg;
@@ -427,6 +432,7 @@ struct qg_plan {
   size_t off_hist = 0, off_lam = 0, off_ini = 0, off_prep = 0;
   // small device tables
   uint32_t lad1 = 0, lad2 = 0;  // the ladder map in shift form (gather/scatter)
+  uint32_t inv1 = 0, inv2 = 0;  // and its inverse
   double* d_init = nullptr;     // n + 1
   DTerm* d_terms = nullptr;     // diagonal terms (max_terms)
   std::vector<DTerm> h_terms;   // host copy of what d_terms holds for the current run
@@ -1425,7 +1431,8 @@ static int mcclean_layout(qg_plan* p) {
   // static tables, staged in pinned memory and copied in stream order (the
   // previous run on this stream ended with a synchronisation, so the staging
   // is free and the tables are no longer read)
-  if (!ladder_shift_form(n, 1, &p->lad1, &p->lad2)) return fail(QG_ERR_INVALID, "ladder map not in shift form");
+  if (!ladder_shift_form(n, 1, &p->lad1, &p->lad2) || !ladder_shift_form(n, 0, &p->inv1, &p->inv2))
+    return fail(QG_ERR_INVALID, "ladder map not in shift form");
   double* hi = (double*)p->h_tabs;
   ry_init_table(n, hi);
   HIPCHK(hipMemcpyAsync(p->d_init, hi, sizeof(double) * (n + 1), hipMemcpyHostToDevice, p->ctx->stream));
@@ -1740,8 +1747,8 @@ static int ensure_arena(qg_plan* p, size_t bytes) {
 // Runs B circuits through the whole-circuit kernel.  The tables of circuit b
 // are written by fill(b, desc, arena); results land in out[b * per_out ...].
 template <class Fill>
-static int run_fused(qg_plan* p, int B, size_t bytes_per_circuit, int per_out, bool grad, void* psi_out, Fill fill,
-                     double* out) {
+static int run_fused(qg_plan* p, int B, int mode, int lut_w, size_t bytes_per_circuit, int per_out, bool grad,
+                     void* psi_out, Fill fill, double* out) {
   qg_ctx* c = p->ctx;
   const size_t need = (size_t)B * (bytes_per_circuit + 16 * 256 + sizeof(FusedDescH) + sizeof(double) * per_out);
   CHK(ensure_arena(p, need));
@@ -1757,6 +1764,9 @@ static int run_fused(qg_plan* p, int B, size_t bytes_per_circuit, int per_out, b
     h_desc[b].ent = p->ent;
     h_desc[b].lad1 = p->lad1;
     h_desc[b].lad2 = p->lad2;
+    h_desc[b].inv1 = p->inv1;
+    h_desc[b].inv2 = p->inv2;
+    h_desc[b].lut_w = lut_w;
     h_desc[b].init_tab = p->d_init;
     h_desc[b].out = d_out + (size_t)b * per_out;
     h_desc[b].grad = grad ? 1 : 0;
@@ -1766,7 +1776,7 @@ static int run_fused(qg_plan* p, int B, size_t bytes_per_circuit, int per_out, b
   }
   HIPCHK(hipMemcpyAsync(p->d_arena, p->h_arena, ar.used, hipMemcpyHostToDevice, c->stream));
   HIPCHK(hipEventRecord(c->ev0, c->stream));
-  HIPCHK(launch_fused(d_desc, B, p->n, c->stream));
+  HIPCHK(launch_fused(d_desc, B, p->n, mode, lut_w, c->stream));
   HIPCHK(hipEventRecord(c->ev1, c->stream));
   const int nout = grad ? per_out : 1;
   for (int b = 0; b < B && !grad; ++b)
@@ -1778,6 +1788,17 @@ static int run_fused(qg_plan* p, int B, size_t bytes_per_circuit, int per_out, b
   HIPCHK(hipEventElapsedTime(&p->last_ms, c->ev0, c->ev1));
   p->launches.clear();
   return QG_OK;
+}
+
+// The gate tables of a whole-circuit run: types, and the shear coefficients
+// set_gate stores.
+static void fused_gates(size_t np, const int32_t* axes, const double* angles, int32_t* type, double* ab) {
+  for (size_t k = 0; k < np; ++k) {
+    type[k] = axes[k] == 0 ? G_X : axes[k] == 1 ? G_Y : G_Z;
+    const GateAB g = gate_ab(angles[k], 1.0);
+    ab[2 * k] = g.a;
+    ab[2 * k + 1] = g.b;
+  }
 }
 
 static int obs_tables(const ObsSplit& obs, FusedDescH& d, Arena& ar) {
@@ -1811,21 +1832,16 @@ static int mcclean_run(qg_plan* p, const int32_t* axes, const double* angles, co
   qg_ctx* c = p->ctx;
   HIPCHK(hipSetDevice(c->device));
   if (p->fused && n <= kFusedMaxN && !ini_state) {
-    // the whole circuit in one workgroup (qg_fused.hip): gates as (type, cos, sin)
+    // the whole circuit in one workgroup (qg_fused.hip)
     std::vector<double> res(1 + (size_t)L * n);
     auto fill = [&](int, FusedDescH& d, Arena& ar) -> int {
-      d.kind = 0;
       int32_t* dt = nullptr;
       int32_t* ht = ar.take<int32_t>((size_t)L * n, &dt);
       double* dg = nullptr;
       double* hg = ar.take<double>((size_t)2 * L * n, &dg);
-      for (int k = 0; k < L * n; ++k) {
-        ht[k] = axes[k] == 0 ? G_X : axes[k] == 1 ? G_Y : G_Z;
-        hg[2 * k] = std::cos(0.5 * angles[k]);
-        hg[2 * k + 1] = std::sin(0.5 * angles[k]);
-      }
+      fused_gates((size_t)L * n, axes, angles, ht, hg);
       d.gtype = dt;
-      d.gcs = dg;
+      d.gab = dg;
       return obs_tables(obs, d, ar);
     };
     const size_t bytes = (size_t)L * n * 20 + (obs.diag.size() + obs.xy.size() + 2) * sizeof(DTerm);
@@ -1837,11 +1853,12 @@ static int mcclean_run(qg_plan* p, const int32_t* axes, const double* angles, co
       HIPCHK(hipMalloc(&p->d_fstate, ((size_t)16) << n));
       p->cap_fstate = (size_t)16 << n;
     }
-    CHK(run_fused(p, 1, bytes, 1 + L * n, grad, p->d_fstate, fill, res.data()));
+    CHK(run_fused(p, 1, FM_MCCLEAN, 0, bytes, 1 + L * n, grad, p->d_fstate, fill, res.data()));
     *E_out = res[0];
     if (grad) std::memcpy(grad_out, res.data() + 1, sizeof(double) * L * n);
     p->last_state_ptr = p->d_fstate;
     p->state_sign = false;
+    for (int k = 0; k < L * n; ++k) p->state_sign ^= gate_flips(angles[k], 1.0);
     return QG_OK;
   }
   if (!obs.xy.empty() && n > 31) return fail(QG_ERR_UNSUPPORTED, "observables with x/y terms need n <= 31");
@@ -1961,7 +1978,8 @@ static int mcclean_batch_layout(qg_plan* p) {
   const int ch = n > kFusedMaxN ? p->chunk : 1;
   p->nrows = ch * (P * L + 1) * (kMaxK + 1);
   CHK(ensure_small(p, ch * 2 * P * L, p->nrows, ch * (1 + L * n)));
-  if (!ladder_shift_form(n, 1, &p->lad1, &p->lad2)) return fail(QG_ERR_INVALID, "ladder map not in shift form");
+  if (!ladder_shift_form(n, 1, &p->lad1, &p->lad2) || !ladder_shift_form(n, 0, &p->inv1, &p->inv2))
+    return fail(QG_ERR_INVALID, "ladder map not in shift form");
   double* hi = (double*)p->h_tabs;
   ry_init_table(n, hi);
   HIPCHK(hipMemcpyAsync(p->d_init, hi, sizeof(double) * (n + 1), hipMemcpyHostToDevice, p->ctx->stream));
@@ -2017,25 +2035,18 @@ extern "C" int qg_mcclean_batch_grad_run(qg_plan* p, int B, const int32_t* axes,
     // the whole-circuit kernel, one workgroup per circuit, one launch
     std::vector<double> res((size_t)B * per_out);
     auto fill = [&](int b, FusedDescH& d, Arena& ar) -> int {
-      d.kind = 0;
       int32_t* dt = nullptr;
       int32_t* ht = ar.take<int32_t>(np, &dt);
       double* dg = nullptr;
       double* hg = ar.take<double>(2 * np, &dg);
-      const int32_t* ax = axes + (size_t)b * np;
-      const double* an = angles + (size_t)b * np;
-      for (size_t k = 0; k < np; ++k) {
-        ht[k] = ax[k] == 0 ? G_X : ax[k] == 1 ? G_Y : G_Z;
-        hg[2 * k] = std::cos(0.5 * an[k]);
-        hg[2 * k + 1] = std::sin(0.5 * an[k]);
-      }
+      fused_gates(np, axes + (size_t)b * np, angles + (size_t)b * np, ht, hg);
       d.gtype = dt;
-      d.gcs = dg;
+      d.gab = dg;
       d.psi_out = nullptr;
       return obs_tables(obs, d, ar);
     };
     const size_t bytes = np * 20 + (obs.diag.size() + 2) * sizeof(DTerm);
-    CHK(run_fused(p, B, bytes, per_out, true, nullptr, fill, res.data()));
+    CHK(run_fused(p, B, FM_MCCLEAN, 0, bytes, per_out, true, nullptr, fill, res.data()));
     for (int b = 0; b < B; ++b) {
       E_out[b] = res[(size_t)b * per_out];
       std::memcpy(grad_out + (size_t)b * np, res.data() + (size_t)b * per_out + 1, sizeof(double) * np);
@@ -2227,7 +2238,7 @@ extern "C" int qg_mcclean_grad_run_noalloc(qg_ctx* c, int n, int L, int entangle
   };
   const size_t o_desc = take(sizeof(FusedDescH));
   const size_t o_type = take(sizeof(int32_t) * np);
-  const size_t o_gcs = take(sizeof(double) * 2 * np);
+  const size_t o_gab = take(sizeof(double) * 2 * np);
   const size_t o_diag = take(sizeof(DTerm) * std::max(1, ndiag));
   const size_t o_xy = take(sizeof(DTerm) * std::max(1, nxy));
   const size_t o_init = take(sizeof(double) * (n + 1));
@@ -2240,14 +2251,8 @@ extern "C" int qg_mcclean_grad_run_noalloc(qg_ctx* c, int n, int L, int entangle
   unsigned char* dev = (unsigned char*)noalloc_scratch(c->device);
   if (!dev) return fail(QG_ERR_HIP, "qg_mcclean_grad_run_noalloc: no scratch address for this device");
   unsigned char* h = c->noalloc_host;
-  // gates as (type, cos, sin), as mcclean_run's whole-circuit tables
-  int32_t* ht = (int32_t*)(h + o_type);
-  double* hg = (double*)(h + o_gcs);
-  for (size_t k = 0; k < np; ++k) {
-    ht[k] = axes[k] == 0 ? G_X : axes[k] == 1 ? G_Y : G_Z;
-    hg[2 * k] = std::cos(0.5 * angles[k]);
-    hg[2 * k + 1] = std::sin(0.5 * angles[k]);
-  }
+  // gates as mcclean_run's whole-circuit tables
+  fused_gates(np, axes, angles, (int32_t*)(h + o_type), (double*)(h + o_gab));
   // observable, in split_observable's order
   DTerm* hd = (DTerm*)(h + o_diag);
   DTerm* hx = (DTerm*)(h + o_xy);
@@ -2261,23 +2266,25 @@ extern "C" int qg_mcclean_grad_run_noalloc(qg_ctx* c, int n, int L, int entangle
     else hx[ix++] = {bi, 1, t.w};
   }
   // the ladder's gather map and the RY(pi/4) table, as a McClean plan's
-  uint32_t lad1 = 0, lad2 = 0;
-  if (!ladder_shift_form(n, 1, &lad1, &lad2)) return fail(QG_ERR_INVALID, "ladder map not in shift form");
+  uint32_t lad1 = 0, lad2 = 0, inv1 = 0, inv2 = 0;
+  if (!ladder_shift_form(n, 1, &lad1, &lad2) || !ladder_shift_form(n, 0, &inv1, &inv2))
+    return fail(QG_ERR_INVALID, "ladder map not in shift form");
   ry_init_table(n, (double*)(h + o_init));
   FusedDescH* hdsc = (FusedDescH*)(h + o_desc);
   std::memset(hdsc, 0, sizeof(FusedDescH));
   hdsc->n = n;
   hdsc->L = L;
-  hdsc->kind = 0;
   hdsc->ent = entangler;
   hdsc->gtype = (const int32_t*)(dev + o_type);
-  hdsc->gcs = (const double*)(dev + o_gcs);
+  hdsc->gab = (const double*)(dev + o_gab);
   hdsc->dterms = (const DTerm*)(dev + o_diag);
   hdsc->ndterms = ndiag;
   hdsc->xy = (const DTerm*)(dev + o_xy);
   hdsc->nxy = nxy;
   hdsc->lad1 = lad1;
   hdsc->lad2 = lad2;
+  hdsc->inv1 = inv1;
+  hdsc->inv2 = inv2;
   hdsc->init_tab = (const double*)(dev + o_init);
   hdsc->out = (double*)(dev + o_out);
   hdsc->grad = 1;
@@ -2286,7 +2293,7 @@ extern "C" int qg_mcclean_grad_run_noalloc(qg_ctx* c, int n, int L, int entangle
   // tables in, one launch, results out (the kernel writes every result, so
   // nothing in the scratch needs clearing)
   HIPCHK(hipMemcpyAsync(dev, h, o_out, hipMemcpyHostToDevice, c->stream));
-  HIPCHK(launch_fused(dev + o_desc, 1, n, c->stream));
+  HIPCHK(launch_fused(dev + o_desc, 1, n, FM_MCCLEAN, 0, c->stream));
   HIPCHK(hipMemcpyAsync(h + o_out, dev + o_out, sizeof(double) * (1 + np), hipMemcpyDeviceToHost, c->stream));
   HIPCHK(hipStreamSynchronize(c->stream));
   const double* res = (const double*)(h + o_out);
@@ -2665,19 +2672,21 @@ static int qaoa_run(qg_plan* p, int B, const qg_term* terms, const int32_t* term
     const int per = 1 + 2 * L;
     std::vector<double> res((size_t)B * per);
     auto fill = [&](int b, FusedDescH& d, Arena& ar) -> int {
-      d.kind = 1;
       double* dp = nullptr;
-      double* hp = ar.take<double>((size_t)2 * L, &dp);
+      double* hp = ar.take<double>((size_t)3 * L, &dp);
       for (int i = 0; i < L; ++i) {
-        hp[2 * i] = betas[(size_t)b * L + i];
-        hp[2 * i + 1] = gammas[(size_t)b * L + i];
+        const GateAB g = gate_ab(betas[(size_t)b * L + i], 1.0);
+        hp[2 * i] = g.a;
+        hp[2 * i + 1] = g.b;
+        hp[2 * L + i] = gammas[(size_t)b * L + i];
       }
-      d.params = dp;
+      d.gab = dp;
+      d.gamma = dp + 2 * L;
       return obs_tables(obs[b], d, ar);
     };
     size_t mx = 0;
     for (int b = 0; b < B; ++b) mx = std::max(mx, obs[b].diag.size());
-    const size_t bytes = (size_t)L * 16 + (mx + 2) * sizeof(DTerm);
+    const size_t bytes = (size_t)L * 24 + (mx + 2) * sizeof(DTerm);
     // a single circuit keeps its final state (qg_plan_get_state, qg_plan_term_prob)
     if (B == 1 && p->cap_fstate < ((size_t)16 << n)) {
       HIPCHK(hipStreamSynchronize(c->stream));
@@ -2687,7 +2696,12 @@ static int qaoa_run(qg_plan* p, int B, const qg_term* terms, const int32_t* term
       HIPCHK(hipMalloc(&p->d_fstate, ((size_t)16) << n));
       p->cap_fstate = (size_t)16 << n;
     }
-    CHK(run_fused(p, B, bytes, per, grad, B == 1 ? p->d_fstate : nullptr, fill, res.data()));
+    // the largest phase angle decides the sincos (W: the largest sum of |w|)
+    double gmax = 0.0;
+    for (int k = 0; k < B * L; ++k) gmax = std::max(gmax, std::fabs(gammas[k]));
+    const int mode = phase == 1 ? FM_QAOA_LUT : gmax * W < kSincosMax ? FM_QAOA_SINCOS : FM_QAOA_LARGE;
+    CHK(run_fused(p, B, mode, phase == 1 ? Wi : 0, bytes, per, grad, B == 1 ? p->d_fstate : nullptr, fill,
+                  res.data()));
     for (int b = 0; b < B; ++b) {
       E_out[b] = res[(size_t)b * per];
       if (grad)
@@ -2695,6 +2709,8 @@ static int qaoa_run(qg_plan* p, int B, const qg_term* terms, const int32_t* term
     }
     p->last_state_ptr = B == 1 ? p->d_fstate : nullptr;
     p->state_sign = false;
+    for (int i = 0; i < L; ++i)
+      if (n % 2 == 1) p->state_sign ^= gate_flips(betas[i], 1.0);
     return QG_OK;
   }
   CHK(ensure_workspace(p));
