@@ -35,7 +35,7 @@ hipError_t simple_convert_out(int dtype, const void* in, void* out_c128, int n, 
 hipError_t simple_term_expec(int dtype, const void* v, int n, const PTerm* t, int nt, double* part, double* out,
                              hipStream_t st, const PTerm* h_t);
 hipError_t simple_sample_basis(int dtype, const void* v, int n, const int32_t* order, const double* u, int shots,
-                               int32_t* idx, double* mass, hipStream_t st);
+                               int32_t* idx, double* mass, int batch, hipStream_t st);
 constexpr int kDotBlocks = 512;
 hipError_t launch_fused(const void* descs, int batch, int n, int mode, int lut_w, hipStream_t st);
 hipError_t set_fused_attributes();
@@ -2531,7 +2531,7 @@ extern "C" int qg_mcclean_shift_sample(qg_plan* p, const int32_t* axes, const do
   CHK(mcclean_shift_run(p, axes, angles, ini_state, nshift, shift_param, shift_delta,
                         [&](int s, const void* fin) {
                           return simple_sample_basis(p->dtype, fin, p->n, b.order, b.u + (size_t)s * shots, shots,
-                                                     b.idx + (size_t)s * shots, b.mass, p->ctx->stream);
+                                                     b.idx + (size_t)s * shots, b.mass, 1, p->ctx->stream);
                         }));
   if (nu) HIPCHK(hipMemcpy(idx, b.idx, (size_t)nu * 4, hipMemcpyDeviceToHost));
   return QG_OK;
@@ -3273,7 +3273,7 @@ extern "C" int qg_state_sample_basis(qg_state* st, const int32_t* order, int sho
   HIPCHK(hipSetDevice(st->ctx->device));
   SampleBufs b;
   CHK(sample_setup(st->n, order, shots, u, b));
-  HIPCHK(simple_sample_basis(st->dtype, st->v, st->n, b.order, b.u, shots, b.idx, b.mass, st->ctx->stream));
+  HIPCHK(simple_sample_basis(st->dtype, st->v, st->n, b.order, b.u, shots, b.idx, b.mass, 1, st->ctx->stream));
   HIPCHK(hipStreamSynchronize(st->ctx->stream));
   HIPCHK(hipMemcpy(idx, b.idx, (size_t)shots * 4, hipMemcpyDeviceToHost));
   return QG_OK;

@@ -4,6 +4,7 @@
 // State method of the reference on the GPU.
 #include <hip/hip_runtime.h>
 #include "qg_internal.h"
+#include "qg_wave.hpp"
 
 namespace qg {
 
@@ -321,7 +322,14 @@ constexpr int kSimpleMaxN = 31;
 // qaoa.py:196-198): a draw u maps to the first position whose cumulative
 // probability reaches u, and to position 0 when none does
 // (argmax(qvals >= u)).  Two levels: masses of 1024-position blocks and
-// their prefix, then a binary search over blocks and a walk inside one.
+// their prefix, then one wave per shot searches the prefix 64 entries at a
+// time and scans its block 64 positions at a time.  blockIdx.y selects one of
+// several states (state b at v + b * N, its masses, uniforms and positions
+// behind each other).
+//
+// One thread per shot walking its block position by position waited for about
+// 500 loads in a row: 170 us for 64 shots on 12 qubits, against 8.7 us with a
+// wave per shot, whose sixteen loads are in flight together.
 // ---------------------------------------------------------------------------
 template <class S>
 __device__ __forceinline__ double prob_at(const typename V2<S>::T* __restrict__ v, const int32_t* __restrict__ order,
@@ -334,70 +342,92 @@ __device__ __forceinline__ double prob_at(const typename V2<S>::T* __restrict__ 
 template <class S>
 __global__ void __launch_bounds__(256) k_block_mass(const typename V2<S>::T* __restrict__ v, uint32_t N,
                                                     const int32_t* __restrict__ order, double* __restrict__ mass) {
-  __shared__ double red[256];
-  const uint32_t base = blockIdx.x * (uint32_t)kSampleBlock + threadIdx.x * 4u;
+  __shared__ double red[4];
+  v += (size_t)blockIdx.y * N;
+  const uint32_t base = blockIdx.x * (uint32_t)kSampleBlock + threadIdx.x;
   double s = 0.0;
+#pragma unroll
   for (uint32_t j = 0; j < 4; ++j)
-    if (base + j < N) s += prob_at<S>(v, order, base + j);
-  red[threadIdx.x] = s;
+    if (base + j * 256u < N) s += prob_at<S>(v, order, base + j * 256u);
+  s = wave_sum(s, 64);
+  if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = s;
   __syncthreads();
-  for (int h = 128; h > 0; h >>= 1) {
-    if ((int)threadIdx.x < h) red[threadIdx.x] += red[threadIdx.x + h];
-    __syncthreads();
-  }
-  if (threadIdx.x == 0) mass[blockIdx.x] = red[0];
+  if (threadIdx.x == 0) mass[(size_t)blockIdx.y * gridDim.x + blockIdx.x] = ((red[0] + red[1]) + red[2]) + red[3];
 }
 
-// Inclusive prefix sums of mass[0, nb) in place, one workgroup of 256 threads.
-__global__ void __launch_bounds__(256) k_mass_prefix(double* __restrict__ mass, int nb) {
-  __shared__ double tot[256];
-  const int chunk = (nb + 255) / 256;
-  const int lo = (int)threadIdx.x * chunk, hi = min(nb, lo + chunk);
-  double s = 0.0;
-  for (int b = lo; b < hi; ++b) s += mass[b];
-  tot[threadIdx.x] = s;
-  __syncthreads();
-  if (threadIdx.x == 0) {
-    double a = 0.0;
-    for (int t = 0; t < 256; ++t) {
-      a += tot[t];
-      tot[t] = a;
+// Inclusive prefix sums of mass[0, nb) in place: one workgroup per state, 1024
+// entries a round (a scan per wave, the waves' totals through LDS).
+__global__ void __launch_bounds__(1024) k_mass_prefix(double* __restrict__ mass, int nb) {
+  __shared__ double tot[16];
+  mass += (size_t)blockIdx.x * nb;
+  const int wave = threadIdx.x >> 6;
+  double carry = 0.0;
+  for (int b0 = 0; b0 < nb; b0 += 1024) {
+    const int b = b0 + (int)threadIdx.x;
+    double s = wave_scan(b < nb ? mass[b] : 0.0);
+    if ((threadIdx.x & 63) == 63) tot[wave] = s;
+    __syncthreads();
+    double before = carry, all = carry;
+    for (int w = 0; w < 16; ++w) {
+      if (w == wave) before = all;
+      all += tot[w];
     }
-  }
-  __syncthreads();
-  double a = threadIdx.x ? tot[threadIdx.x - 1] : 0.0;
-  for (int b = lo; b < hi; ++b) {
-    a += mass[b];
-    mass[b] = a;
+    if (b < nb) mass[b] = before + s;
+    carry = all;
+    __syncthreads();
   }
 }
 
 template <class S>
-__global__ void k_basis_search(const typename V2<S>::T* __restrict__ v, uint32_t N, const int32_t* __restrict__ order,
-                               const double* __restrict__ pref, int nb, const double* __restrict__ u, int shots,
-                               int32_t* __restrict__ idx) {
-  const int s = blockIdx.x * blockDim.x + threadIdx.x;
+__global__ void __launch_bounds__(256) k_basis_search(const typename V2<S>::T* __restrict__ v, uint32_t N,
+                                                      const int32_t* __restrict__ order,
+                                                      const double* __restrict__ pref, int nb,
+                                                      const double* __restrict__ u, int shots,
+                                                      int32_t* __restrict__ idx) {
+  const int s = (int)(blockIdx.x * 4 + (threadIdx.x >> 6));
+  const uint32_t lane = threadIdx.x & 63;
   if (s >= shots) return;
-  const double us = u[s];
+  v += (size_t)blockIdx.y * N;
+  pref += (size_t)blockIdx.y * nb;
+  const size_t at = (size_t)blockIdx.y * shots + s;
+  const double us = u[at];
   if (!(pref[nb - 1] >= us)) {
-    idx[s] = 0;
+    if (lane == 0) idx[at] = 0;
     return;
   }
-  int lo = 0, hi = nb - 1;  // the first block whose prefix reaches us
+  // the first block whose prefix reaches us: [lo, hi] shrinks 64-fold a round
+  int lo = 0, hi = nb - 1;
   while (lo < hi) {
-    const int mid = (lo + hi) >> 1;
-    if (pref[mid] >= us) hi = mid;
-    else lo = mid + 1;
+    const int step = (hi - lo + 64) / 64;
+    const int e = min(lo + ((int)lane + 1) * step - 1, hi);
+    const int f = __builtin_ctzll(__ballot(pref[e] >= us));  // the lane at hi always reaches
+    hi = min(lo + (f + 1) * step - 1, hi);
+    lo = lo + f * step;
   }
   double acc = lo ? pref[lo - 1] : 0.0;
   const uint32_t k0 = (uint32_t)lo * (uint32_t)kSampleBlock;
   const uint32_t k1 = min(N, k0 + (uint32_t)kSampleBlock);
-  uint32_t k = k0;
-  for (; k < k1; ++k) {
-    acc += prob_at<S>(v, order, k);
-    if (acc >= us) break;
+  double p[kSampleBlock / 64];
+#pragma unroll
+  for (int j = 0; j < kSampleBlock / 64; ++j) {
+    const uint32_t k = k0 + (uint32_t)j * 64u + lane;
+    p[j] = k < k1 ? prob_at<S>(v, order, k) : 0.0;
   }
-  idx[s] = (int32_t)(k < k1 ? k : k1 - 1);  // rounding between the two levels: the block's last position
+  uint32_t found = k1 - 1;  // rounding between the two levels: the block's last position
+  bool done = false;
+#pragma unroll
+  for (int j = 0; j < kSampleBlock / 64; ++j) {
+    if (!done) {
+      const double c = wave_scan(p[j]);
+      const unsigned long long m = __ballot(acc + c >= us);
+      if (m) {
+        found = min(k0 + (uint32_t)j * 64u + (uint32_t)__builtin_ctzll(m), k1 - 1);
+        done = true;
+      }
+      acc += wave_lane(c, 63);
+    }
+  }
+  if (lane == 0) idx[at] = (int32_t)found;
 }
 
 static inline dim3 grid_for(uint64_t n, int threads) { return dim3((unsigned)((n + threads - 1) / threads)); }
@@ -522,18 +552,20 @@ hipError_t simple_convert_out(int dtype, const void* in, void* out_c128, int n, 
   return hipGetLastError();
 }
 
-// mass: (2^n + kSampleBlock - 1) / kSampleBlock doubles of scratch.
+// Draws for `batch` states behind each other at v: u and idx hold shots
+// entries per state, mass (2^n + kSampleBlock - 1) / kSampleBlock doubles of
+// scratch per state.
 hipError_t simple_sample_basis(int dtype, const void* v, int n, const int32_t* order, const double* u, int shots,
-                               int32_t* idx, double* mass, hipStream_t st) {
-  if (n < 1 || n > kSimpleMaxN || shots < 1) return hipErrorInvalidValue;
+                               int32_t* idx, double* mass, int batch, hipStream_t st) {
+  if (n < 1 || n > kSimpleMaxN || shots < 1 || batch < 1 || batch > 65535) return hipErrorInvalidValue;
   const uint32_t N = (uint32_t)(1ull << n);
   const int nb = (int)((N + kSampleBlock - 1) / kSampleBlock);
-  QG_DT_SWITCH(dtype, hipLaunchKernelGGL(k_block_mass<S>, dim3(nb), dim3(256), 0, st, (const typename V2<S>::T*)v, N,
-                                         order, mass));
-  hipLaunchKernelGGL(k_mass_prefix, dim3(1), dim3(256), 0, st, mass, nb);
-  QG_DT_SWITCH(dtype, hipLaunchKernelGGL(k_basis_search<S>, grid_for((uint64_t)shots, 256), dim3(256), 0, st,
-                                         (const typename V2<S>::T*)v, N, order, (const double*)mass, nb, u, shots,
-                                         idx));
+  QG_DT_SWITCH(dtype, hipLaunchKernelGGL(k_block_mass<S>, dim3(nb, batch), dim3(256), 0, st,
+                                         (const typename V2<S>::T*)v, N, order, mass));
+  hipLaunchKernelGGL(k_mass_prefix, dim3(batch), dim3(1024), 0, st, mass, nb);
+  QG_DT_SWITCH(dtype, hipLaunchKernelGGL(k_basis_search<S>, dim3((unsigned)(((uint64_t)shots + 3) / 4), batch),
+                                         dim3(256), 0, st, (const typename V2<S>::T*)v, N, order, (const double*)mass,
+                                         nb, u, shots, idx));
   return hipGetLastError();
 }
 
