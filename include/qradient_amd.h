@@ -214,6 +214,21 @@ int qg_qaoa_grad_run_ini(qg_plan* plan, int B, const qg_term* terms, const int32
 int qg_qaoa_expec_val_ini(qg_plan* plan, int B, const qg_term* terms, const int32_t* term_off, const double* betas,
                           const double* gammas, const double* ini_states, double* E_out);
 
+/* The shifted circuits of Qaoa.sample_grad_dense (qaoa.py:83-158) of one
+ * circuit (terms[0, nterms): its z / zz classical Hamiltonian), measured in the
+ * computational basis.  Layer i has 2 * (nterms + n) of them, in this order:
+ * for each component j the cost phase followed by exp(-i pi/4 C_j), then by
+ * exp(+i pi/4 C_j); for each qubit q the mixer followed by RX(pi/2), then by
+ * RX(-pi/2).  u and idx hold `shots` entries per shifted circuit, layer after
+ * layer; idx[k] is the basis state that the uniform u[k] draws, as
+ * qg_state_sample_basis maps it (natural order).  expec[k] = <P_k> of
+ * mterms[0, nm) (weights ignored) in the unshifted circuit's final state,
+ * expec[nm] its squared norm.  The plan's own state is left as it is.
+ * ini_state: NULL (|+>^n) or 2^n complex128 amplitudes.  Needs n <= 31. */
+int qg_qaoa_shift_sample(qg_plan* plan, const qg_term* terms, int nterms, const double* betas, const double* gammas,
+                         const double* ini_state, const qg_term* mterms, int nm, double* expec, int shots,
+                         const double* u, int32_t* idx);
+
 /* Lays a McClean plan out again for another circuit shape: n qubits, L
  * layers, ckpt_every as for qg_mcclean_plan; dtype, entangler, context and
  * tile options are kept.  The plan's small device tables only grow, so after

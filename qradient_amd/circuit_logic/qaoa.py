@@ -13,7 +13,7 @@ import numpy as np
 
 from .. import _native
 from ..physical_components import Gates
-from .base import ParametrizedCircuit, sample_projectors
+from .base import ParametrizedCircuit, draw_uniforms, sample_projectors
 
 
 class Qaoa(ParametrizedCircuit):
@@ -87,73 +87,43 @@ class Qaoa(ParametrizedCircuit):
         gives grad[i, 0] = sum_q (o_plus_q - o_minus_q) / 2.  An estimate o is
         the mean of C(x) over shot_num basis draws of the shifted circuit's
         final state.  The reference carries each suffix circuit as a dense
-        left-hand-side matrix; here the shifted states run the suffix on the
-        device from device copies of the forward history, and are sampled
-        there by the inverse CDF at uniforms drawn on the host in the
+        left-hand-side matrix; here the shifted copies of a layer's stored
+        states run the rest of the circuit on the device together, and are
+        sampled there by the inverse CDF at uniforms drawn on the host in the
         reference's order.  E is <C> (or, with exact_expec_val=False, the
         shot estimate of the whole observable).  The reference mutates
         ``ini_state``; it is only read here."""
-        from ..physical_components import State
         betas, gammas = self.__check_parameters(betas, gammas)
         n, L = self.qnum, self.lnum
         cterms = self.observable.classical_terms()
         arr, k = _native.terms_array(cterms)
         C = self._classical_values(cterms)
-
-        def new_state():
-            st = State(n, '+', dtype=self.dtype, device=self.device)
-            st.gates = self._gates
-            return st
-
-        st = new_state()
-        if ini_state is not None:
-            st.vec = ini_state
-        hist = []
-        for i in range(L):
-            st.exp_ham_classical(gammas[i])
-            hist.append(new_state().copy_from(st))
-            st.xrot_all(betas[i])
-            hist.append(new_state().copy_from(st))
-        terms = self.observable.terms
-        if exact_expec_val:
-            Eo = ctypes.c_double()
-            _native.call('qg_state_expec_val', st._h, arr, k, ctypes.byref(Eo))
-            E = np.float64(Eo.value)
-        else:
-            E = sample_projectors(st.term_probs(self.observable), [t[3] for t in terms], shot_num)
-        work = new_state()
+        _keep, ini = self._ini(ini_state, n)
+        terms = cterms if exact_expec_val else self.observable.terms
+        w = np.array([t[3] for t in terms])
         shots = int(shot_num)
-
-        def estimate(first_layer, mixer_first):
-            """Runs the suffix from ``work`` and returns the shot mean of C."""
-            if mixer_first:
-                work.xrot_all(betas[first_layer - 1])
-            for j in range(first_layer, L):
-                work.exp_ham_classical(gammas[j])
-                work.xrot_all(betas[j])
-            u = np.random.uniform(size=shots)
-            return C[work.sample_basis(u)].mean()
-
+        # draws in the reference's order: E's shots, then per layer each
+        # component's two circuits and each qubit's
+        u_E = None if exact_expec_val else draw_uniforms(len(terms), shots)
+        u = draw_uniforms(L * 2 * (k + n), shots)
+        if shots == 0:
+            u = np.zeros((u.shape[0], 1))  # no shots: E alone, the estimates are nan
+        m_arr, m = _native.terms_array(terms)
+        expec = np.empty(m + 1)
+        idx = np.empty(u.shape, dtype=np.int32)
+        _native.call('qg_qaoa_shift_sample', self._get_plan(), arr, k, _native.dptr(betas), _native.dptr(gammas), ini,
+                     m_arr, m, _native.dptr(expec), u.shape[1], _native.dptr(u), _native.iptr(idx))
+        if exact_expec_val:
+            E = np.float64((w * expec[:m]).sum())
+        else:
+            E = sample_projectors(.5 * (expec[m] + expec[:m]), w, shots, uniforms=u_E)
+        o = C[idx[:, :shots]].mean(axis=1).reshape(L, k + n, 2)
+        diff = o[:, :, 0] - o[:, :, 1]
         grad = np.empty((L, 2), dtype='double')
         for i in range(L):
-            dg = 0.
-            for j in range(len(cterms)):
-                out = []
-                for angle in (np.pi / 4, -np.pi / 4):
-                    work.copy_from(hist[2 * i])
-                    work.exp_ham_classical_component(angle, j)
-                    out.append(estimate(i + 1, True))
-                dg += out[0] - out[1]
-            db = 0.
-            for q in range(n):
-                out = []
-                for angle in (np.pi / 2, -np.pi / 2):
-                    work.copy_from(hist[2 * i + 1])
-                    work.xrot(angle, q)
-                    out.append(estimate(i + 1, False))
-                db += out[0] - out[1]
-            grad[i, 0] = .5 * db
-            grad[i, 1] = dg
+            # summed component by component and qubit by qubit, in order
+            grad[i, 0] = .5 * sum(diff[i, k:].tolist(), 0.)
+            grad[i, 1] = sum(diff[i, :k].tolist(), 0.)
         return E, grad
 
     def _classical_values(self, cterms):

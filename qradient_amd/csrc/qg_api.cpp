@@ -32,8 +32,11 @@ hipError_t simple_init(int dtype, void* v, int n, const double* tab, hipStream_t
 hipError_t simple_scale(int dtype, void* v, int n, double re, double im, hipStream_t st);
 hipError_t simple_convert_in(int dtype, const void* in_c128, void* out, int n, hipStream_t st);
 hipError_t simple_convert_out(int dtype, const void* in, void* out_c128, int n, hipStream_t st);
+size_t simple_term_part(int n, int batch);
 hipError_t simple_term_expec(int dtype, const void* v, int n, const PTerm* t, int nt, double* part, double* out,
-                             hipStream_t st, const PTerm* h_t);
+                             hipStream_t st, const PTerm* h_t, int batch);
+hipError_t simple_shift_copies(int dtype, const void* in, void* out, int n, const ShiftOp* op, int batch,
+                               hipStream_t st);
 hipError_t simple_sample_basis(int dtype, const void* v, int n, const int32_t* order, const double* u, int shots,
                                int32_t* idx, double* mass, int batch, hipStream_t st);
 constexpr int kDotBlocks = 512;
@@ -383,12 +386,14 @@ enum PlanKind { PK_MCCLEAN = 0, PK_QAOA = 1 };
 struct Launch {
   int desc;  // index into the descriptor table (first of `batch` consecutive ones)
   int batch = 1;
+  bool shared = false;  // one descriptor for the whole batch (PassDesc::bstride)
   int K = 0;
   bool post = false;  // the pass has diagonal ops after its gates (set at launch from the flags)
   int tab = 0;        // bytes of the table the pass stages in LDS (set at launch)
   int R, threads, grid, phase;
   bool two;
   int kind;  // 0 pass kernel, 1 generic observable, 2 convert-in (ini state)
+  int ndesc() const { return shared ? 1 : batch; }
 };
 
 struct qg_plan {
@@ -422,6 +427,8 @@ struct qg_plan {
   char* d_arena = nullptr;  // and their device copy
   size_t arena_cap = 0;
   void* d_fstate = nullptr;  // final state of the last fused McClean run
+  char* d_shift = nullptr;   // shifted circuits: their states (grows; freed with the plan)
+  size_t shift_cap = 0;
   std::vector<Geo> geo;
   size_t S = 0;  // bytes per state
   // workspace
@@ -755,14 +762,14 @@ static int term_expec(qg_ctx* c, int dtype, const void* v, int n, const qg_term*
   const int nt = nterms + 1;
   HIPCHK(hipSetDevice(c->device));
   const size_t tb = ((sizeof(PTerm) * nt + 255) / 256) * 256;
-  const size_t pb = sizeof(double) * kTermBlocks * kTermPartRows;
+  const size_t pb = sizeof(double) * simple_term_part(n, 1);
   char* buf = nullptr;
   HIPCHK(hipMalloc(&buf, tb + pb + sizeof(double) * nt));
   PTerm* d_t = (PTerm*)buf;
   double* d_part = (double*)(buf + tb);
   double* d_out = (double*)(buf + tb + pb);
   hipError_t err = hipMemcpyAsync(d_t, h.data(), sizeof(PTerm) * nt, hipMemcpyHostToDevice, c->stream);
-  if (err == hipSuccess) err = simple_term_expec(dtype, v, n, d_t, nt, d_part, d_out, c->stream, h.data());
+  if (err == hipSuccess) err = simple_term_expec(dtype, v, n, d_t, nt, d_part, d_out, c->stream, h.data(), 1);
   if (err == hipSuccess) err = hipMemcpyAsync(e, d_out, sizeof(double) * nt, hipMemcpyDeviceToHost, c->stream);
   if (err == hipSuccess) err = hipStreamSynchronize(c->stream);
   (void)hipFree(buf);
@@ -1047,12 +1054,12 @@ static int run_launches(qg_plan* p, int ndesc, int first_desc = 0) {
       // the d/dgamma reduction; the rest the general form
       l.post = l.two && ((d.flags & (F_DRED_POST | F_PHASE_POST | F_OBS_DIAG | F_STORE_A)) != 0 ||
                          !(d.flags & F_LOAD_A) || ((d.flags & F_PHASE_PRE) && !(d.flags & F_DRED_PRE)));
-      for (int b = 0; b < l.batch; ++b) {
+      for (int b = 0; b < l.ndesc(); ++b) {
         desc_slots(p->h_desc[l.desc + b], l.R, l.two, l.two && !l.post);
         desc_order(p, p->h_desc[l.desc + b]);
       }
       if (d.flags & (F_PHASE_PRE | F_PHASE_POST | F_DRED_PRE | F_DRED_POST | F_OBS_DIAG))
-        for (int b = 0; b < l.batch; ++b)
+        for (int b = 0; b < l.ndesc(); ++b)
           cterm_at.push_back({l.desc + b, split_terms(p, p->h_desc[l.desc + b], l.R, p->h_cterms)});
       l.tab = ((d.flags & F_INIT_TAB) ? (int)sizeof(double) * (p->n + 1) : 0) +
               ((l.phase == 1 && (d.flags & (F_PHASE_PRE | F_PHASE_POST))) ? (int)sizeof(double) * 2 * (2 * d.lut_off + 1)
@@ -1188,12 +1195,12 @@ static int stream_flush(qg_plan* p) {
     if (!(d.flags & (F_PHASE_PRE | F_PHASE_POST))) l.phase = 0;
     l.post = l.two && ((d.flags & (F_DRED_POST | F_PHASE_POST | F_OBS_DIAG | F_STORE_A)) != 0 ||
                        !(d.flags & F_LOAD_A) || ((d.flags & F_PHASE_PRE) && !(d.flags & F_DRED_PRE)));
-    for (int b = 0; b < l.batch; ++b) {
+    for (int b = 0; b < l.ndesc(); ++b) {
       desc_slots(p->h_desc[l.desc + b], l.R, l.two, l.two && !l.post);
       desc_order(p, p->h_desc[l.desc + b]);
     }
     if (d.flags & split_flags)
-      for (int b = 0; b < l.batch; ++b) {
+      for (int b = 0; b < l.ndesc(); ++b) {
         if (p->h_cterms.size() + (size_t)std::max(0, p->h_desc[l.desc + b].ndterms) > p->stream_bound)
           return fail(QG_ERR_HIP, "internal: split terms exceed their bound");
         const size_t off = split_terms(p, p->h_desc[l.desc + b], l.R, p->h_cterms);
@@ -1203,7 +1210,7 @@ static int stream_flush(qg_plan* p) {
             ((l.phase == 1 && (d.flags & (F_PHASE_PRE | F_PHASE_POST))) ? (int)sizeof(double) * 2 * (2 * d.lut_off + 1)
                                                                          : 0);
     d0 = std::min(d0, l.desc);
-    d1 = std::max(d1, l.desc + l.batch);
+    d1 = std::max(d1, l.desc + l.ndesc());
   }
   const size_t ct1 = p->h_cterms.size();
   if (ct1 > ct0) {
@@ -1316,6 +1323,9 @@ static void free_small(qg_plan* p) {
   p->cstage_cap = 0;
   (void)hipFree(p->d_arena);
   (void)hipFree(p->d_fstate);
+  (void)hipFree(p->d_shift);
+  p->d_shift = nullptr;
+  p->shift_cap = 0;
   p->h_stage = nullptr;
   p->stage_cap = 0;
   p->h_arena = nullptr;
@@ -2306,64 +2316,99 @@ extern "C" int qg_mcclean_grad_run_noalloc(qg_ctx* c, int n, int L, int entangle
 // Parameter-shifted McClean circuits (McClean.sample_grad, mc_clean.py:117-198)
 // ---------------------------------------------------------------------------
 
-// Appends the forward passes of layers [first, L) to the plan's launch list,
-// from the state at src (nullptr: the RY(pi/4) product state, generated by the
-// first pass).  The states go to the two buffers buf: the low pass gathers
-// out of place, high passes work in place, so src is only read.  Returns the
-// buffer that holds the final state.
-static void* mcclean_forward_suffix(qg_plan* p, const int32_t* axes, const double* angles, int first,
-                                    const void* src, void* const buf[2], int& nd) {
-  const int n = p->n, L = p->L, P = (int)p->geo.size();
+// Device scratch for shifted circuits, grown as needed.
+static int ensure_shift(qg_plan* p, size_t bytes) {
+  if (bytes <= p->shift_cap) return QG_OK;
+  HIPCHK(hipStreamSynchronize(p->ctx->stream));
+  (void)hipFree(p->d_shift);
+  p->d_shift = nullptr;
+  p->shift_cap = 0;
+  HIPCHK(hipMalloc(&p->d_shift, bytes));
+  p->shift_cap = bytes;
+  return QG_OK;
+}
+
+// Shifted circuits run this many amplitudes at a time (all circuits of a
+// launch together): enough tiles to fill the device, and states that the
+// memory-side cache holds.  From 22 qubits on they run one by one, as one
+// circuit fills the device.  sample_grad on 14 qubits (112 shifted circuits of
+// 8 workgroups each): one by one 7.6 ms, batched 1.7 ms.
+constexpr int kShiftAmpsLog2 = 22;
+static int shift_batch(int n) { return n >= kShiftAmpsLog2 ? 1 : std::min(4096, 1 << (kShiftAmpsLog2 - n)); }
+
+// Appends one launch of a forward pass of geometry G0 over `batch` circuits to
+// the plan's launch list and returns its first descriptor (shared: the only
+// one), with the fields that do not depend on the circuit.
+static PassDesc& push_forward(qg_plan* p, const Geo& G0, int batch, bool shared, int& nd) {
+  bool tf = false;
+  const Geo G = with_role(G0, p->dtype, ROLE_FWD, &tf);
+  Launch l;
+  l.desc = nd;
+  l.batch = batch;
+  l.shared = shared;
+  l.R = G.R;
+  l.K = G.K;
+  l.post = tf;
+  l.threads = G.threads;
+  l.grid = grid_for_pass(p, G, false, tf, 0);
+  l.phase = 0;
+  l.two = false;
+  l.kind = 0;
+  p->launches.push_back(l);
+  PassDesc& d = p->h_desc[nd];
+  nd += l.ndesc();
+  desc_geo(d, p->n, G);
+  d.grid = p->gmax;
+  d.lad1 = p->lad1;
+  d.lad2 = p->lad2;
+  d.init_tab = p->d_init;
+  d.dterms = p->d_terms;
+  d.ndterms = 0;
+  d.part = p->d_part;
+  return d;
+}
+
+// The gates of layer i on the bits a forward pass owns.
+static void layer_gates(PassDesc& d, const Geo& G0, int n, int i, const int32_t* axes, const double* angles) {
+  for (int lb = G0.own_lo; lb < G0.own_hi; ++lb) {
+    const int b = (lb < G0.c) ? lb : G0.p + (lb - G0.c);
+    const int q = n - 1 - b;
+    set_gate(d, lb, axes[i * n + q], angles[i * n + q], 1.0);
+  }
+}
+
+// Appends the forward passes of layers [first, last) over `batch` states to the
+// plan's launch list, from the states at src (nullptr: the RY(pi/4) product
+// state, generated by the first pass).  The states go to the two buffers buf:
+// the low pass gathers out of place, high passes work in place, so src is only
+// read.  Returns the buffer that holds the final states.
+static void* mcclean_forward_layers(qg_plan* p, const int32_t* axes, const double* angles, int first, int last,
+                                    const void* src, void* const buf[2], int batch, int& nd) {
   const uint32_t ent = p->ent == QG_ENT_CNOT ? F_GATHER : F_CZ_PRE;
   const void* cur = src;
-  for (int i = first; i < L; ++i) {
-    for (int g = 0; g < P; ++g) {
-      const Geo& G0 = p->geo[g];
-      bool tf = false;
-      const Geo G = with_role(G0, p->dtype, ROLE_FWD, &tf);
-      Launch l;
-      l.desc = nd;
-      l.R = G.R;
-      l.K = G.K;
-      l.post = tf;
-      l.threads = G.threads;
-      l.grid = grid_for_pass(p, G, false, tf, 0);
-      l.phase = 0;
-      l.two = false;
-      l.kind = 0;
-      p->launches.push_back(l);
-      PassDesc& d = p->h_desc[nd++];
-      desc_geo(d, n, G);
-      d.grid = p->gmax;
-      d.lad1 = p->lad1;
-      d.lad2 = p->lad2;
-      d.init_tab = p->d_init;
-      d.dterms = p->d_terms;
-      d.ndterms = 0;
-      d.part = p->d_part;
-      uint32_t f = F_ROT_A | F_STORE_A;
-      f |= (g == 0) ? (ent | (cur ? F_LOAD_A : F_INIT_TAB)) : F_LOAD_A;
+  for (int i = first; i < last; ++i)
+    for (int g = 0; g < (int)p->geo.size(); ++g) {
+      PassDesc& d = push_forward(p, p->geo[g], batch, true, nd);
+      d.flags = F_ROT_A | F_STORE_A | (g == 0 ? (ent | (cur ? F_LOAD_A : F_INIT_TAB)) : (uint32_t)F_LOAD_A);
       void* out = (g == 0) ? (cur == buf[0] ? buf[1] : buf[0]) : (void*)cur;
-      d.flags = f;
       d.a_in = cur;
       d.a_out = out;
-      for (int lb = G0.own_lo; lb < G0.own_hi; ++lb) {
-        const int b = (lb < G0.c) ? lb : G0.p + (lb - G0.c);
-        const int q = n - 1 - b;
-        set_gate(d, lb, axes[i * n + q], angles[i * n + q], 1.0);
-      }
+      d.bstride = (int64_t)p->S;
+      layer_gates(d, p->geo[g], p->n, i, axes, angles);
       cur = out;
     }
-  }
   return (void*)cur;
 }
 
 // Runs the unshifted circuit through the pass kernels, keeping its layer-end
 // states (history) or checkpoints, then each shifted circuit from the nearest
 // stored state before its shifted layer (the reference restarts from
-// state_history[i], mc_clean.py:140-151), and calls on_shift(s, final state)
-// to enqueue that shift's measurement on the plan's stream.  Afterwards the
-// plan's state is the unshifted circuit's final state.
+// state_history[i], mc_clean.py:140-151), and calls on_shift(s, count, states)
+// to enqueue the measurement of shifts [s, s + count), whose final states lie
+// behind each other, on the plan's stream.  Consecutive shifts of one layer
+// share their launches: the shifted layer has a descriptor per circuit, the
+// layers after it are the same for all.  Afterwards the plan's state is the
+// unshifted circuit's final state.
 template <class OnShift>
 static int mcclean_shift_run(qg_plan* p, const int32_t* axes, const double* angles, const double* ini_state,
                              int nshift, const int32_t* shift_param, const double* shift_delta, OnShift on_shift) {
@@ -2392,13 +2437,31 @@ static int mcclean_shift_run(qg_plan* p, const int32_t* axes, const double* angl
   }
   float total_ms = p->last_ms;  // the unshifted run's
   const void* start0 = ini_state ? wsp(p, p->off_prep) : nullptr;
-  // the adjoint's two lambda buffers are free in a forward-only run
-  void* buf[2] = {wsp(p, p->off_lam), wsp(p, p->off_lam + p->S)};
-  std::vector<double> ang(angles, angles + (size_t)L * n);
-  // Two halves of the descriptor table (a suffix has at most P * L passes):
-  // the host builds shift s + 1 while the device runs shift s, and waits for
-  // shift s - 1, the last user of a half, before rewriting it.
-  const int half = P * L;
+  // the groups of consecutive shifts of one layer
+  std::vector<int> group;  // first shift of each, and nshift
+  int most = 1;
+  for (int s = 0; s < nshift;) {
+    int e = s + 1;
+    while (e < nshift && shift_param[e] / n == shift_param[s] / n && e - s < shift_batch(n)) ++e;
+    group.push_back(s);
+    most = std::max(most, e - s);
+    s = e;
+  }
+  group.push_back(nshift);
+  // the adjoint's two lambda buffers are free in a forward-only run; more
+  // than one circuit takes states of its own
+  void* one[2] = {wsp(p, p->off_lam), wsp(p, p->off_lam + p->S)};
+  void* many[2] = {one[0], one[1]};
+  if (most > 1) {
+    CHK(ensure_shift(p, 2 * (size_t)most * p->S));
+    many[0] = p->d_shift;
+    many[1] = p->d_shift + (size_t)most * p->S;
+  }
+  // Two halves of the descriptor table: the host builds group k + 1 while the
+  // device runs group k, and waits for group k - 1, the last user of a half,
+  // before rewriting it.
+  const int half = P * (L + most);
+  CHK(ensure_small(p, 2 * half, p->nrows, p->nout));
   struct Ev {
     hipEvent_t e[4] = {nullptr, nullptr, nullptr, nullptr};
     ~Ev() {
@@ -2409,24 +2472,44 @@ static int mcclean_shift_run(qg_plan* p, const int32_t* axes, const double* angl
   for (int k = 0; k < 4; ++k) HIPCHK(hipEventCreate(&ev.e[k]));  // done[0], done[1], start, end
   const bool graph = p->use_graph;
   p->use_graph = false;  // suffixes differ in length: no graph replay here
+  const uint32_t ent = p->ent == QG_ENT_CNOT ? F_GATHER : F_CZ_PRE;
   int rc = QG_OK;
   hipError_t he = hipSuccess;
-  for (int s = 0; s < nshift && rc == QG_OK && he == hipSuccess; ++s) {
-    const int k = shift_param[s], i = k / n, h = s & 1;
-    if (s >= 2) he = hipEventSynchronize(ev.e[h]);
+  for (int k = 0; k + 1 < (int)group.size() && rc == QG_OK && he == hipSuccess; ++k) {
+    const int s0 = group[k], cnt = group[k + 1] - s0, i = shift_param[s0] / n, h = k & 1;
+    if (k >= 2) he = hipEventSynchronize(ev.e[h]);
     if (he != hipSuccess) break;
     int j = i - 1;
     while (j >= 0 && !layer_end[j]) --j;
-    ang[k] = angles[k] + shift_delta[s];
     p->launches.clear();
     int nd = h * half;
-    void* fin = mcclean_forward_suffix(p, axes, ang.data(), j + 1, j >= 0 ? layer_end[j] : start0, buf, nd);
-    ang[k] = angles[k];
-    if (s == 0) he = hipEventRecord(ev.e[2], c->stream);
+    // unshifted layers past the nearest stored state
+    const void* src = mcclean_forward_layers(p, axes, angles, j + 1, i, j >= 0 ? layer_end[j] : start0, one, 1, nd);
+    void* const* buf = cnt > 1 ? many : one;
+    char* out = (char*)(src == buf[0] ? buf[1] : buf[0]);
+    for (int g = 0; g < P; ++g) {  // the shifted layer
+      PassDesc& d = push_forward(p, p->geo[g], cnt, false, nd);
+      d.flags = F_ROT_A | F_STORE_A | (g == 0 ? (ent | (src ? F_LOAD_A : F_INIT_TAB)) : (uint32_t)F_LOAD_A);
+      layer_gates(d, p->geo[g], n, i, axes, angles);
+      for (int b = cnt - 1; b >= 0; --b) {
+        PassDesc& db = p->h_desc[p->launches.back().desc + b];
+        if (b) db = d;
+        db.a_out = out + (size_t)b * p->S;
+        db.a_in = g == 0 ? src : db.a_out;
+        const int q = shift_param[s0 + b] % n, bit = n - 1 - q;
+        const Geo& G = p->geo[g];
+        for (int lb = G.own_lo; lb < G.own_hi; ++lb)
+          if (((lb < G.c) ? lb : G.p + (lb - G.c)) == bit)
+            set_gate(db, lb, axes[i * n + q], angles[i * n + q] + shift_delta[s0 + b], 1.0);
+      }
+    }
+    void* const rest[2] = {out, out == (char*)buf[0] ? buf[1] : buf[0]};
+    const void* fin = mcclean_forward_layers(p, axes, angles, i + 1, L, out, rest, cnt, nd);
+    if (k == 0) he = hipEventRecord(ev.e[2], c->stream);
     if (he != hipSuccess) break;
     rc = run_launches(p, nd, h * half);
     if (rc != QG_OK) break;
-    he = on_shift(s, (const void*)fin);
+    he = on_shift(s0, cnt, fin);
     if (he == hipSuccess) he = hipEventRecord(ev.e[h], c->stream);
   }
   p->use_graph = graph;
@@ -2464,7 +2547,10 @@ extern "C" int qg_mcclean_shift_term_prob(qg_plan* p, const int32_t* axes, const
   CHK(pterm_table(p->n, terms, nterms, h));
   const int nt = nterms + 1;
   const size_t tb = ((sizeof(PTerm) * nt + 255) / 256) * 256;
-  const size_t pb = sizeof(double) * kTermBlocks * kTermPartRows;
+  size_t part = 0;  // whatever number of circuits a launch holds
+  for (int b = 1; b <= std::min(shift_batch(p->n), std::max(nshift, 1)); ++b)
+    part = std::max(part, simple_term_part(p->n, b));
+  const size_t pb = sizeof(double) * part;
   HIPCHK(hipSetDevice(p->ctx->device));
   DevBuf db;
   HIPCHK(hipMalloc(&db.p, tb + pb + sizeof(double) * (size_t)nt * std::max(nshift, 1)));
@@ -2473,9 +2559,9 @@ extern "C" int qg_mcclean_shift_term_prob(qg_plan* p, const int32_t* axes, const
   double* d_res = (double*)(db.p + tb + pb);
   HIPCHK(hipMemcpy(d_t, h.data(), sizeof(PTerm) * nt, hipMemcpyHostToDevice));
   CHK(mcclean_shift_run(p, axes, angles, ini_state, nterms ? nshift : 0, shift_param, shift_delta,
-                        [&](int s, const void* fin) {
+                        [&](int s, int count, const void* fin) {
                           return simple_term_expec(p->dtype, fin, p->n, d_t, nt, d_part, d_res + (size_t)s * nt,
-                                                   p->ctx->stream, h.data());
+                                                   p->ctx->stream, h.data(), count);
                         }));
   if (nshift == 0 || nterms == 0) return QG_OK;
   std::vector<double> res((size_t)nt * nshift);
@@ -2496,7 +2582,8 @@ struct SampleBufs {
   double* mass = nullptr;
 };
 
-static int sample_setup(int n, const int32_t* order, int64_t nu, const double* u, SampleBufs& b) {
+// states: how many are sampled at a time.
+static int sample_setup(int n, const int32_t* order, int64_t nu, const double* u, int states, SampleBufs& b) {
   if (n > 31) return fail(QG_ERR_UNSUPPORTED, "basis sampling needs n <= 31");
   const uint64_t N = 1ull << n;
   if (order)
@@ -2508,7 +2595,7 @@ static int sample_setup(int n, const int32_t* order, int64_t nu, const double* u
   const size_t ob = order ? ((N * 4 + 255) / 256) * 256 : 0;
   const size_t ub = (((size_t)nu * 8 + 255) / 256) * 256;
   const size_t ib = (((size_t)nu * 4 + 255) / 256) * 256;
-  HIPCHK(hipMalloc(&b.db.p, ob + ub + ib + nb * 8));
+  HIPCHK(hipMalloc(&b.db.p, ob + ub + ib + nb * 8 * states));
   b.order = order ? (int32_t*)b.db.p : nullptr;
   b.u = (double*)(b.db.p + ob);
   b.idx = (int32_t*)(b.db.p + ob + ub);
@@ -2527,11 +2614,11 @@ extern "C" int qg_mcclean_shift_sample(qg_plan* p, const int32_t* axes, const do
   HIPCHK(hipSetDevice(p->ctx->device));
   SampleBufs b;
   const int64_t nu = (int64_t)nshift * shots;
-  CHK(sample_setup(p->n, order, nu, u, b));
+  CHK(sample_setup(p->n, order, nu, u, std::min(shift_batch(p->n), std::max(nshift, 1)), b));
   CHK(mcclean_shift_run(p, axes, angles, ini_state, nshift, shift_param, shift_delta,
-                        [&](int s, const void* fin) {
+                        [&](int s, int count, const void* fin) {
                           return simple_sample_basis(p->dtype, fin, p->n, b.order, b.u + (size_t)s * shots, shots,
-                                                     b.idx + (size_t)s * shots, b.mass, 1, p->ctx->stream);
+                                                     b.idx + (size_t)s * shots, b.mass, count, p->ctx->stream);
                         }));
   if (nu) HIPCHK(hipMemcpy(idx, b.idx, (size_t)nu * 4, hipMemcpyDeviceToHost));
   return QG_OK;
@@ -3004,6 +3091,156 @@ static int qaoa_run(qg_plan* p, int B, const qg_term* terms, const int32_t* term
   return QG_OK;
 }
 
+// Shots of the shifted QAOA circuits of Qaoa.sample_grad_dense (qaoa.py:83-158):
+// layer i's shifts are exp(-+i pi/4 C_j) after the cost phase (component j of
+// the classical Hamiltonian) and RX(+-pi/2) on qubit q after the mixer.  The
+// unshifted circuit keeps both of a layer's states; the shifted copies of one
+// state run the rest of the circuit together, every pass one launch with one
+// descriptor (push_forward), and are sampled together.
+extern "C" int qg_qaoa_shift_sample(qg_plan* p, const qg_term* terms, int nterms, const double* betas,
+                                    const double* gammas, const double* ini_state, const qg_term* mterms, int nm,
+                                    double* expec, int shots, const double* u, int32_t* idx) {
+  if (!p || p->kind != PK_QAOA) return fail(QG_ERR_INVALID, "not a QAOA plan");
+  if (!betas || !gammas || !expec || !u || !idx || nterms < 0 || (nterms > 0 && !terms))
+    return fail(QG_ERR_INVALID, "NULL argument");
+  if (shots < 1) return fail(QG_ERR_INVALID, "shots must be >= 1");
+  const int n = p->n, L = p->L, P = (int)p->geo.size();
+  if (n > 31) return fail(QG_ERR_UNSUPPORTED, "basis sampling needs n <= 31");
+  ObsSplit obs;
+  CHK(split_observable(n, terms, nterms, obs));
+  if (!obs.xy.empty())
+    return fail(QG_ERR_INVALID, "the QAOA classical Hamiltonian takes z / zz terms only (state.py:268-271)");
+  if (nterms > p->max_terms) return fail(QG_ERR_INVALID, "too many observable terms");
+  bool integral = true;
+  double W = 0.0;
+  for (const DTerm& t : obs.diag) {
+    W += std::fabs(t.w);
+    if (t.w != std::rint(t.w)) integral = false;
+  }
+  const int phase = (integral && 2.0 * W + 1.0 <= (double)kLutMax) ? 1 : 2;
+  const int Wi = phase == 1 ? (int)W : 0, lut_len = 2 * Wi + 1;
+  qg_ctx* c = p->ctx;
+  HIPCHK(hipSetDevice(c->device));
+  // states: the history (after each phase and each mixer), the initial state
+  // when given, and the copies of a batch
+  const int per_layer = 2 * (nterms + n);
+  const int most = std::min(shift_batch(n), 2 * std::max(nterms, n));
+  const size_t S = p->S;
+  CHK(ensure_shift(p, (size_t)(2 * L + 1 + most) * S));
+  auto hist = [&](int k) { return (void*)(p->d_shift + (size_t)k * S); };
+  char* copies = p->d_shift + (size_t)(2 * L + 1) * S;
+  SampleBufs b;
+  CHK(sample_setup(n, nullptr, (int64_t)L * per_layer * shots, u, most, b));
+  // the shift operations of a layer (the same for every layer)
+  std::vector<ShiftOp> ops((size_t)per_layer);
+  for (int j = 0; j < nterms; ++j)
+    for (int k = 0; k < 2; ++k) {
+      const double phi = (k == 0 ? 1 : -1) * (M_PI / 4) * obs.diag[j].w;
+      const uint32_t m = (1u << obs.diag[j].a) | (obs.diag[j].b >= 0 ? 1u << obs.diag[j].b : 0u);
+      ops[2 * j + k] = {0, m, std::cos(phi), std::sin(phi)};
+    }
+  for (int q = 0; q < n; ++q)
+    for (int k = 0; k < 2; ++k) {
+      const double phi = (k == 0 ? 1 : -1) * (M_PI / 4);
+      ops[2 * (nterms + q) + k] = {1, 1u << (n - 1 - q), std::cos(phi), std::sin(phi)};
+    }
+  DevBuf ob;
+  HIPCHK(hipMalloc(&ob.p, sizeof(ShiftOp) * ops.size()));
+  HIPCHK(hipMemcpy(ob.p, ops.data(), sizeof(ShiftOp) * ops.size(), hipMemcpyHostToDevice));
+  const ShiftOp* d_ops = (const ShiftOp*)ob.p;
+  if (nterms)
+    HIPCHK(hipMemcpy(p->d_terms, obs.diag.data(), sizeof(DTerm) * nterms, hipMemcpyHostToDevice));
+  p->h_terms = obs.diag;
+  DevBuf lb;
+  if (phase == 1) {
+    // exp(-i gamma k), k = -W .. W, per layer
+    std::vector<double> lut((size_t)L * lut_len * 2);
+    for (int i = 0; i < L; ++i)
+      for (int k = -Wi; k <= Wi; ++k) {
+        lut[((size_t)i * lut_len + Wi + k) * 2] = std::cos(gammas[i] * (double)std::abs(k));
+        lut[((size_t)i * lut_len + Wi + k) * 2 + 1] =
+            (k > 0 ? -1.0 : 1.0) * std::sin(gammas[i] * (double)std::abs(k));
+      }
+    HIPCHK(hipMalloc(&lb.p, sizeof(double) * lut.size()));
+    HIPCHK(hipMemcpy(lb.p, lut.data(), sizeof(double) * lut.size(), hipMemcpyHostToDevice));
+  }
+  if (ini_state) {
+    const size_t N = 1ull << n;
+    DevBuf tmp;
+    HIPCHK(hipMalloc(&tmp.p, N * 16));
+    HIPCHK(hipMemcpyAsync(tmp.p, ini_state, N * 16, hipMemcpyHostToDevice, c->stream));
+    HIPCHK(simple_convert_in(p->dtype, tmp.p, hist(2 * L), n, c->stream));
+    HIPCHK(hipStreamSynchronize(c->stream));
+  }
+  // descriptors go out as they are built and are not rewritten while in
+  // flight: when the table is full, the stream is waited for
+  const int table = 512;
+  CHK(ensure_small(p, std::max(table, 2 * P * L), p->nrows, p->nout));
+  const size_t split_bound = (size_t)std::max(1, nterms) * table;
+  p->launches.clear();
+  CHK(stream_begin(p, split_bound));
+  int nd = 0;
+  // cost phase (ph) and mixer (mix) of layer i on `count` states, in -> out
+  auto emit = [&](const void* in, void* out, int count, int i, bool ph, bool mix) -> int {
+    if (nd + P > table) {
+      HIPCHK(hipStreamSynchronize(c->stream));
+      p->launches.clear();
+      p->h_cterms.clear();
+      p->stream_next = 0;
+      nd = 0;
+    }
+    const GateAB ab = gate_ab(betas[i], 1.0);
+    for (int g = 0; g < (mix ? P : 1); ++g) {
+      const Geo& G = p->geo[g];
+      PassDesc& d = push_forward(p, G, count, true, nd);
+      Launch& l = p->launches.back();
+      while (l.grid > 1 && (uint64_t)l.grid * count > (uint64_t)p->wg_per_cu * c->num_cu) l.grid >>= 1;
+      l.phase = phase;
+      d.ndterms = nterms;
+      d.lut_off = Wi;
+      d.bstride = (int64_t)S;
+      d.a_in = g == 0 ? in : out;
+      d.a_out = out;
+      d.flags = F_STORE_A | (phase == 1 ? F_PHASE_LUT : 0u) | (d.a_in ? F_LOAD_A : F_INIT_TAB);
+      if (ph && g == 0) {
+        d.flags |= F_PHASE_PRE;
+        d.phase_gamma = gammas[i];
+        d.lut = phase == 1 ? (const double*)lb.p + (size_t)i * lut_len * 2 : nullptr;
+      }
+      if (mix) {
+        d.flags |= F_ROT_A;
+        for (int k = G.own_lo; k < G.own_hi; ++k) {
+          d.gtype[k] = G_X;
+          d.ga[k] = ab.a;
+          d.gb[k] = ab.b;
+        }
+      }
+    }
+    return stream_flush(p);
+  };
+  for (int i = 0; i < L; ++i) {
+    const void* prev = i ? hist(2 * i - 1) : (ini_state ? hist(2 * L) : nullptr);
+    CHK(emit(prev, hist(2 * i), 1, i, true, false));
+    CHK(emit(hist(2 * i), hist(2 * i + 1), 1, i, false, true));
+  }
+  for (int i = 0; i < L; ++i)
+    for (int kind = 0; kind < 2; ++kind) {
+      const int first = kind == 0 ? 0 : 2 * nterms, all = kind == 0 ? 2 * nterms : 2 * n;
+      for (int s = 0; s < all; s += most) {
+        const int count = std::min(most, all - s);
+        HIPCHK(simple_shift_copies(p->dtype, hist(2 * i + kind), copies, n, d_ops + first + s, count, c->stream));
+        if (kind == 0) CHK(emit(copies, copies, count, i, false, true));
+        for (int j = i + 1; j < L; ++j) CHK(emit(copies, copies, count, j, true, true));
+        const size_t at = ((size_t)i * per_layer + first + s) * shots;
+        HIPCHK(simple_sample_basis(p->dtype, copies, n, nullptr, b.u + at, shots, b.idx + at, b.mass, count,
+                                   c->stream));
+      }
+    }
+  CHK(term_expec(c, p->dtype, hist(2 * L - 1), n, mterms, nm, expec));
+  HIPCHK(hipMemcpy(idx, b.idx, (size_t)L * per_layer * shots * 4, hipMemcpyDeviceToHost));
+  return QG_OK;
+}
+
 extern "C" int qg_qaoa_grad_run(qg_plan* p, int B, const qg_term* terms, const int32_t* term_off,
                                 const double* betas, const double* gammas, double* E_out, double* grad_out) {
   return qaoa_run(p, B, terms, term_off, betas, gammas, nullptr, E_out, grad_out, true);
@@ -3272,7 +3509,7 @@ extern "C" int qg_state_sample_basis(qg_state* st, const int32_t* order, int sho
   if (shots < 1) return fail(QG_ERR_INVALID, "shots must be >= 1");
   HIPCHK(hipSetDevice(st->ctx->device));
   SampleBufs b;
-  CHK(sample_setup(st->n, order, shots, u, b));
+  CHK(sample_setup(st->n, order, shots, u, 1, b));
   HIPCHK(simple_sample_basis(st->dtype, st->v, st->n, b.order, b.u, shots, b.idx, b.mass, 1, st->ctx->stream));
   HIPCHK(hipStreamSynchronize(st->ctx->stream));
   HIPCHK(hipMemcpy(idx, b.idx, (size_t)shots * 4, hipMemcpyDeviceToHost));

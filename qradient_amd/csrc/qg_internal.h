@@ -69,6 +69,14 @@ constexpr int kTermPartRows = kDiagTermsPerLaunch;  // partial rows a term launc
 constexpr int kTermBlocks = 2048;    // workgroups of a term pass (partials per term)
 constexpr int kSampleBlock = 1024;   // positions per block of the basis sampler
 
+// One shifted copy of a state: kind 0 multiplies by exp(-i phi z), z = (-1)^popcount(x & mask)
+// (c = cos(phi), s = sin(phi)); kind 1 rotates bit `mask` about X, cos I - i sin X.
+struct ShiftOp {
+  int32_t kind;
+  uint32_t mask;
+  double c, s;
+};
+
 struct PassDesc {
   // geometry: local bits = [0, c) U [p, p + K - c); tile bits = the rest, in order
   int32_t n, K, t, c, p;
@@ -77,6 +85,9 @@ struct PassDesc {
   int32_t row_base;      // first partial row written by this pass (-1: none)
   const void* a_in;
   void* a_out;
+  // forward passes: nonzero = every circuit of a batched launch takes this one
+  // descriptor, circuit y's states y * bstride bytes behind a_in and a_out
+  int64_t bstride;
   const void* b_in;
   void* b_out;
   // gates, indexed by local bit: U = cos(phi) I - i sin(phi) P with the

@@ -686,7 +686,7 @@ __device__ __forceinline__ void tile_addresses(const PassDesc* __restrict__ d, b
 // ---------------------------------------------------------------------------
 template <class S, int R, bool TWO, int PH, bool POST, bool BIG, bool WIDE = false>
 __device__ __forceinline__ void run_pass(const PassDesc* __restrict__ d, void* lds, uint32_t tid_in, uint32_t blk,
-                                         uint32_t nblk) {
+                                         uint32_t nblk, size_t boff = 0) {
   constexpr int A = 1 << R;
   typedef typename Store<S>::G G;  // HBM element type
   typedef typename Store<S>::L LT; // LDS tile element type
@@ -787,6 +787,10 @@ __device__ __forceinline__ void run_pass(const PassDesc* __restrict__ d, void* l
     return xcd ? (blk % 8) * per_x + r * slots + blk / 8 : blk + r * nblk;
   };
 
+  // boff: see PassDesc::bstride (read where it is used: adjoint passes have no scalar registers to spare)
+  auto a_in = [&]() __attribute__((always_inline)) -> const void* {
+    return TWO ? d->a_in : (const char*)d->a_in + boff;
+  };
   Cx<G> ra[A];
   Cx<G> rb[TWO ? A : 1];
   // Issues the loads of tile tt into ra / rb (addresses derived from a
@@ -812,12 +816,12 @@ __device__ __forceinline__ void run_pass(const PassDesc* __restrict__ d, void* l
         asm volatile("");
 #pragma unroll
         for (int a = 0; a < A; ++a)
-          ra[a] = BIG ? Stor<G>::template ld_big<G>(d->a_in, adr[a]) : Stor<G>::template ld_o_nt<G>(d->a_in, adr[a]);
+          ra[a] = BIG ? Stor<G>::template ld_big<G>(a_in(), adr[a]) : Stor<G>::template ld_o_nt<G>(a_in(), adr[a]);
         asm volatile("");
       } else {
 #pragma unroll
         for (int a = 0; a < A; ++a)
-          ra[a] = BIG ? Stor<G>::template ld_big<G>(d->a_in, adr[a]) : Stor<G>::template ld_o<G>(d->a_in, adr[a]);
+          ra[a] = BIG ? Stor<G>::template ld_big<G>(a_in(), adr[a]) : Stor<G>::template ld_o<G>(a_in(), adr[a]);
       }
     } else {
 #pragma unroll
@@ -1145,8 +1149,8 @@ __device__ __forceinline__ void run_pass(const PassDesc* __restrict__ d, void* l
     if (!RF && (flags & F_STORE_A)) {
 #pragma unroll
       for (int a = 0; a < A; ++a) {
-        if (BIG) Stor<G>::st_big(d->a_out, adr[a], xa[a]);
-        else Stor<G>::st_o(d->a_out, adr[a], xa[a]);
+        if (BIG) Stor<G>::st_big(TWO ? d->a_out : (char*)d->a_out + boff, adr[a], xa[a]);
+        else Stor<G>::st_o(TWO ? d->a_out : (char*)d->a_out + boff, adr[a], xa[a]);
       }
     }
     if constexpr (TWO) {
@@ -1191,17 +1195,31 @@ __device__ __forceinline__ void run_pass(const PassDesc* __restrict__ d, void* l
 }
 
 // blockIdx.y selects one of gridDim.y consecutive descriptors: a batched
-// launch runs the same pass of gridDim.y independent circuits.
+// launch runs the same pass of gridDim.y independent circuits.  Forward passes
+// whose circuits differ in their states only share one descriptor (bstride).
+template <bool TWO>
+__device__ __forceinline__ size_t batch_desc(const PassDesc*& d) {
+  if constexpr (!TWO) {
+    const int64_t bs = ldc(&d->bstride, 0);
+    if (bs) return (size_t)bs * blockIdx.y;
+  }
+  d += blockIdx.y;
+  return 0;
+}
 template <class S, int R, bool TWO, int PH, bool POST, bool BIG>
 __global__ __launch_bounds__(512) void k_pass(const PassDesc* __restrict__ d) {
   extern __shared__ __align__(16) char lds_dyn[];
-  run_pass<S, R, TWO, PH, POST, BIG>(d + blockIdx.y, lds_dyn, threadIdx.x, blockIdx.x, gridDim.x);
+  const PassDesc* dd = d;
+  const size_t boff = batch_desc<TWO>(dd);
+  run_pass<S, R, TWO, PH, POST, BIG>(dd, lds_dyn, threadIdx.x, blockIdx.x, gridDim.x, boff);
 }
 // 1024-thread workgroups: 14 local bits with 16 amplitudes per thread.
 template <class S, int R, bool TWO, int PH, bool POST, bool BIG>
 __global__ __launch_bounds__(1024) void k_pass_w(const PassDesc* __restrict__ d) {
   extern __shared__ __align__(16) char lds_dyn[];
-  run_pass<S, R, TWO, PH, POST, BIG, true>(d + blockIdx.y, lds_dyn, threadIdx.x, blockIdx.x, gridDim.x);
+  const PassDesc* dd = d;
+  const size_t boff = batch_desc<TWO>(dd);
+  run_pass<S, R, TWO, PH, POST, BIG, true>(dd, lds_dyn, threadIdx.x, blockIdx.x, gridDim.x, boff);
 }
 // Variants built with 1024-thread workgroups: complex64 (FP32 tiles),
 // 16 amplitudes per thread, phase-free forward and reduce-first adjoint passes.

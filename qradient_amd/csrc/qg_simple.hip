@@ -130,8 +130,8 @@ __global__ void k_dot(const typename V2<S>::T* __restrict__ a, const typename V2
   if (threadIdx.x == 0) part[blockIdx.x] = red[0];
 }
 
-// part[k * gridDim.x + block] = this block's share of <P_k> for the terms
-// t[0, nt), nt <= kTermsPerLaunch, in FP64:
+// part[(b * nt + k) * gridDim.x + block] = this block's share of <P_k> in state
+// b = blockIdx.y (at v + b * N) for the terms t[0, nt), nt <= kTermsPerLaunch, in FP64:
 //   Z / ZZ: |v_x|^2 z(x);  X: Re(conj(v_x) v_{x^m});  Y: Re(conj(v_x) (Y v)_x);
 //   identity (kind 3): |v_x|^2
 // with (Y v)_x = -i v_{x^m} on bit 0 and +i v_{x^m} on bit 1.  Fixed order:
@@ -140,6 +140,8 @@ template <class S>
 __global__ void __launch_bounds__(256) k_term_expec(const typename V2<S>::T* __restrict__ v, uint32_t N,
                                                     const PTerm* __restrict__ t, int nt, double* __restrict__ part) {
   __shared__ double red[4][kTermsPerLaunch];
+  v += (size_t)blockIdx.y * N;
+  part += (size_t)blockIdx.y * nt * gridDim.x;
   double acc[kTermsPerLaunch];
 #pragma unroll
   for (int k = 0; k < kTermsPerLaunch; ++k) acc[k] = 0.0;
@@ -189,52 +191,71 @@ __global__ void __launch_bounds__(256) k_term_expec(const typename V2<S>::T* __r
 // (2^sb amplitudes), so x = g + j 2^sb with g the thread's global index and j
 // the iteration: the sign splits into (-1)^popc(g & m_k), fixed per thread,
 // and (-1)^popc(j & (m_k >> sb)), the same for the whole grid at iteration j.
-// Each thread sums (-1)^popc(j & mh_k) |v_x|^2 over its iterations (one FMA
-// per term and amplitude) and applies its own sign at the end.
-// Up to kDiagTermsPerLaunch terms per launch: the per-thread sign of a term
-// is recomputed from its mask after the loop, so a term costs one FP64
-// accumulator in the loop.
+// A thread takes 16 iterations at a time: their Walsh-Hadamard transform (64
+// additions) holds the sixteen probabilities summed with every sign pattern of
+// the low four bits of j, so a term costs one read of the pattern it needs
+// (from the thread's own LDS column, the pattern being uniform) and one
+// addition per 16 amplitudes.
+// A sign select and an FMA per term and amplitude, as before, was bound by
+// those: 24 terms at 24 qubits, complex64, 75 us -> 53 us (one read of
+// the state at the copy rate is 22 us).
 template <class S>
 __global__ void __launch_bounds__(256) k_term_expec_diag(const typename V2<S>::T* __restrict__ v, uint32_t N,
                                                          const PTerm* __restrict__ t, int nt, int sb,
                                                          double* __restrict__ part) {
   constexpr int NT = kDiagTermsPerLaunch;
+  __shared__ double wht[16][256];
   __shared__ double red[4][NT];
+  v += (size_t)blockIdx.y * N;
+  part += (size_t)blockIdx.y * nt * gridDim.x;
   const uint32_t g = blockIdx.x * blockDim.x + threadIdx.x;
   auto mask_of = [&](int k) -> uint32_t {
     return (k < nt && t[k].kind == 0) ? (1u << t[k].a) | (t[k].b >= 0 ? (1u << t[k].b) : 0u) : 0u;
   };
-  uint32_t mh[NT];
   double acc[NT];
 #pragma unroll
-  for (int k = 0; k < NT; ++k) {
-    const uint32_t m = mask_of(k);
-    mh[k] = sb < 32 ? m >> sb : 0u;
-    acc[k] = 0.0;
-  }
+  for (int k = 0; k < NT; ++k) acc[k] = 0.0;
   const uint32_t iters = N >> sb;  // N and the stride are powers of two
-  for (uint32_t j = 0; j < iters; j += 2) {
-    const typename V2<S>::T a0 = v[g + (j << sb)];
-    const double p0 = (double)a0.x * a0.x + (double)a0.y * a0.y;
-    double p1 = 0.0;
-    if (j + 1 < iters) {
-      const typename V2<S>::T a1 = v[g + ((j + 1) << sb)];
-      p1 = (double)a1.x * a1.x + (double)a1.y * a1.y;
+  for (uint32_t jj = 0; jj * 16u < iters; ++jj) {
+    double p[16];
+#pragma unroll
+    for (uint32_t r = 0; r < 16; ++r) {
+      // fewer than 16 iterations in all: the missing ones hold nothing
+      const uint32_t j = jj * 16u + r;
+      p[r] = 0.0;
+      if (j < iters) {
+        const typename V2<S>::T a = v[g + (j << sb)];
+        p[r] = (double)a.x * a.x + (double)a.y * a.y;
+      }
     }
 #pragma unroll
+    for (int h = 1; h < 16; h <<= 1)
+#pragma unroll
+      for (int r = 0; r < 16; ++r)
+        if (!(r & h)) {
+          const double x = p[r], y = p[r | h];
+          p[r] = x + y;
+          p[r | h] = x - y;
+        }
+#pragma unroll
+    for (int r = 0; r < 16; ++r) wht[r][threadIdx.x] = p[r];
+    // (the thread reads its own column only: no barrier)
+#pragma unroll
     for (int k = 0; k < NT; ++k) {
-      const double s0 = (__popc(j & mh[k]) & 1u) ? -1.0 : 1.0;
-      const double s1 = (__popc((j + 1) & mh[k]) & 1u) ? -1.0 : 1.0;
-      acc[k] = __builtin_fma(s1, p1, __builtin_fma(s0, p0, acc[k]));
+      if (k < nt) {
+        const uint32_t m = sb < 32 ? mask_of(k) >> sb : 0u;
+        const double w = wht[m & 15u][threadIdx.x];
+        acc[k] += (__popc(jj & (m >> 4)) & 1) ? -w : w;
+      }
     }
   }
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
 #pragma unroll
   for (int k = 0; k < NT; ++k) {
-    const double sl = (__popc(g & mask_of(k)) & 1u) ? -1.0 : 1.0;
-    double s = sl * acc[k];
-    for (int o = 32; o > 0; o >>= 1) s += __shfl_xor(s, o, 64);
-    if (lane == 0) red[wave][k] = s;
+    if (k < nt) {
+      const double s = wave_sum((__popc(g & mask_of(k) & ((1u << sb) - 1u)) & 1) ? -acc[k] : acc[k], 64);
+      if (lane == 0) red[wave][k] = s;
+    }
   }
   __syncthreads();
   if ((int)threadIdx.x < nt) {
@@ -243,22 +264,46 @@ __global__ void __launch_bounds__(256) k_term_expec_diag(const typename V2<S>::T
   }
 }
 
-// out[k] = sum of part[k * np + 0 .. np): one 256-thread workgroup per term,
-// coalesced strided partial sums, then a fixed-order tree.
+// out[b * ldo + k] = sum of part[(b * nt + k) * np + 0 .. np), b = blockIdx.y: one
+// 256-thread workgroup per term, coalesced strided partial sums, then a
+// fixed-order tree.
 __global__ void __launch_bounds__(256) k_sum_terms(const double* __restrict__ part, int np, int nt,
-                                                   double* __restrict__ out) {
-  __shared__ double red[256];
+                                                   double* __restrict__ out, int ldo) {
+  __shared__ double red[4];
   const int k = blockIdx.x;
   if (k >= nt) return;
+  part += ((size_t)blockIdx.y * nt + k) * np;
   double s = 0.0;
-  for (int i = threadIdx.x; i < np; i += 256) s += part[(size_t)k * np + i];
-  red[threadIdx.x] = s;
+  for (int i = threadIdx.x; i < np; i += 256) s += part[i];
+  s = wave_sum(s, 64);
+  if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = s;
   __syncthreads();
-  for (int h = 128; h > 0; h >>= 1) {
-    if ((int)threadIdx.x < h) red[threadIdx.x] += red[threadIdx.x + h];
-    __syncthreads();
+  if (threadIdx.x == 0) out[(size_t)blockIdx.y * ldo + k] = ((red[0] + red[1]) + red[2]) + red[3];
+}
+
+// Shifted copies of one state, copy b = blockIdx.y at out + b * N: op[b] applied to `in`.
+template <class S>
+__global__ void __launch_bounds__(256) k_shift_copies(const typename V2<S>::T* __restrict__ in,
+                                                      typename V2<S>::T* __restrict__ out, uint32_t N,
+                                                      const ShiftOp* __restrict__ op) {
+  const uint32_t x = blockIdx.x * blockDim.x + threadIdx.x;
+  if (x >= N) return;
+  const ShiftOp o = op[blockIdx.y];
+  const double re = in[x].x, im = in[x].y;
+  double r, i;
+  if (o.kind == 0) {
+    const double s = (__popc(x & o.mask) & 1) ? -o.s : o.s;
+    r = o.c * re + s * im;
+    i = o.c * im - s * re;
+  } else {
+    const double pr = in[x ^ o.mask].x, pi = in[x ^ o.mask].y;
+    r = o.c * re + o.s * pi;
+    i = o.c * im - o.s * pr;
   }
-  if (threadIdx.x == 0) out[k] = red[0];
+  typename V2<S>::T w;
+  w.x = (S)r;
+  w.y = (S)i;
+  out[(size_t)blockIdx.y * N + x] = w;
 }
 
 // *out = sum of part[0, np): one 256-thread workgroup, fixed-order tree.
@@ -490,16 +535,33 @@ hipError_t simple_dot(int dtype, const void* a, const void* b, int n, int mode, 
   return hipGetLastError();
 }
 
-// out[k] = <P_k> for the nt terms t (device arrays); part needs
-// kTermBlocks * kTermPartRows doubles.  h_t: a host copy of t, or NULL; with
-// it, a run of up to kDiagTermsPerLaunch diagonal terms takes one launch of
-// the mask kernel, other terms go kTermsPerLaunch at a time to the general
-// kernel.  Each term's sum does not depend on the launch it is in.
+// Workgroups per state of a term launch over `batch` states: 16 amplitudes
+// per thread where the states fill the device that way (a thread's final
+// cross-lane sums cost as much as some 30 amplitudes), at most kTermBlocks in all.
+static int term_blocks(uint32_t N, int batch) {
+  int most = kTermBlocks / batch;
+  int b = 1;
+  while (b * 2 <= most && (uint64_t)b * 2 * 256 * 16 <= N) b *= 2;
+  return b;
+}
+
+// Doubles of `part` that simple_term_expec needs.
+size_t simple_term_part(int n, int batch) {
+  return (size_t)term_blocks((uint32_t)(1ull << n), batch) * kTermPartRows * batch;
+}
+
+// out[b * nt + k] = <P_k> in state b for the nt terms t (device arrays) and
+// the `batch` states behind each other at v; part: simple_term_part doubles.
+// h_t: a host copy of t, or NULL; with it, a run of up to kDiagTermsPerLaunch
+// diagonal terms takes one launch of the mask kernel, other terms go
+// kTermsPerLaunch at a time to the general kernel.  Each term's sum does not
+// depend on the other terms of its launch.
 hipError_t simple_term_expec(int dtype, const void* v, int n, const PTerm* t, int nt, double* part, double* out,
-                             hipStream_t st, const PTerm* h_t) {
-  if (n < 1 || n > kSimpleMaxN) return hipErrorInvalidValue;
+                             hipStream_t st, const PTerm* h_t, int batch) {
+  if (n < 1 || n > kSimpleMaxN || batch < 1 || batch > 65535) return hipErrorInvalidValue;
   const uint32_t N = (uint32_t)(1ull << n);
-  const int blocks = (int)((N + 255) / 256) < kTermBlocks ? (int)((N + 255) / 256) : kTermBlocks;
+  const int blocks = term_blocks(N, batch);
+  const dim3 grid(blocks, batch);
   auto is_diag = [&](int k) { return h_t[k].kind == 0 || h_t[k].kind == 3; };
   for (int k0 = 0, m = 0; k0 < nt; k0 += m) {
     // the diagonal kernel needs one thread per amplitude or fewer: N >= 256
@@ -509,16 +571,26 @@ hipError_t simple_term_expec(int dtype, const void* v, int n, const PTerm* t, in
     const bool diag = m > 0;
     if (!diag) m = nt - k0 < kTermsPerLaunch ? nt - k0 : kTermsPerLaunch;
     if (diag) {
-      int sb = 0;
+      int sb = 8;
       while ((1u << sb) < (uint32_t)blocks * 256u) ++sb;
-      QG_DT_SWITCH(dtype, hipLaunchKernelGGL(k_term_expec_diag<S>, dim3(blocks), dim3(256), 0, st,
+      QG_DT_SWITCH(dtype, hipLaunchKernelGGL(k_term_expec_diag<S>, grid, dim3(256), 0, st,
                                              (const typename V2<S>::T*)v, N, t + k0, m, sb, part));
     } else {
-      QG_DT_SWITCH(dtype, hipLaunchKernelGGL(k_term_expec<S>, dim3(blocks), dim3(256), 0, st,
+      QG_DT_SWITCH(dtype, hipLaunchKernelGGL(k_term_expec<S>, grid, dim3(256), 0, st,
                                              (const typename V2<S>::T*)v, N, t + k0, m, part));
     }
-    hipLaunchKernelGGL(k_sum_terms, dim3(m), dim3(256), 0, st, (const double*)part, blocks, m, out + k0);
+    hipLaunchKernelGGL(k_sum_terms, dim3(m, batch), dim3(256), 0, st, (const double*)part, blocks, m, out + k0, nt);
   }
+  return hipGetLastError();
+}
+
+// out state b = op[b] applied to in, b < batch (op: device array).
+hipError_t simple_shift_copies(int dtype, const void* in, void* out, int n, const ShiftOp* op, int batch,
+                               hipStream_t st) {
+  if (n < 1 || n > kSimpleMaxN || batch < 1 || batch > 65535) return hipErrorInvalidValue;
+  const uint32_t N = (uint32_t)(1ull << n);
+  QG_DT_SWITCH(dtype, hipLaunchKernelGGL(k_shift_copies<S>, dim3((unsigned)((N + 255) / 256), batch), dim3(256), 0, st,
+                                         (const typename V2<S>::T*)in, (typename V2<S>::T*)out, N, op));
   return hipGetLastError();
 }
 
