@@ -14,8 +14,9 @@ adjoint method, each statevector counted once per layer: per layer the
 forward sweep reads and writes psi (2 S) and the reverse sweep reads and
 writes psi and lambda (4 S), plus S for the initial state and 2 S for
 lambda = O psi with E, so B_alg = (6 L + 3) S for the whole run (S = 2^n
-amplitudes x bytes per amplitude).  A launch that covers one of the P passes
-of a layer is credited 1/P of its layer's bytes.  ``roofline.achieved`` is
+amplitudes x bytes per amplitude).  With P passes per layer a launch is
+credited 1/P of a layer's bytes; multi-layer passes make P less than 1, and a
+launch then moves fewer bytes than it is credited (``hbm`` has those).  ``roofline.achieved`` is
 the dominant kernel's algorithmic bytes per launch over its average launch
 time (HIP events on the library's stream around every launch of the last
 timed step: events between all launches would add about 0.8 ms per step);
@@ -93,15 +94,16 @@ def roofline(per, state_bytes, steps, layers):
     """Dominant launch class of the timed steps and its algorithmic rate.
 
     ``per``: (ms, kinds) of every launch of the ``steps`` profiled steps; kinds
-    0 forward pass, 1 adjoint two-state pass, 2 last forward pass fused with
-    lambda = O psi and E.  With P passes per layer, a forward launch is
-    credited 2 S / P, an adjoint launch 4 S / P and the fused one 2 S / P + 2 S.
+    0 forward pass, 1 adjoint two-state pass, 2 lambda = O psi with E.  With P
+    passes per layer (a fraction where a pass runs several layers), a forward
+    launch is credited 2 S / P, an adjoint launch 4 S / P and the observable's
+    2 S.
     """
     ms = np.concatenate([p[0] for p in per])
     kinds = np.concatenate([p[1] for p in per])
-    P = int(round(float(np.sum(kinds == 1)) / (steps * layers)))
+    P = float(np.sum(kinds == 1)) / (steps * layers)
     S = state_bytes
-    alg = {0: 2 * S / P, 1: 4 * S / P, 2: 2 * S / P + 2 * S}
+    alg = {0: 2 * S / P, 1: 4 * S / P, 2: 2 * S}
     totals = {k: ms[kinds == k].sum() for k in set(kinds.tolist())}
     dom = max((k for k in totals if k in alg), key=totals.get)
     avg_ms = float(ms[kinds == dom].mean())
@@ -553,7 +555,7 @@ def main():
         'E': c64['E'],
         'roofline': {'bound': 'hbm', 'achieved': rf['achieved'], 'peak': HBM_PEAK_GBS, 'unit': 'GB/s',
                      'frac': rf['achieved'] / HBM_PEAK_GBS, 'traffic': traffic,
-                     'kernel': {0: 'forward pass', 1: 'adjoint two-state pass', 2: 'forward + observable pass'}[
+                     'kernel': {0: 'forward pass', 1: 'adjoint two-state pass', 2: 'observable pass'}[
                          rf['kind']],
                      'avg_launch_ms': rf['avg_ms'], 'algorithmic_bytes_per_launch': rf['alg_bytes'],
                      'passes_per_layer': rf['passes_per_layer'],

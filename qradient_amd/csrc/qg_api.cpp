@@ -13,9 +13,13 @@
 
 #include "../../include/qradient_amd.h"
 #include "qg_internal.h"
+#include "qg_sweep_plan.hpp"
 
 namespace qg {
 hipError_t set_pass_attributes();
+hipError_t set_sweep_attributes();
+hipError_t launch_sweep(int dtype, bool two, const SweepDesc* d, int K, int grid, int batch, int n, hipStream_t st,
+                        int* occ, int tab);
 hipError_t launch_pass(int dtype, int R, bool two, int phase, bool post, const PassDesc* d, int K, int grid,
                        int batch, int threads, int n, hipStream_t st, int* occ, int tab);
 hipError_t launch_finalize(int nout, const int* ptr, const int* rows, const int* cnt, const double* scale,
@@ -151,7 +155,7 @@ extern "C" int qg_ctx_create(int device, void* stream, qg_ctx** out) {
     c->own_stream = true;
   }
   if (hipEventCreate(&c->ev0) != hipSuccess || hipEventCreate(&c->ev1) != hipSuccess ||
-      set_pass_attributes() != hipSuccess || set_fused_attributes() != hipSuccess ||
+      set_pass_attributes() != hipSuccess || set_sweep_attributes() != hipSuccess || set_fused_attributes() != hipSuccess ||
       fused_desc_size() != sizeof(FusedDescH) ||
       hipHostMalloc((void**)&c->noalloc_host, kNoAllocScratchBytes, hipHostMallocDefault) != hipSuccess) {
     if (c->noalloc_host) (void)hipHostFree(c->noalloc_host);
@@ -387,6 +391,7 @@ struct Launch {
   int desc;  // index into the descriptor table (first of `batch` consecutive ones)
   int batch = 1;
   bool shared = false;  // one descriptor for the whole batch (PassDesc::bstride)
+  bool sweep = false;   // a multi-layer pass: desc indexes the plan's sweep descriptors
   int K = 0;
   bool post = false;  // the pass has diagonal ops after its gates (set at launch from the flags)
   int tab = 0;        // bytes of the table the pass stages in LDS (set at launch)
@@ -474,6 +479,13 @@ struct qg_plan {
   double* h_out = nullptr;
   int nout = 0;
   std::vector<Launch> launches;
+  // multi-layer passes of a McClean plan (qg_sweep.hpp)
+  std::vector<PlanPass> sweep;
+  int sweep_rounds = 0;     // rounds of all of them
+  int sweep_for[5] = {0, 0, 0, 0, 0};  // n, L, entangler, local bits, contiguous bits it was planned for
+  SweepDesc* d_sweep = nullptr;
+  SweepDesc* h_sweep = nullptr;
+  int sweep_cap = 0;
   float last_ms = 0.f;
   // per-launch profiling: one event before every launch and one after the last
   bool profile = false;
@@ -576,6 +588,18 @@ static int grid_for_pass(const qg_plan* p, const Geo& g, bool two, bool post, in
   return (int)grid;
 }
 
+// Multi-layer passes: several times the resident workgroups either way (no
+// per-thread sums outlive a tile).
+static int grid_for_sweep(const qg_plan* p, int K, bool two) {
+  int occ = 0;
+  if (launch_sweep(kdtype(p, two), two, nullptr, K, 0, 1, p->n, nullptr, &occ, 0) != hipSuccess || occ < 1) occ = 1;
+  const uint64_t ntiles = 1ull << (p->n - K);
+  const uint64_t target = (uint64_t)p->ctx->num_cu * occ * kWgOversub;
+  uint64_t grid = 1;
+  while (grid * 2 <= target && grid * 2 <= ntiles) grid *= 2;
+  return (int)grid;
+}
+
 // Geometry of the gate-free pass that forms lambda = D psi and E when the
 // last forward pass cannot carry it (a 1024-thread pass).
 static Geo obs_geo(int n) {
@@ -597,6 +621,7 @@ static int grid_max(const qg_plan* p) {
         gm = std::max(gm, grid_for_pass(p, G, role != ROLE_FWD, false, phase));
         gm = std::max(gm, grid_for_pass(p, G, true, true, phase));
       }
+  if (!p->sweep.empty()) gm = std::max(gm, grid_for_sweep(p, p->sweep_for[3], true));
   return gm;
 }
 
@@ -1021,19 +1046,38 @@ static hipError_t launch_generic_obs(qg_plan* p) {
   return e;
 }
 
+static hipError_t launch_one(qg_plan* p, const Launch& l) {
+  if (l.kind == 1) return launch_generic_obs(p);
+  if (l.kind != 0) return hipSuccess;
+  if (l.sweep)
+    return launch_sweep(kdtype(p, l.two), l.two, p->d_sweep + l.desc, l.K, l.grid, l.batch, p->n, p->ctx->stream,
+                        nullptr, l.tab);
+  return launch_pass(kdtype(p, l.two), l.R, l.two, l.phase, l.post, p->d_desc + l.desc, l.K, l.grid, l.batch, l.threads,
+                     p->n, p->ctx->stream, nullptr, l.tab);
+}
+
 static hipError_t launch_all(qg_plan* p) {
-  qg_ctx* c = p->ctx;
   for (const Launch& l : p->launches) {
-    if (l.kind == 1) {
-      const hipError_t e = launch_generic_obs(p);
-      if (e != hipSuccess) return e;
-    }
-    if (l.kind != 0) continue;
-    const hipError_t e = launch_pass(kdtype(p, l.two), l.R, l.two, l.phase, l.post, p->d_desc + l.desc, l.K, l.grid,
-                                     l.batch, l.threads, p->n, c->stream, nullptr, l.tab);
+    const hipError_t e = launch_one(p, l);
     if (e != hipSuccess) return e;
   }
   return hipSuccess;
+}
+
+// Sends the sweep descriptors of launches [g0, g1) to the device.
+static int send_sweeps(qg_plan* p, size_t g0, size_t g1) {
+  int s0 = 0x7fffffff, s1 = 0;
+  for (size_t k = g0; k < g1; ++k) {
+    const Launch& l = p->launches[k];
+    if (l.kind != 0 || !l.sweep) continue;
+    if (l.grid > p->gmax) return fail(QG_ERR_HIP, "internal: pass grid exceeds the partial-row stride");
+    s0 = std::min(s0, l.desc);
+    s1 = std::max(s1, l.desc + l.batch);
+  }
+  if (s1 > s0)
+    HIPCHK(hipMemcpyAsync(p->d_sweep + s0, p->h_sweep + s0, sizeof(SweepDesc) * (s1 - s0), hipMemcpyHostToDevice,
+                          p->ctx->stream));
+  return QG_OK;
 }
 
 // Prepares and uploads descriptors [first_desc, ndesc) and launches the
@@ -1043,7 +1087,7 @@ static int run_launches(qg_plan* p, int ndesc, int first_desc = 0) {
   p->h_cterms.clear();
   std::vector<std::pair<int, size_t>> cterm_at;  // (descriptor, offset of its split terms)
   for (Launch& l : p->launches)
-    if (l.kind == 0) {
+    if (l.kind == 0 && !l.sweep) {
       // partial rows are strided by gmax: a larger grid would overlap them
       if (l.grid > p->gmax) return fail(QG_ERR_HIP, "internal: pass grid exceeds the partial-row stride");
       const PassDesc& d = p->h_desc[l.desc];
@@ -1078,23 +1122,26 @@ static int run_launches(qg_plan* p, int ndesc, int first_desc = 0) {
                           hipMemcpyHostToDevice, c->stream));
   }
   for (const auto& e : cterm_at) p->h_desc[e.first].cterms = p->d_cterms + e.second;
-  HIPCHK(hipMemcpyAsync(p->d_desc + first_desc, p->h_desc + first_desc, sizeof(PassDesc) * (ndesc - first_desc),
-                        hipMemcpyHostToDevice, c->stream));
+  if (ndesc > first_desc)
+    HIPCHK(hipMemcpyAsync(p->d_desc + first_desc, p->h_desc + first_desc, sizeof(PassDesc) * (ndesc - first_desc),
+                          hipMemcpyHostToDevice, c->stream));
+  CHK(send_sweeps(p, 0, p->launches.size()));
   HIPCHK(hipEventRecord(c->ev0, c->stream));
   if (p->use_graph && !p->profile) {
     std::vector<int64_t> sig;
-    sig.reserve(p->launches.size() * 11 + 2);
+    sig.reserve(p->launches.size() * 12 + 8);
     sig.push_back(kdtype(p, false) * 4 + kdtype(p, true));
     sig.push_back(p->n);
     sig.push_back((int64_t)(intptr_t)p->d_desc);
+    sig.push_back((int64_t)(intptr_t)p->d_sweep);
     // the elementwise observable launch bakes its buffers and term counts in
     sig.push_back((int64_t)(intptr_t)p->gen_in);
     sig.push_back((int64_t)(intptr_t)p->gen_out);
     sig.push_back(p->gen_ndiag);
     sig.push_back(p->gen_nxy);
     for (const Launch& l : p->launches) {
-      const int64_t v[11] = {l.kind, l.R, l.two, l.phase, l.post, l.desc, l.K, l.grid, l.batch, l.threads, l.tab};
-      sig.insert(sig.end(), v, v + 11);
+      const int64_t v[12] = {l.kind, l.R, l.two, l.phase, l.post, l.desc, l.K, l.grid, l.batch, l.threads, l.tab, l.sweep};
+      sig.insert(sig.end(), v, v + 12);
     }
     if (!p->gexec || sig != p->gsig) {
       drop_graph(p);
@@ -1137,12 +1184,7 @@ static int run_launches(qg_plan* p, int ndesc, int first_desc = 0) {
   for (size_t k = 0; k < nl; ++k) {
     const Launch& l = p->launches[k];
     if (pev) HIPCHK(hipEventRecord((*pev)[k], c->stream));
-    if (l.kind == 0) {
-      HIPCHK(launch_pass(kdtype(p, l.two), l.R, l.two, l.phase, l.post, p->d_desc + l.desc, l.K, l.grid, l.batch,
-                         l.threads, p->n, c->stream, nullptr, l.tab));
-    } else if (l.kind == 1) {
-      HIPCHK(launch_generic_obs(p));
-    }
+    HIPCHK(launch_one(p, l));
   }
   if (pev) HIPCHK(hipEventRecord((*pev)[nl], c->stream));
   return QG_OK;
@@ -1188,7 +1230,7 @@ static int stream_flush(qg_plan* p) {
   int d0 = 0x7fffffff, d1 = 0;
   for (size_t k = g0; k < g1; ++k) {
     Launch& l = p->launches[k];
-    if (l.kind != 0) continue;
+    if (l.kind != 0 || l.sweep) continue;
     if (l.grid > p->gmax) return fail(QG_ERR_HIP, "internal: pass grid exceeds the partial-row stride");
     const PassDesc& d = p->h_desc[l.desc];
     // the preparation of run_launches
@@ -1221,15 +1263,8 @@ static int stream_flush(qg_plan* p) {
   if (d1 > d0)
     HIPCHK(hipMemcpyAsync(p->d_desc + d0, p->h_desc + d0, sizeof(PassDesc) * (d1 - d0), hipMemcpyHostToDevice,
                           c->stream));
-  for (size_t k = g0; k < g1; ++k) {
-    const Launch& l = p->launches[k];
-    if (l.kind == 0) {
-      HIPCHK(launch_pass(kdtype(p, l.two), l.R, l.two, l.phase, l.post, p->d_desc + l.desc, l.K, l.grid, l.batch,
-                         l.threads, p->n, c->stream, nullptr, l.tab));
-    } else if (l.kind == 1) {
-      HIPCHK(launch_generic_obs(p));
-    }
-  }
+  CHK(send_sweeps(p, g0, g1));
+  for (size_t k = g0; k < g1; ++k) HIPCHK(launch_one(p, p->launches[k]));
   p->stream_next = g1;
   return QG_OK;
 }
@@ -1247,6 +1282,10 @@ static int collect_profile(qg_plan* p) {
   for (size_t k = 0; k < nl; ++k) {
     if (p->launches[k].kind != 0) {
       kinds[k] = 3;  // not a pass kernel
+      continue;
+    }
+    if (p->launches[k].sweep) {
+      kinds[k] = p->launches[k].two ? 1 : 0;
       continue;
     }
     const PassDesc& d = p->h_desc[p->launches[k].desc];
@@ -1314,6 +1353,11 @@ static void free_small(qg_plan* p) {
   (void)hipFree(p->d_out);
   (void)hipFree(p->d_dot);
   (void)hipFree(p->d_desc);
+  (void)hipFree(p->d_sweep);
+  if (p->h_sweep) (void)hipHostFree(p->h_sweep);
+  p->d_sweep = nullptr;
+  p->h_sweep = nullptr;
+  p->sweep_cap = 0;
   if (p->h_desc) (void)hipHostFree(p->h_desc);
   if (p->h_out) (void)hipHostFree(p->h_out);
   if (p->h_arena) (void)hipHostFree(p->h_arena);
@@ -1430,14 +1474,83 @@ static int mcclean_geometry(qg_plan* p) {
   return QG_OK;
 }
 
+// Plans the multi-layer passes of a McClean plan, or none where they do not
+// apply: circuits that run whole in one workgroup, tiles of less than whole
+// waves or of 1024 threads.
+//
+// The tile (K local bits, c of them the low bits that make the runs of
+// contiguous amplitudes) and the steps (layers) that a pass may run on it,
+// unless the tile was chosen by the caller.  Device us of a gradient run, 20
+// layers, complex64 | complex128:
+//  - below 20 qubits a pass takes as long as its chain of rounds, and tiles
+//    of 2^12 are fewer than the CUs: K = 11, c = 2, 4 steps (16 qubits 502 |
+//    479, 19 qubits 684 | 694) against K = 12, c = 3 (523 | 539, 756 | 799);
+//    at 18 qubits the larger tile is ahead (582 against 672), its plan has 11
+//    passes instead of 15;
+//  - from there on the larger tile needs fewer passes.  While psi and lambda
+//    stay in the last-level cache, short runs cost nothing and a wide window
+//    is worth more: c = 2, 6 steps (22 qubits 1705 | 2092) against c = 3, 4
+//    steps (1761 | 2132);
+//  - beyond, the state streams from memory in whole 64-byte lines: c = 3, 4
+//    steps (25 qubits 12.6 ms against 13.5 ms).
+constexpr size_t kCachedState = (size_t)64 << 20;  // bytes; two of them fit the 256 MiB cache
+
+static void plan_sweeps(qg_plan* p) {
+  int K = p->kmax, c = p->cmin, steps = 4;
+  if (p->kmax_auto) {
+    K = p->n < 20 ? 11 : 12;
+    if (p->S <= kCachedState) c = 2;
+    if (p->n >= 20 && c == 2) steps = 6;
+  }
+  const int key[5] = {p->n, p->L, p->ent, K, c};
+  if (p->n <= kFusedMaxN || K < kSweepMinK || K > kSweepMaxK || c < 1 || K - c < 4) {
+    p->sweep.clear();
+    p->sweep_rounds = 0;
+    return;
+  }
+  if (!p->sweep.empty() && std::equal(key, key + 5, p->sweep_for)) return;
+  p->sweep = SweepPlanner(p->n, p->L, p->ent == QG_ENT_CZ, K, c).plan(steps);
+  p->sweep_rounds = 0;
+  for (const PlanPass& s : p->sweep) p->sweep_rounds += (int)s.rounds.size();
+  std::copy(key, key + 5, p->sweep_for);
+  // the layout holds one state per single-layer pass
+  if (p->sweep.size() > p->geo.size() * (size_t)p->L) p->sweep.clear();
+}
+
+// Room for the sweep descriptors of `circuits` circuits at a time.
+static int ensure_sweeps(qg_plan* p, int circuits) {
+  const int need = 2 * (int)p->sweep.size() * circuits;
+  if (need <= p->sweep_cap) return QG_OK;
+  HIPCHK(hipStreamSynchronize(p->ctx->stream));
+  drop_graph(p);
+  (void)hipFree(p->d_sweep);
+  if (p->h_sweep) (void)hipHostFree(p->h_sweep);
+  p->d_sweep = nullptr;
+  p->h_sweep = nullptr;
+  p->sweep_cap = 0;
+  HIPCHK(hipMalloc(&p->d_sweep, sizeof(SweepDesc) * need));
+  HIPCHK(hipHostMalloc(&p->h_sweep, sizeof(SweepDesc) * need, hipHostMallocDefault));
+  p->sweep_cap = need;
+  return QG_OK;
+}
+
+// Partial rows of one circuit: of the single-layer passes (shifted circuits
+// and plans without multi-layer passes), or of the multi-layer ones and the
+// observable's pass.
+static int mcclean_rows(const qg_plan* p) {
+  return std::max(((int)p->geo.size() * p->L + 1) * (kMaxK + 1), 4 * p->sweep_rounds + kMaxK + 1);
+}
+
 // mcclean_geometry plus the partial-row stride and the small device tables.
 static int mcclean_layout(qg_plan* p) {
   CHK(mcclean_geometry(p));
+  plan_sweeps(p);
   const int n = p->n, L = p->L, P = (int)p->geo.size();
   p->gmax = grid_max(p);
   const int npass = 2 * P * L + 2 * P + 1;  // forward + reverse + ini-state preparation + observable
-  p->nrows = (P * L + 1) * (kMaxK + 1);
+  p->nrows = mcclean_rows(p);
   CHK(ensure_small(p, npass, p->nrows, 1 + L * n));
+  CHK(ensure_sweeps(p, 1));
   // static tables, staged in pinned memory and copied in stream order (the
   // previous run on this stream ended with a synchronisation, so the staging
   // is free and the tables are no longer read)
@@ -1695,6 +1808,267 @@ static int mcclean_schedule(qg_plan* p, const int32_t* axes, const double* angle
   return flush_rc;
 }
 
+// Appends one launch of a forward pass of geometry G0 over `batch` circuits to
+// the plan's launch list and returns its first descriptor (shared: the only
+// one), with the fields that do not depend on the circuit.
+static PassDesc& push_forward(qg_plan* p, const Geo& G0, int batch, bool shared, int& nd) {
+  bool tf = false;
+  const Geo G = with_role(G0, p->dtype, ROLE_FWD, &tf);
+  Launch l;
+  l.desc = nd;
+  l.batch = batch;
+  l.shared = shared;
+  l.R = G.R;
+  l.K = G.K;
+  l.post = tf;
+  l.threads = G.threads;
+  l.grid = grid_for_pass(p, G, false, tf, 0);
+  l.phase = 0;
+  l.two = false;
+  l.kind = 0;
+  p->launches.push_back(l);
+  PassDesc& d = p->h_desc[nd];
+  nd += l.ndesc();
+  desc_geo(d, p->n, G);
+  d.grid = p->gmax;
+  d.lad1 = p->lad1;
+  d.lad2 = p->lad2;
+  d.init_tab = p->d_init;
+  d.dterms = p->d_terms;
+  d.ndterms = 0;
+  d.part = p->d_part;
+  return d;
+}
+
+// The shift-form masks of the bonds in b1 and b2 (the group acting first in
+// b1), for bits numbered from `shift` above their global position: the index
+// map through which a state is read to apply them (inverse: to undo them).
+// Reading new(y) = old(map(y)) applies the first group last to the index.
+static void bond_masks(uint32_t b1, uint32_t b2, bool inverse, int shift, uint32_t* m1, uint32_t* m2) {
+  auto put = [&](uint32_t b) { return shift >= 0 ? b << shift : b >> -shift; };
+  *m1 = put((b1 | b2) << 1);  // bond k: bit k + 1 flips bit k
+  // bit k + 1 reaches bit k - 1 where its own bond acts on the index first
+  const uint32_t first = inverse ? b1 : b2, second = inverse ? b2 : b1;
+  *m2 = put((first << 1) & (second << 2));
+}
+
+// Builds the launches of one McClean run (nb circuits: circuit j's parameters
+// at axes + j * L * n and angles + j * L * n) from the plan's multi-layer
+// passes.  out_rows and cnt: the finalize tables (1 + L * n outputs per
+// circuit, E first).  streamed as in mcclean_schedule.
+static int sweep_schedule(qg_plan* p, int nb, const int32_t* axes, const double* angles, const ObsSplit& obs,
+                          bool with_ini, bool grad, bool streamed, std::vector<std::vector<int>>& out_rows,
+                          std::vector<int>& cnt, int& ndesc_out) {
+  const int n = p->n, L = p->L, NP = (int)p->sweep.size();
+  const size_t np = (size_t)L * n, per_out = 1 + np, stride = p->geo.size() * (size_t)L;
+  const bool diag_obs = obs.xy.empty();
+  const bool cz = p->ent == QG_ENT_CZ;
+  const bool nt = p->history && ((uint64_t)nb << n) <= kNtMaxLaunchAmps;
+  int flush_rc = QG_OK;
+  p->launches.clear();
+  int nd = 0, ns = 0, row = 0;
+  auto hist = [&](int j, int k) { return wsp(p, p->off_hist + ((size_t)j * stride + k) * p->S); };
+  auto lam = [&](int j) { return wsp(p, p->off_lam + (size_t)j * 2 * p->S); };
+  // checkpoints: the outputs of nckpt passes, evenly spaced, the last among them
+  std::vector<int> slot(NP, -1);
+  if (!p->history) {
+    const int m = std::min(p->nckpt, NP);
+    for (int i = 0; i < m; ++i) slot[(size_t)(i + 1) * NP / m - 1] = i;
+  }
+  auto ckpt = [&](int k) { return wsp(p, p->off_ckpt + (size_t)slot[k] * p->S); };
+  void* work = wsp(p, p->off_work);
+  // doubling groups, as in mcclean_schedule
+  auto due = [&]() {
+    if (streamed && flush_rc == QG_OK && p->launches.size() - p->stream_next >= std::max<size_t>(2, p->stream_next))
+      flush_rc = stream_flush(p);
+  };
+  if (with_ini) {
+    // RY(pi/4) on every qubit of the given vector: one layer, single-layer passes
+    const void* src = wsp(p, p->off_ini);
+    for (const Geo& G : p->geo) {
+      PassDesc& d = push_forward(p, G, 1, false, nd);
+      d.flags = F_LOAD_A | F_ROT_A | F_STORE_A;
+      d.a_in = src;
+      d.a_out = wsp(p, p->off_prep);
+      for (int lb = G.own_lo; lb < G.own_hi; ++lb) set_gate(d, lb, QG_AXIS_Y, M_PI / 4, 1.0);
+      src = wsp(p, p->off_prep);
+    }
+  }
+  // one launch of pass k; fill(j, d) sets circuit j's states
+  auto launch = [&](int k, bool two, auto fill) {
+    due();
+    const PlanPass& s = p->sweep[k];
+    const int K = p->sweep_for[3];
+    const Geo G = s.lo == 0 ? make_geo(K, K, n, 0, K) : make_geo(K, s.c, s.lo, s.c, K);
+    const int NR = (int)s.rounds.size();
+    Launch l;
+    l.sweep = true;
+    l.desc = ns;
+    l.batch = nb;
+    l.K = K;
+    l.R = 4;
+    l.threads = G.threads;
+    l.grid = grid_for_sweep(p, K, two);
+    l.phase = 0;
+    l.two = two;
+    l.kind = 0;
+    for (int j = 0; j < nb; ++j) {
+      SweepDesc& d = p->h_sweep[ns++];
+      std::memset(&d, 0, offsetof(SweepDesc, r));
+      d.n = n;
+      d.K = K;
+      d.t = G.t;
+      d.c = G.c;
+      d.p = G.p;
+      d.hi = s.hi < n ? s.hi : 32;
+      d.grid = p->gmax;
+      d.nr = NR;
+      d.init_tab = p->d_init;
+      d.part = p->d_part;
+      d.row_base = row;
+      const int to_local = s.lo == 0 ? 0 : s.c - s.lo;
+      int lo = G.t;
+      bool exchanged = false;
+      // the exchange into a round, as slot offsets: of the registers it is
+      // written from, of those it is read into, of the tile bit above
+      auto exchange = [&](SweepRound& o) {
+        const int sh = kdtype(p, two) == 1 ? 3 : 4;
+        auto slot = [&](uint32_t x) { return (x ^ ((x >> 4) & (sh == 3 ? 31u : 15u))) << sh; };
+        auto map = [&](uint32_t x) { return x ^ ((x & o.m1) >> 1) ^ ((x & o.m2) >> 2); };
+        for (int kk = 0; kk < 4; ++kk) {
+          o.we[kk] = slot(1u << (lo + kk));
+          o.re[kk] = slot(map(1u << (o.lo + kk)));
+        }
+        o.off = slot(map(1u << K) & ~(1u << K));
+        exchanged |= o.lo != lo || (o.m1 | o.m2);
+        lo = o.lo;
+      };
+      for (int r = 0; r < NR; ++r) {
+        const int q = two ? NR - 1 - r : r;  // the adjoint runs the rounds backwards
+        const PlanRound& pr = s.rounds[q];
+        SweepRound& o = d.r[r];
+        o.lo = pr.lo;
+        o.m1 = o.m2 = o.cz = 0;
+        if (cz) {
+          o.cz = pr.b1 | pr.b2;
+        } else if (two) {
+          // on the way from round q + 1 back to round q: undo the bonds before round q + 1
+          if (q + 1 < NR) bond_masks(s.rounds[q + 1].b1, s.rounds[q + 1].b2, true, to_local, &o.m1, &o.m2);
+        } else if (q > 0) {
+          bond_masks(pr.b1, pr.b2, false, to_local, &o.m1, &o.m2);
+        }
+        exchange(o);
+        for (int kk = 0; kk < 4; ++kk) {
+          o.type[kk] = G_NONE;
+          o.a[kk] = o.b[kk] = 0.0;
+          if (pr.bit[kk] < 0) continue;
+          const size_t at = (size_t)pr.layer[kk] * n + (n - 1 - pr.bit[kk]);
+          const int axis = axes[(size_t)j * np + at];
+          const GateAB g = gate_ab(angles[(size_t)j * np + at], two ? -1.0 : 1.0);
+          o.type[kk] = axis == 0 ? G_X : axis == 1 ? G_Y : G_Z;
+          o.a[kk] = g.a;
+          o.b[kk] = g.b;
+          if (two) out_rows[(size_t)j * per_out + 1 + at].push_back(row + 4 * r + kk);
+        }
+      }
+      // back to the natural layout
+      d.r[NR].lo = G.t;
+      d.r[NR].m1 = d.r[NR].m2 = d.r[NR].cz = 0;
+      exchange(d.r[NR]);
+      uint32_t f = two ? F_LOAD_A | F_LOAD_B : 0u;
+      if (!cz && (s.rounds[0].b1 | s.rounds[0].b2)) {
+        // the bonds before the first round: on the load, or undone on the store
+        f |= two ? F_SCATTER : F_GATHER;
+        if (!exchanged) f |= F_SWEEP_SYNC;
+        bond_masks(s.rounds[0].b1, s.rounds[0].b2, false, 0, &d.g1, &d.g2);
+      }
+      // tile order as desc_order gives it
+      if (d.c + (p->dtype == QG_C64 ? 3 : 4) < 7) f |= F_XCD_ORDER;
+      d.flags = f;
+      fill(j, d);
+      if (two) {
+        for (int i = 0; i < 4 * NR; ++i) cnt[row + i] = l.grid;
+        row += 4 * NR;
+      }
+    }
+    l.tab = (p->h_sweep[l.desc].flags & F_INIT_TAB) ? (int)sizeof(double) * (n + 1) : 0;
+    p->launches.push_back(l);
+  };
+  // forward sweep
+  std::vector<const void*> cur(nb, with_ini ? wsp(p, p->off_prep) : nullptr);
+  for (int k = 0; k < NP; ++k)
+    launch(k, false, [&](int j, SweepDesc& d) {
+      d.a_in = cur[j];
+      d.a_out = p->history ? hist(j, k) : slot[k] >= 0 ? ckpt(k) : work;
+      d.flags |= F_STORE_A | (cur[j] ? F_LOAD_A | (nt ? F_NT_A : 0u) : (uint32_t)F_INIT_TAB);
+      cur[j] = d.a_out;
+    });
+  // lambda = O psi and E: a pass of its own, or the elementwise kernels (x / y terms)
+  due();
+  if (diag_obs) {
+    const Geo og = obs_geo(n);
+    Launch l;
+    l.desc = nd;
+    l.batch = nb;
+    l.R = og.R;
+    l.K = og.K;
+    l.threads = og.threads;
+    l.grid = grid_for_pass(p, og, true, false, 0);
+    l.phase = 0;
+    l.two = true;
+    l.kind = 0;
+    for (int j = 0; j < nb; ++j) {
+      PassDesc& d = p->h_desc[nd++];
+      desc_geo(d, n, og);
+      d.grid = p->gmax;
+      d.dterms = p->d_terms;
+      d.ndterms = (int)obs.diag.size();
+      d.part = p->d_part;
+      d.flags = F_LOAD_A | F_OBS_DIAG | (grad ? (uint32_t)F_STORE_B : 0u);
+      d.a_in = cur[j];
+      d.b_out = lam(j);
+      d.row_base = row;
+      out_rows[(size_t)j * per_out].push_back(row + og.K);
+      for (int i = 0; i <= kMaxK; ++i) cnt[row + i] = l.grid;
+      row += kMaxK + 1;
+    }
+    p->launches.push_back(l);
+  } else {
+    Launch l;
+    l.desc = -1;
+    l.R = l.K = l.threads = l.grid = l.phase = l.tab = 0;
+    l.two = false;
+    l.kind = 1;
+    p->launches.push_back(l);
+    p->gen_in = cur[0];
+    p->gen_out = lam(0);
+    p->gen_ndiag = (int)obs.diag.size();
+    p->gen_nxy = (int)obs.xy.size();
+  }
+  p->last_state_ptr = (void*)cur[0];
+  // adjoint sweep; lambda is updated in place, psi read from the history or
+  // taken back in place from the nearest checkpoint
+  if (grad) {
+    std::vector<const void*> psi(cur);
+    for (int k = NP - 1; k >= 0; --k)
+      launch(k, true, [&](int j, SweepDesc& d) {
+        d.b_in = lam(j);
+        d.b_out = lam(j);
+        if (k > 0) d.flags |= F_STORE_B;
+        if (p->history) {
+          d.a_in = hist(j, k);
+          if (nt) d.flags |= F_NT_A;
+        } else {
+          d.a_in = slot[k] >= 0 ? ckpt(k) : work;
+          d.a_out = work;
+          if (k > 0 && slot[k - 1] < 0) d.flags |= F_STORE_A;
+        }
+      });
+  }
+  ndesc_out = nd;
+  return flush_rc;
+}
+
 static int upload_finalize(qg_plan* p, const std::vector<std::vector<int>>& out_rows, const std::vector<int>& cnt,
                            const std::vector<double>& scale) {
   const int nout = (int)out_rows.size();
@@ -1825,8 +2199,10 @@ static int obs_tables(const ObsSplit& obs, FusedDescH& d, Arena& ar) {
   return QG_OK;
 }
 
+// layered: one layer at a time, keeping the layer-end states that shifted
+// circuits start from (mcclean_shift_run).
 static int mcclean_run(qg_plan* p, const int32_t* axes, const double* angles, const qg_term* terms, int nterms,
-                       const double* ini_state, double* E_out, double* grad_out, bool grad) {
+                       const double* ini_state, double* E_out, double* grad_out, bool grad, bool layered = false) {
   if (!p || p->kind != PK_MCCLEAN) return fail(QG_ERR_INVALID, "not a McClean plan");
   if (p->mc_batch) return fail(QG_ERR_INVALID, "a batch plan runs through qg_mcclean_batch_grad_run");
   if (!axes || !angles || !E_out || (grad && !grad_out)) return fail(QG_ERR_INVALID, "NULL argument");
@@ -1896,20 +2272,28 @@ static int mcclean_run(qg_plan* p, const int32_t* axes, const double* angles, co
   // at the end); only the observable's pass splits terms
   const bool streamed = !p->use_graph && !p->profile;
   if (streamed) CHK(stream_begin(p, std::max<size_t>(1, obs.diag.size())));
-  CHK(mcclean_schedule(p, axes, angles, obs, ini_state != nullptr, grad, nd, streamed));
+  std::vector<std::vector<int>> out_rows(grad ? 1 + L * n : 1);
+  std::vector<int> cnt(p->nrows, 0);
+  const bool sweeps = !layered && !p->sweep.empty();
+  if (sweeps) {
+    p->state_sign = false;
+    for (int k = 0; k < L * n; ++k) p->state_sign ^= gate_flips(angles[k], 1.0);
+    p->obs_desc = obs.xy.empty() ? 0 : -1;
+    CHK(sweep_schedule(p, 1, axes, angles, obs, ini_state != nullptr, grad, streamed, out_rows, cnt, nd));
+  } else {
+    CHK(mcclean_schedule(p, axes, angles, obs, ini_state != nullptr, grad, nd, streamed));
+  }
   // uncompute passes of a checkpointed adjoint overwrite the final state
   if (grad && !p->history) p->last_state_ptr = nullptr;
   // rows written by each pass and the finalize table
   const int P = (int)p->geo.size();
-  std::vector<std::vector<int>> out_rows(grad ? 1 + L * n : 1);
-  std::vector<int> cnt(p->nrows, 0);
   for (const Launch& l : p->launches) {
-    if (l.kind != 0) continue;  // no descriptor
+    if (l.kind != 0 || sweeps) continue;  // no descriptor, or counted already
     const PassDesc& d = p->h_desc[l.desc];
     if (d.row_base < 0) continue;
     for (int k = 0; k <= kMaxK; ++k) cnt[d.row_base + k] = l.grid;
   }
-  {
+  if (!sweeps) {
     // E: row K of the observable pass (none with x / y terms: from d_dot)
     if (p->obs_desc >= 0) {
       const PassDesc& d = p->h_desc[p->obs_desc];
@@ -1984,10 +2368,12 @@ static int mcclean_batch_layout(qg_plan* p) {
   p->off_hist = 0;
   p->off_lam = (size_t)p->chunk * P * L * p->S;
   p->ws_bytes = n > kFusedMaxN ? (size_t)p->chunk * per : 0;
+  plan_sweeps(p);
   p->gmax = grid_max(p);
   const int ch = n > kFusedMaxN ? p->chunk : 1;
-  p->nrows = ch * (P * L + 1) * (kMaxK + 1);
+  p->nrows = ch * mcclean_rows(p);
   CHK(ensure_small(p, ch * 2 * P * L, p->nrows, ch * (1 + L * n)));
+  CHK(ensure_sweeps(p, ch));
   if (!ladder_shift_form(n, 1, &p->lad1, &p->lad2) || !ladder_shift_form(n, 0, &p->inv1, &p->inv2))
     return fail(QG_ERR_INVALID, "ladder map not in shift form");
   double* hi = (double*)p->h_tabs;
@@ -2080,100 +2466,106 @@ extern "C" int qg_mcclean_batch_grad_run(qg_plan* p, int B, const int32_t* axes,
     int nd = 0, row = 0;
     std::vector<std::vector<int>> out_rows((size_t)nb * per_out);
     std::vector<int> cnt(p->nrows, 0);
-    // one launch per pass over the chunk's circuits, at a single plan's grid
-    auto begin = [&](const Geo& G0, bool two, int role, int* grid) -> Geo {
-      bool tf = false;
-      const Geo G = with_role(G0, p->dtype, role, &tf);
-      Launch l;
-      l.desc = nd;
-      l.batch = nb;
-      l.R = G.R;
-      l.K = G.K;
-      l.post = tf;
-      l.threads = G.threads;
-      l.grid = grid_for_pass(p, G, two, tf, 0);
-      l.phase = 0;
-      l.two = two;
-      l.kind = 0;
-      p->launches.push_back(l);
-      *grid = l.grid;
-      return G;
-    };
-    auto base = [&](const Geo& G) -> PassDesc& {
-      PassDesc& d = p->h_desc[nd++];
-      desc_geo(d, n, G);
-      d.grid = p->gmax;
-      d.lad1 = p->lad1;
-      d.lad2 = p->lad2;
-      d.init_tab = p->d_init;
-      d.dterms = p->d_terms;
-      d.ndterms = (int)obs.diag.size();
-      d.part = p->d_part;
-      return d;
-    };
-    auto gates = [&](PassDesc& d, const Geo& G, int j, int i, double sign, int rb) {
-      const int32_t* ax = axes + (size_t)(c0 + j) * np;
-      const double* an = angles + (size_t)(c0 + j) * np;
-      for (int lb = G.own_lo; lb < G.own_hi; ++lb) {
-        const int b = (lb < G.c) ? lb : G.p + (lb - G.c);
-        const int q = n - 1 - b;
-        set_gate(d, lb, ax[i * n + q], an[i * n + q], sign);
-        if (rb >= 0) {
-          d.own[lb] = 1;
-          out_rows[(size_t)j * per_out + 1 + i * n + q].push_back(rb + lb);
+    const bool sweeps = !p->sweep.empty();
+    if (sweeps) {
+      CHK(sweep_schedule(p, nb, axes + (size_t)c0 * np, angles + (size_t)c0 * np, obs, false, true, false, out_rows,
+                         cnt, nd));
+    } else {
+      // one layer at a time: one launch per pass over the chunk's circuits, at a single plan's grid
+      auto begin = [&](const Geo& G0, bool two, int role, int* grid) -> Geo {
+        bool tf = false;
+        const Geo G = with_role(G0, p->dtype, role, &tf);
+        Launch l;
+        l.desc = nd;
+        l.batch = nb;
+        l.R = G.R;
+        l.K = G.K;
+        l.post = tf;
+        l.threads = G.threads;
+        l.grid = grid_for_pass(p, G, two, tf, 0);
+        l.phase = 0;
+        l.two = two;
+        l.kind = 0;
+        p->launches.push_back(l);
+        *grid = l.grid;
+        return G;
+      };
+      auto base = [&](const Geo& G) -> PassDesc& {
+        PassDesc& d = p->h_desc[nd++];
+        desc_geo(d, n, G);
+        d.grid = p->gmax;
+        d.lad1 = p->lad1;
+        d.lad2 = p->lad2;
+        d.init_tab = p->d_init;
+        d.dterms = p->d_terms;
+        d.ndterms = (int)obs.diag.size();
+        d.part = p->d_part;
+        return d;
+      };
+      auto gates = [&](PassDesc& d, const Geo& G, int j, int i, double sign, int rb) {
+        const int32_t* ax = axes + (size_t)(c0 + j) * np;
+        const double* an = angles + (size_t)(c0 + j) * np;
+        for (int lb = G.own_lo; lb < G.own_hi; ++lb) {
+          const int b = (lb < G.c) ? lb : G.p + (lb - G.c);
+          const int q = n - 1 - b;
+          set_gate(d, lb, ax[i * n + q], an[i * n + q], sign);
+          if (rb >= 0) {
+            d.own[lb] = 1;
+            out_rows[(size_t)j * per_out + 1 + i * n + q].push_back(rb + lb);
+          }
+        }
+      };
+      // forward sweep; lambda = D psi and E ride on the last pass
+      for (int i = 0; i < L; ++i) {
+        for (int g = 0; g < P; ++g) {
+          const bool last = (i == L - 1) && (g == P - 1);
+          int gr = 0;
+          const Geo G = begin(p->geo[g], last, last ? ROLE_TWO_FP64 : ROLE_FWD, &gr);
+          for (int j = 0; j < nb; ++j) {
+            PassDesc& d = base(G);
+            uint32_t f = F_ROT_A | F_STORE_A;
+            if (g == 0) f |= ent_fwd | (i == 0 ? F_INIT_TAB : F_LOAD_A);
+            else f |= F_LOAD_A;
+            // history passes: the input is read once here
+            if ((f & F_LOAD_A) && ((uint64_t)nb << n) <= kNtMaxLaunchAmps) f |= F_NT_A;
+            d.a_in = (i == 0 && g == 0) ? nullptr : (g == 0 ? hist(j, i - 1, P - 1) : hist(j, i, g - 1));
+            d.a_out = hist(j, i, g);
+            gates(d, p->geo[g], j, i, 1.0, -1);
+            if (last) {
+              f |= F_OBS_DIAG | F_STORE_B;
+              d.b_out = lam(j, 0);
+              d.row_base = row;
+              out_rows[(size_t)j * per_out].push_back(row + G.K);
+              for (int k = 0; k <= kMaxK; ++k) cnt[row + k] = gr;
+              row += kMaxK + 1;
+            }
+            d.flags = f;
+          }
         }
       }
-    };
-    // forward sweep; lambda = D psi and E ride on the last pass
-    for (int i = 0; i < L; ++i) {
-      for (int g = 0; g < P; ++g) {
-        const bool last = (i == L - 1) && (g == P - 1);
-        int gr = 0;
-        const Geo G = begin(p->geo[g], last, last ? ROLE_TWO_FP64 : ROLE_FWD, &gr);
-        for (int j = 0; j < nb; ++j) {
-          PassDesc& d = base(G);
-          uint32_t f = F_ROT_A | F_STORE_A;
-          if (g == 0) f |= ent_fwd | (i == 0 ? F_INIT_TAB : F_LOAD_A);
-          else f |= F_LOAD_A;
-          // history passes: the input is read once here
-          if ((f & F_LOAD_A) && ((uint64_t)nb << n) <= kNtMaxLaunchAmps) f |= F_NT_A;
-          d.a_in = (i == 0 && g == 0) ? nullptr : (g == 0 ? hist(j, i - 1, P - 1) : hist(j, i, g - 1));
-          d.a_out = hist(j, i, g);
-          gates(d, p->geo[g], j, i, 1.0, -1);
-          if (last) {
-            f |= F_OBS_DIAG | F_STORE_B;
-            d.b_out = lam(j, 0);
+      // adjoint sweep (reduce-first history passes)
+      int lc = 0;
+      for (int i = L - 1; i >= 0; --i) {
+        for (int g = P - 1; g >= 0; --g) {
+          int gr = 0;
+          const Geo G = begin(p->geo[g], true, ROLE_REV_HIST, &gr);
+          const bool swap = g == 0 && p->ent == QG_ENT_CNOT;
+          for (int j = 0; j < nb; ++j) {
+            PassDesc& d = base(G);
+            uint32_t f = F_LOAD_A | F_ROT_A | F_LOAD_B | F_ROT_B | F_STORE_B | F_REDUCE;
+            if (g == 0) f |= ent_rev;
+            if (((uint64_t)nb << n) <= kNtMaxLaunchAmps) f |= F_NT_A;  // the history state is read once here
+            d.a_in = hist(j, i, g);
+            d.b_in = lam(j, lc);
+            d.b_out = lam(j, swap ? lc ^ 1 : lc);
+            d.flags = f;
             d.row_base = row;
-            out_rows[(size_t)j * per_out].push_back(row + G.K);
+            gates(d, p->geo[g], j, i, -1.0, row);
             for (int k = 0; k <= kMaxK; ++k) cnt[row + k] = gr;
             row += kMaxK + 1;
           }
-          d.flags = f;
+          if (swap) lc ^= 1;
         }
-      }
-    }
-    // adjoint sweep (reduce-first history passes)
-    int lc = 0;
-    for (int i = L - 1; i >= 0; --i) {
-      for (int g = P - 1; g >= 0; --g) {
-        int gr = 0;
-        const Geo G = begin(p->geo[g], true, ROLE_REV_HIST, &gr);
-        const bool swap = g == 0 && p->ent == QG_ENT_CNOT;
-        for (int j = 0; j < nb; ++j) {
-          PassDesc& d = base(G);
-          uint32_t f = F_LOAD_A | F_ROT_A | F_LOAD_B | F_ROT_B | F_STORE_B | F_REDUCE;
-          if (g == 0) f |= ent_rev;
-          if (((uint64_t)nb << n) <= kNtMaxLaunchAmps) f |= F_NT_A;  // the history state is read once here
-          d.a_in = hist(j, i, g);
-          d.b_in = lam(j, lc);
-          d.b_out = lam(j, swap ? lc ^ 1 : lc);
-          d.flags = f;
-          d.row_base = row;
-          gates(d, p->geo[g], j, i, -1.0, row);
-          for (int k = 0; k <= kMaxK; ++k) cnt[row + k] = gr;
-          row += kMaxK + 1;
-        }
-        if (swap) lc ^= 1;
       }
     }
     std::vector<double> scale(out_rows.size(), 1.0);
@@ -2336,38 +2728,6 @@ static int ensure_shift(qg_plan* p, size_t bytes) {
 constexpr int kShiftAmpsLog2 = 22;
 static int shift_batch(int n) { return n >= kShiftAmpsLog2 ? 1 : std::min(4096, 1 << (kShiftAmpsLog2 - n)); }
 
-// Appends one launch of a forward pass of geometry G0 over `batch` circuits to
-// the plan's launch list and returns its first descriptor (shared: the only
-// one), with the fields that do not depend on the circuit.
-static PassDesc& push_forward(qg_plan* p, const Geo& G0, int batch, bool shared, int& nd) {
-  bool tf = false;
-  const Geo G = with_role(G0, p->dtype, ROLE_FWD, &tf);
-  Launch l;
-  l.desc = nd;
-  l.batch = batch;
-  l.shared = shared;
-  l.R = G.R;
-  l.K = G.K;
-  l.post = tf;
-  l.threads = G.threads;
-  l.grid = grid_for_pass(p, G, false, tf, 0);
-  l.phase = 0;
-  l.two = false;
-  l.kind = 0;
-  p->launches.push_back(l);
-  PassDesc& d = p->h_desc[nd];
-  nd += l.ndesc();
-  desc_geo(d, p->n, G);
-  d.grid = p->gmax;
-  d.lad1 = p->lad1;
-  d.lad2 = p->lad2;
-  d.init_tab = p->d_init;
-  d.dterms = p->d_terms;
-  d.ndterms = 0;
-  d.part = p->d_part;
-  return d;
-}
-
 // The gates of layer i on the bits a forward pass owns.
 static void layer_gates(PassDesc& d, const Geo& G0, int n, int i, const int32_t* axes, const double* angles) {
   for (int lb = G0.own_lo; lb < G0.own_hi; ++lb) {
@@ -2422,7 +2782,7 @@ static int mcclean_shift_run(qg_plan* p, const int32_t* axes, const double* angl
   p->fused = false;
   double E = 0.0;
   const qg_term none{QG_TERM_Z, 0, -1, 0, 0.0};  // the forward run's own observable: unused
-  const int r = mcclean_run(p, axes, angles, &none, 1, ini_state, &E, nullptr, false);
+  const int r = mcclean_run(p, axes, angles, &none, 1, ini_state, &E, nullptr, false, true);
   p->fused = fused;
   CHK(r);
   qg_ctx* c = p->ctx;

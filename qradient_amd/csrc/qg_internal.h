@@ -47,6 +47,7 @@ enum : uint32_t {
   F_DRED_PRE    = 1u << 17,  // (adjoint, with F_PHASE_PRE) extra += 2*sum D(x) Im(conj(B)A) before the pre phase
   F_XCD_ORDER   = 1u << 18,  // XCD-aware tile order (else round-robin); set by the planner
   F_NT_A        = 1u << 19,  // A is read with non-temporal loads (read once in this sweep; set by the planner)
+  F_SWEEP_SYNC  = 1u << 20,  // multi-layer pass: a barrier between the loads and the stores of a tile
 };
 
 // One term of the diagonal quadratic form D(x) = sum w * z_a(x) [* z_b(x)],
@@ -130,6 +131,45 @@ struct PassDesc {
   double phase_gamma;    // angle multiplying D(x) in the phase
   const double* lut;     // (re, im) pairs: exp(-i*gamma*d) at d = idx - lut_off
   double* part;          // partial sums: part[row * grid + block]
+};
+
+// ---------------------------------------------------------------------------
+// Multi-layer passes of the McClean circuit (qg_sweep.hpp)
+// ---------------------------------------------------------------------------
+constexpr int kMaxRounds = 14;   // rounds of a multi-layer pass
+constexpr int kSweepMinK = 10;   // local bits of one: whole waves of 16 amplitudes per lane
+constexpr int kSweepMaxK = 13;
+
+// One round: four local bits in registers, a rotation on each.
+struct SweepRound {
+  double a[4], b[4];   // shear coefficients (see PassDesc::ga), by register bit
+  int32_t type[4];     // GateType; G_NONE: no gate on that bit
+  // the exchange into the round: LDS byte offsets of the four register bits
+  // it is written from and read into, and of the tile bit above the window
+  uint32_t we[4], re[4], off;
+  int32_t lo;          // the register bits are local bits [lo, lo + 4)
+  uint32_t m1, m2;     // nonzero: the index map applied on the way into this round,
+                       // new(y) = old(y ^ ((y & m1) >> 1) ^ ((y & m2) >> 2)) in local bits;
+                       // bit K stands for the tile bit just above the window
+  uint32_t cz;         // CZ bonds (bond k: global bits k, k + 1) whose sign the round
+                       // applies: before its gates forward, after them in the adjoint
+};
+
+struct SweepDesc {
+  // geometry as in PassDesc; hi: the global bit just above the window (32: none)
+  int32_t n, K, t, c, p, hi;
+  uint32_t flags;      // PassFlag bits
+  int32_t grid;        // stride of the partial rows
+  int32_t row_base;    // adjoint: row_base + 4 r + k holds round r's reduction of register bit k
+  int32_t nr;          // rounds
+  uint32_t g1, g2;     // index map of the load (F_GATHER) or the store (F_SCATTER), global bits
+  const void* a_in;
+  void* a_out;
+  const void* b_in;
+  void* b_out;
+  const double* init_tab;  // n + 1 entries when F_INIT_TAB
+  double* part;
+  SweepRound r[kMaxRounds + 1];  // and the exchange back to the natural layout
 };
 
 }  // namespace qg
