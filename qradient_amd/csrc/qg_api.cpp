@@ -18,6 +18,9 @@
 namespace qg {
 hipError_t set_pass_attributes();
 hipError_t set_sweep_attributes();
+hipError_t set_turn_attributes();
+hipError_t launch_turn(int dtype, bool two, int ph, const TurnDesc* d, int K, int grid, int batch, int n,
+                       hipStream_t st, int* occ, int tab);
 hipError_t launch_sweep(int dtype, bool two, const SweepDesc* d, int K, int grid, int batch, int n, hipStream_t st,
                         int* occ, int tab);
 hipError_t launch_pass(int dtype, int R, bool two, int phase, bool post, const PassDesc* d, int K, int grid,
@@ -155,7 +158,8 @@ extern "C" int qg_ctx_create(int device, void* stream, qg_ctx** out) {
     c->own_stream = true;
   }
   if (hipEventCreate(&c->ev0) != hipSuccess || hipEventCreate(&c->ev1) != hipSuccess ||
-      set_pass_attributes() != hipSuccess || set_sweep_attributes() != hipSuccess || set_fused_attributes() != hipSuccess ||
+      set_pass_attributes() != hipSuccess || set_sweep_attributes() != hipSuccess ||
+      set_turn_attributes() != hipSuccess || set_fused_attributes() != hipSuccess ||
       fused_desc_size() != sizeof(FusedDescH) ||
       hipHostMalloc((void**)&c->noalloc_host, kNoAllocScratchBytes, hipHostMallocDefault) != hipSuccess) {
     if (c->noalloc_host) (void)hipHostFree(c->noalloc_host);
@@ -392,6 +396,7 @@ struct Launch {
   int batch = 1;
   bool shared = false;  // one descriptor for the whole batch (PassDesc::bstride)
   bool sweep = false;   // a multi-layer pass: desc indexes the plan's sweep descriptors
+  bool turn = false;    // a QAOA turning pass: desc indexes the plan's turn descriptors
   int K = 0;
   bool post = false;  // the pass has diagonal ops after its gates (set at launch from the flags)
   int tab = 0;        // bytes of the table the pass stages in LDS (set at launch)
@@ -486,6 +491,11 @@ struct qg_plan {
   SweepDesc* d_sweep = nullptr;
   SweepDesc* h_sweep = nullptr;
   int sweep_cap = 0;
+  // turning passes of a QAOA plan (qg_turn.hpp)
+  bool turn = false;
+  TurnDesc* d_turn = nullptr;
+  TurnDesc* h_turn = nullptr;
+  int turn_cap = 0;
   float last_ms = 0.f;
   // per-launch profiling: one event before every launch and one after the last
   bool profile = false;
@@ -600,6 +610,19 @@ static int grid_for_sweep(const qg_plan* p, int K, bool two) {
   return (int)grid;
 }
 
+// QAOA turning passes of tiles of 2^K amplitudes, for one circuit.
+static int grid_for_turn(const qg_plan* p, int K, bool two, int ph) {
+  int occ = 0;
+  if (launch_turn(p->dtype == QG_C64 ? 1 : 0, two, ph, nullptr, K, 0, 1, p->n, nullptr, &occ, 0) != hipSuccess ||
+      occ < 1)
+    occ = 1;
+  const uint64_t ntiles = 1ull << (p->n - K);
+  const uint64_t target = (uint64_t)p->ctx->num_cu * occ * kWgOversub;
+  uint64_t grid = 1;
+  while (grid * 2 <= target && grid * 2 <= ntiles) grid *= 2;
+  return (int)grid;
+}
+
 // Geometry of the gate-free pass that forms lambda = D psi and E when the
 // last forward pass cannot carry it (a 1024-thread pass).
 static Geo obs_geo(int n) {
@@ -622,6 +645,8 @@ static int grid_max(const qg_plan* p) {
         gm = std::max(gm, grid_for_pass(p, G, true, true, phase));
       }
   if (!p->sweep.empty()) gm = std::max(gm, grid_for_sweep(p, p->sweep_for[3], true));
+  if (p->turn)
+    for (int v = 0; v < 6; ++v) gm = std::max(gm, grid_for_turn(p, p->geo[0].K, v & 1, v / 2));
   return gm;
 }
 
@@ -1052,8 +1077,11 @@ static hipError_t launch_one(qg_plan* p, const Launch& l) {
   if (l.sweep)
     return launch_sweep(kdtype(p, l.two), l.two, p->d_sweep + l.desc, l.K, l.grid, l.batch, p->n, p->ctx->stream,
                         nullptr, l.tab);
-  return launch_pass(kdtype(p, l.two), l.R, l.two, l.phase, l.post, p->d_desc + l.desc, l.K, l.grid, l.batch, l.threads,
-                     p->n, p->ctx->stream, nullptr, l.tab);
+  if (l.turn)
+    return launch_turn(p->dtype == QG_C64 ? 1 : 0, l.two, l.phase, p->d_turn + l.desc, l.K, l.grid, l.batch, p->n,
+                       p->ctx->stream, nullptr, l.tab);
+  return launch_pass(kdtype(p, l.two), l.R, l.two, l.phase, l.post, p->d_desc + l.desc, l.K, l.grid, l.batch,
+                     l.threads, p->n, p->ctx->stream, nullptr, l.tab);
 }
 
 static hipError_t launch_all(qg_plan* p) {
@@ -1064,19 +1092,22 @@ static hipError_t launch_all(qg_plan* p) {
   return hipSuccess;
 }
 
-// Sends the sweep descriptors of launches [g0, g1) to the device.
+// Sends the sweep and turn descriptors of launches [g0, g1) to the device.
 static int send_sweeps(qg_plan* p, size_t g0, size_t g1) {
-  int s0 = 0x7fffffff, s1 = 0;
+  int s0[2] = {0x7fffffff, 0x7fffffff}, s1[2] = {0, 0};
   for (size_t k = g0; k < g1; ++k) {
     const Launch& l = p->launches[k];
-    if (l.kind != 0 || !l.sweep) continue;
+    if (l.kind != 0 || !(l.sweep || l.turn)) continue;
     if (l.grid > p->gmax) return fail(QG_ERR_HIP, "internal: pass grid exceeds the partial-row stride");
-    s0 = std::min(s0, l.desc);
-    s1 = std::max(s1, l.desc + l.batch);
+    s0[l.turn] = std::min(s0[l.turn], l.desc);
+    s1[l.turn] = std::max(s1[l.turn], l.desc + l.batch);
   }
-  if (s1 > s0)
-    HIPCHK(hipMemcpyAsync(p->d_sweep + s0, p->h_sweep + s0, sizeof(SweepDesc) * (s1 - s0), hipMemcpyHostToDevice,
-                          p->ctx->stream));
+  if (s1[0] > s0[0])
+    HIPCHK(hipMemcpyAsync(p->d_sweep + s0[0], p->h_sweep + s0[0], sizeof(SweepDesc) * (s1[0] - s0[0]),
+                          hipMemcpyHostToDevice, p->ctx->stream));
+  if (s1[1] > s0[1])
+    HIPCHK(hipMemcpyAsync(p->d_turn + s0[1], p->h_turn + s0[1], sizeof(TurnDesc) * (s1[1] - s0[1]),
+                          hipMemcpyHostToDevice, p->ctx->stream));
   return QG_OK;
 }
 
@@ -1087,7 +1118,7 @@ static int run_launches(qg_plan* p, int ndesc, int first_desc = 0) {
   p->h_cterms.clear();
   std::vector<std::pair<int, size_t>> cterm_at;  // (descriptor, offset of its split terms)
   for (Launch& l : p->launches)
-    if (l.kind == 0 && !l.sweep) {
+    if (l.kind == 0 && !l.sweep && !l.turn) {
       // partial rows are strided by gmax: a larger grid would overlap them
       if (l.grid > p->gmax) return fail(QG_ERR_HIP, "internal: pass grid exceeds the partial-row stride");
       const PassDesc& d = p->h_desc[l.desc];
@@ -1134,13 +1165,15 @@ static int run_launches(qg_plan* p, int ndesc, int first_desc = 0) {
     sig.push_back(p->n);
     sig.push_back((int64_t)(intptr_t)p->d_desc);
     sig.push_back((int64_t)(intptr_t)p->d_sweep);
+    sig.push_back((int64_t)(intptr_t)p->d_turn);
     // the elementwise observable launch bakes its buffers and term counts in
     sig.push_back((int64_t)(intptr_t)p->gen_in);
     sig.push_back((int64_t)(intptr_t)p->gen_out);
     sig.push_back(p->gen_ndiag);
     sig.push_back(p->gen_nxy);
     for (const Launch& l : p->launches) {
-      const int64_t v[12] = {l.kind, l.R, l.two, l.phase, l.post, l.desc, l.K, l.grid, l.batch, l.threads, l.tab, l.sweep};
+      const int64_t v[12] = {l.kind,  l.R,     l.two,     l.phase, l.post, l.desc, l.K,
+                             l.grid, l.batch, l.threads, l.tab,   l.sweep + 2 * l.turn};
       sig.insert(sig.end(), v, v + 12);
     }
     if (!p->gexec || sig != p->gsig) {
@@ -1230,7 +1263,7 @@ static int stream_flush(qg_plan* p) {
   int d0 = 0x7fffffff, d1 = 0;
   for (size_t k = g0; k < g1; ++k) {
     Launch& l = p->launches[k];
-    if (l.kind != 0 || l.sweep) continue;
+    if (l.kind != 0 || l.sweep || l.turn) continue;
     if (l.grid > p->gmax) return fail(QG_ERR_HIP, "internal: pass grid exceeds the partial-row stride");
     const PassDesc& d = p->h_desc[l.desc];
     // the preparation of run_launches
@@ -1284,7 +1317,7 @@ static int collect_profile(qg_plan* p) {
       kinds[k] = 3;  // not a pass kernel
       continue;
     }
-    if (p->launches[k].sweep) {
+    if (p->launches[k].sweep || p->launches[k].turn) {
       kinds[k] = p->launches[k].two ? 1 : 0;
       continue;
     }
@@ -1358,6 +1391,11 @@ static void free_small(qg_plan* p) {
   p->d_sweep = nullptr;
   p->h_sweep = nullptr;
   p->sweep_cap = 0;
+  (void)hipFree(p->d_turn);
+  if (p->h_turn) (void)hipHostFree(p->h_turn);
+  p->d_turn = nullptr;
+  p->h_turn = nullptr;
+  p->turn_cap = 0;
   if (p->h_desc) (void)hipHostFree(p->h_desc);
   if (p->h_out) (void)hipHostFree(p->h_out);
   if (p->h_arena) (void)hipHostFree(p->h_arena);
@@ -2987,15 +3025,52 @@ extern "C" int qg_mcclean_shift_sample(qg_plan* p, const int32_t* axes, const do
 // ---------------------------------------------------------------------------
 // QAOA (qradient/circuit_logic/qaoa.py:40-70), batched over circuits
 // ---------------------------------------------------------------------------
+// Passes of a QAOA circuit's forward half (and of its adjoint), each of whose
+// outputs the history keeps.
+static int qaoa_passes(const qg_plan* p) {
+  const int P = (int)p->geo.size();
+  return p->turn ? (P - 1) * p->L + 1 : P * p->L;
+}
+
+// Room for `need` turn descriptors.
+static int ensure_turn(qg_plan* p, int need) {
+  if (need <= p->turn_cap) return QG_OK;
+  HIPCHK(hipStreamSynchronize(p->ctx->stream));
+  drop_graph(p);
+  (void)hipFree(p->d_turn);
+  if (p->h_turn) (void)hipHostFree(p->h_turn);
+  p->d_turn = nullptr;
+  p->h_turn = nullptr;
+  p->turn_cap = 0;
+  HIPCHK(hipMalloc(&p->d_turn, sizeof(TurnDesc) * need));
+  HIPCHK(hipHostMalloc(&p->h_turn, sizeof(TurnDesc) * need, hipHostMallocDefault));
+  p->turn_cap = need;
+  return QG_OK;
+}
+
 // Geometry, chunk and tables of a QAOA plan (tile shape from kmax / cmin,
 // chunk from chunk_req and device memory).
 static int qaoa_layout(qg_plan* p) {
   const int n = p->n, L = p->L;
-  if (p->kmax_auto) p->kmax = default_kmax(n, p->dtype, p->cmin);
+  if (p->kmax_auto) {
+    p->kmax = default_kmax(n, p->dtype, p->cmin);
+    // turning passes of states below 2^20 last as long as one tile's chain of
+    // rounds: the smallest tile that needs no more passes is the fastest.
+    // Device us of a gradient run, 6 layers, complex128, K = 10 or 11 against
+    // 12: 15 qubits 188 | 208, 17 qubits 208 | 237, 19 qubits 254 | 272
+    // (24 qubits complex64, 11 against 12: 2589 | 2382).
+    if (n > kFusedMaxN && n < 20)
+      for (int K = kSweepMinK; K < p->kmax; ++K)
+        if (passes_per_layer(n, K, p->cmin) == passes_per_layer(n, 13, p->cmin)) p->kmax = K;
+  }
   p->geo = layer_geometry(n, p->kmax, p->cmin);
   const int P = (int)p->geo.size();
   p->S = (size_t)(1ull << n) * (p->dtype == QG_C64 ? 8 : 16);
-  const size_t per_circuit = (size_t)(P * L + 2) * p->S;
+  // turning passes need whole waves of 16 amplitudes per lane, and a layer of
+  // one pass has nothing to turn
+  p->turn = P >= 2 && p->kmax >= kSweepMinK && p->kmax <= kSweepMaxK;
+  const int NP = qaoa_passes(p);
+  const size_t per_circuit = (size_t)(NP + 2) * p->S;
   size_t budget = 0;
   CHK(plan_budget(p, &budget));
   if (per_circuit > budget)
@@ -3003,11 +3078,12 @@ static int qaoa_layout(qg_plan* p) {
   const int fit = (int)std::min<size_t>((size_t)p->batch, budget / per_circuit);
   p->chunk = p->chunk_req > 0 ? std::min(p->chunk_req, fit) : fit;
   p->off_hist = 0;
-  p->off_lam = (size_t)p->chunk * P * L * p->S;
+  p->off_lam = (size_t)p->chunk * NP * p->S;
   p->ws_bytes = p->off_lam + (size_t)p->chunk * 2 * p->S;
   p->gmax = grid_max(p);
-  const int ndesc = p->chunk * 2 * P * L;
-  p->nrows = p->chunk * (P * L + 1) * (kMaxK + 1);
+  const int ndesc = p->turn ? 1 : p->chunk * 2 * NP;
+  p->nrows = p->turn ? p->chunk * (3 * NP + 1) : p->chunk * (NP + 1) * (kMaxK + 1);
+  if (p->turn) CHK(ensure_turn(p, p->chunk * 2 * NP));
   CHK(ensure_small(p, ndesc, p->nrows, p->chunk * (1 + 2 * L)));
   // each circuit of a chunk has its own classical Hamiltonian
   const int mt = n + n * (n - 1) / 2;
@@ -3082,6 +3158,239 @@ extern "C" int qg_qaoa_tune(qg_plan* p, int kmax, int cmin, int chunk, int wg_pe
   return QG_OK;
 }
 
+// One run of a QAOA plan's turning passes over nb circuits.
+struct TurnRun {
+  qg_plan* p;
+  int nb;
+  bool grad;
+  int ph;                // TurnPhase
+  int lut_w;             // phase table: entries -lut_w .. lut_w
+  const int* tcnt;       // terms of each circuit, from toff on in p->h_terms
+  const int* toff;
+  const GateAB* gab;     // [circuit][layer][forward, inverse]
+  const double* gammas;  // [circuit][layer]
+  const char* ini = nullptr;  // initial states in the storage type (null: |+>^n)
+};
+
+// The diagonal form of one circuit split by register bits (see split_terms).
+struct TurnSplit {
+  size_t off;
+  int nct, nht[4];
+  double pwc[16];
+};
+
+static void turn_split(const DTerm* terms, int nt, const int (&rpos)[4], std::vector<DTerm>& out, TurnSplit& s) {
+  auto regk = [&](int b) {
+    for (int k = 0; k < 4; ++k)
+      if (rpos[k] == b) return k;
+    return -1;
+  };
+  auto sgn = [](int a, int k) { return ((a >> k) & 1) ? -1.0 : 1.0; };
+  s.off = out.size();
+  s.nct = 0;
+  for (int k = 0; k < 4; ++k) s.nht[k] = 0;
+  for (int a = 0; a < 16; ++a) s.pwc[a] = 0.0;
+  for (int i = 0; i < nt; ++i) {
+    const DTerm& t = terms[i];
+    const int ka = regk(t.a), kb = t.b >= 0 ? regk(t.b) : -1;
+    if (ka < 0 && kb < 0) {
+      out.push_back({(int32_t)((1u << t.a) | (t.b >= 0 ? 1u << t.b : 0u)), 0, t.w});
+      s.nct++;
+    } else if (t.b < 0 || (ka >= 0 && kb >= 0)) {
+      for (int a = 0; a < 16; ++a) s.pwc[a] += t.w * sgn(a, ka) * (t.b < 0 ? 1.0 : sgn(a, kb));
+    }
+  }
+  for (int k = 0; k < 4; ++k)
+    for (int i = 0; i < nt; ++i) {
+      const DTerm& t = terms[i];
+      if (t.b < 0) continue;
+      const int ka = regk(t.a), kb = regk(t.b);
+      if ((ka < 0) == (kb < 0) || (ka >= 0 ? ka : kb) != k) continue;
+      out.push_back({(int32_t)(1u << (ka >= 0 ? t.b : t.a)), 0, t.w});
+      s.nht[k]++;
+    }
+}
+
+// Builds (and, unless the plan replays graphs or profiles, launches) the
+// turning passes of a run; out_rows and cnt as in qaoa_run.
+template <class Hist, class Lam, class LutPtr, class LutFill>
+static int turn_schedule(const TurnRun& tr, Hist hist, Lam lam, LutPtr lut_ptr, LutFill lut_fill,
+                         std::vector<std::vector<int>>& out_rows, std::vector<int>& cnt) {
+  qg_plan* p = tr.p;
+  const int n = p->n, L = p->L, P = (int)p->geo.size(), NP = qaoa_passes(p), nb = tr.nb;
+  const int per_out = 1 + 2 * L, sh = p->dtype == QG_C64 ? 3 : 4;
+  const bool streamed = !p->use_graph && !p->profile;
+  // the register windows of each pass window: [lo, lo + 4) and the owned bits
+  // that gate there
+  struct Win {
+    int lo;
+    uint32_t mask;
+  };
+  std::vector<std::vector<Win>> wins(P);
+  for (int g = 0; g < P; ++g) {
+    const Geo& G = p->geo[g];
+    uint32_t left = ((1u << G.own_hi) - 1u) & ~((1u << G.own_lo) - 1u);
+    for (int lo = G.K - 4; left; lo = std::max(0, lo - 4)) {
+      const uint32_t m = (left >> lo) & 15u;
+      if (m) wins[g].push_back({lo, m});
+      left &= ~(m << lo);
+    }
+  }
+  // passes: a window, the layers it runs (two: it turns), the phase it applies
+  struct Pass {
+    int g, layer[2], nl, phase;
+  };
+  std::vector<Pass> passes;
+  for (int i = 0; i < L; ++i)
+    for (int k = 0; k < P; ++k) {
+      const int g = i % 2 ? P - 1 - k : k;
+      if (i > 0 && k == 0) {
+        passes.back().layer[passes.back().nl++] = i;
+        passes.back().phase = i;
+      } else {
+        passes.push_back({g, {i, -1}, 1, i == 0 && k == 0 ? 0 : -1});
+      }
+    }
+  // the layouts in which a diagonal operation meets a circuit: window and register window
+  std::vector<std::pair<int, int>> at;
+  auto layout = [&](int g, int lo) -> int {
+    for (size_t i = 0; i < at.size(); ++i)
+      if (at[i] == std::make_pair(g, lo)) return (int)i;
+    at.push_back({g, lo});
+    return (int)at.size() - 1;
+  };
+  auto diag_layout = [&](int k, bool two) -> int {
+    const Pass& ps = passes[k];
+    const bool end = ps.nl == 2 || (two && k == 0);  // met in the last register window
+    return layout(ps.g, end ? wins[ps.g].back().lo : p->geo[ps.g].K - 4);
+  };
+  for (int k = 0; k < NP; ++k)
+    for (int two = 0; two < 2; ++two)
+      if (passes[k].phase >= 0 || k == NP - 1) diag_layout(k, two);
+  size_t bound = 0;
+  for (int j = 0; j < nb; ++j) bound += (size_t)tr.tcnt[j];
+  CHK(stream_begin(p, std::max<size_t>(1, bound * at.size())));
+  std::vector<TurnSplit> split((size_t)nb * at.size());
+  for (size_t a = 0; a < at.size(); ++a) {
+    const Geo& G = p->geo[at[a].first];
+    int rpos[4];
+    for (int k = 0; k < 4; ++k) {
+      const int l = at[a].second + k;
+      rpos[k] = l < G.c ? l : G.p + (l - G.c);
+    }
+    for (int j = 0; j < nb; ++j)
+      turn_split(p->h_terms.data() + tr.toff[j], tr.tcnt[j], rpos, p->h_cterms, split[a * nb + j]);
+  }
+  if (!p->h_cterms.empty()) {
+    std::memcpy(p->h_cstage, p->h_cterms.data(), sizeof(DTerm) * p->h_cterms.size());
+    HIPCHK(hipMemcpyAsync(p->d_cterms, p->h_cstage, sizeof(DTerm) * p->h_cterms.size(), hipMemcpyHostToDevice,
+                          p->ctx->stream));
+  }
+  int nd = 0, row = 0;
+  auto launch = [&](int k, bool two) -> int {
+    const Pass& ps = passes[k];
+    const Geo& G = p->geo[ps.g];
+    const std::vector<Win>& w = wins[ps.g];
+    const int m = (int)w.size(), nr = ps.nl * m, last = k == NP - 1;
+    const bool diag = ps.phase >= 0 || last;
+    Launch l;
+    l.turn = true;
+    l.desc = nd;
+    l.batch = nb;
+    l.K = G.K;
+    l.R = 4;
+    l.threads = 1 << (G.K - 4);
+    l.grid = grid_for_turn(p, G.K, two, tr.ph);
+    // as in the single-layer passes: a batched launch fills the device across circuits
+    while (l.grid > 1 && (uint64_t)l.grid * nb > (uint64_t)p->wg_per_cu * p->ctx->num_cu) l.grid >>= 1;
+    l.phase = tr.ph;
+    l.two = two;
+    l.kind = 0;
+    // the rounds, and the operation's place among them (shared by the circuits)
+    TurnDesc base;
+    std::memset(&base, 0, sizeof base);
+    base.n = n;
+    base.K = G.K;
+    base.t = G.K - 4;
+    base.c = G.c;
+    base.p = G.p;
+    base.grid = p->gmax;
+    base.nr = nr;
+    base.dq = ps.nl == 2 ? m : !diag ? -1 : two == (k == 0) ? nr : 0;
+    base.lut_off = tr.lut_w;
+    base.amp0 = std::pow(2.0, -0.5 * n);
+    base.part = p->d_part;
+    base.flags = F_XCD_ORDER | (last ? (uint32_t)F_OBS_DIAG : 0u);
+    // a phase that opens or splits the pass; the first layer's is not undone
+    if (ps.phase >= 0 && !(two && k == 0)) base.flags |= F_PHASE_PRE;
+    if (two) base.flags |= F_NT_A | (k > 0 ? (uint32_t)F_STORE_B : 0u);
+    l.tab = tr.ph == TP_LUT && (base.flags & F_PHASE_PRE) ? (int)sizeof(double) * 2 * (2 * tr.lut_w + 1) : 0;
+    auto slot = [&](uint32_t x) { return (x ^ ((x >> 4) & (sh == 3 ? 31u : 15u))) << sh; };
+    int lo = base.t;
+    for (int r = 0; r <= nr; ++r) {
+      TurnRound& o = base.r[r];
+      const bool back = r >= m;
+      o.lo = r == nr ? base.t : w[back ? nr - 1 - r : r].lo;
+      if (r < nr) o.mask = w[back ? nr - 1 - r : r].mask;
+      o.block = ps.nl == 2 && back != two;
+      for (int kk = 0; kk < 4; ++kk) {
+        o.we[kk] = slot(1u << (lo + kk));
+        o.re[kk] = slot(1u << (o.lo + kk));
+      }
+      lo = o.lo;
+    }
+    const int al = diag ? diag_layout(k, two) : -1;
+    for (int j = 0; j < nb; ++j) {
+      TurnDesc& d = p->h_turn[nd++];
+      d = base;
+      if (al >= 0) {
+        const TurnSplit& s = split[(size_t)al * nb + j];
+        d.cterms = p->d_cterms + s.off;
+        d.nct = s.nct;
+        std::copy(s.nht, s.nht + 4, d.nht);
+        std::copy(s.pwc, s.pwc + 16, d.pwc);
+      }
+      if (ps.phase >= 0) {
+        d.phase_gamma = (two ? -1.0 : 1.0) * tr.gammas[(size_t)j * L + ps.phase];
+        d.lut = lut_ptr(j, ps.phase, two ? 1 : 0);
+      }
+      for (int r = 0; r < nr; ++r) {
+        const GateAB g = tr.gab[((size_t)j * L + ps.layer[d.r[r].block]) * 2 + (two ? 1 : 0)];
+        d.r[r].a = g.a;
+        d.r[r].b = g.b;
+      }
+      d.row_base = row;
+      const size_t out = (size_t)j * per_out;
+      if (!two) {
+        d.a_in = k > 0 ? hist(j, k - 1) : tr.ini ? (const void*)(tr.ini + (size_t)j * p->S) : nullptr;
+        if (!d.a_in) d.flags |= F_INIT_TAB;
+        d.a_out = hist(j, k);
+        if (last) {
+          out_rows[out].push_back(row);
+          cnt[row++] = l.grid;
+        }
+      } else {
+        d.a_in = hist(j, k);
+        d.b_in = d.b_out = lam(j);
+        for (int b = 0; b < ps.nl; ++b) out_rows[out + 1 + 2 * ps.layer[b]].push_back(row + b);
+        if (ps.phase >= 0) out_rows[out + 2 + 2 * ps.phase].push_back(row + 2);
+        for (int b = 0; b < 3; ++b) cnt[row++] = l.grid;
+      }
+    }
+    p->launches.push_back(l);
+    // passes go to the device as they are built (graph replay and profiled
+    // runs launch the whole list at the end)
+    if (streamed && p->launches.size() - p->stream_next >= 2) CHK(stream_flush(p));
+    return QG_OK;
+  };
+  for (int k = 0; k < NP; ++k) {
+    if (passes[k].phase >= 0) CHK(lut_fill(passes[k].phase + 1));
+    CHK(launch(k, false));
+  }
+  for (int k = NP - 1; tr.grad && k >= 0; --k) CHK(launch(k, true));
+  return QG_OK;
+}
+
 // ini: B initial states (complex128, 2^n each) or null for |+>^n (qaoa.py:17)
 static int qaoa_run(qg_plan* p, int B, const qg_term* terms, const int32_t* term_off, const double* betas,
                     const double* gammas, const double* ini, double* E_out, double* grad_out, bool grad) {
@@ -3113,6 +3422,10 @@ static int qaoa_run(qg_plan* p, int B, const qg_term* terms, const int32_t* term
   // integer weights: exp(-i gamma C) from a table of 2W + 1 entries staged in LDS
   const int phase = (integral && 2.0 * W + 1.0 <= (double)kLutMax) ? 1 : 2;
   const int Wi = (int)W;
+  // otherwise the largest phase angle decides the sincos (W: the largest sum of |w|)
+  double gmax = 0.0;
+  for (int k = 0; k < B * L; ++k) gmax = std::max(gmax, std::fabs(gammas[k]));
+  const int turn_ph = phase == 1 ? TP_LUT : gmax * W < kSincosMax ? TP_SINCOS : TP_LARGE;
   qg_ctx* c = p->ctx;
   HIPCHK(hipSetDevice(c->device));
   if (p->fused && n <= kFusedMaxN && !ini) {
@@ -3143,10 +3456,7 @@ static int qaoa_run(qg_plan* p, int B, const qg_term* terms, const int32_t* term
       HIPCHK(hipMalloc(&p->d_fstate, ((size_t)16) << n));
       p->cap_fstate = (size_t)16 << n;
     }
-    // the largest phase angle decides the sincos (W: the largest sum of |w|)
-    double gmax = 0.0;
-    for (int k = 0; k < B * L; ++k) gmax = std::max(gmax, std::fabs(gammas[k]));
-    const int mode = phase == 1 ? FM_QAOA_LUT : gmax * W < kSincosMax ? FM_QAOA_SINCOS : FM_QAOA_LARGE;
+    const int mode = turn_ph == TP_LUT ? FM_QAOA_LUT : turn_ph == TP_SINCOS ? FM_QAOA_SINCOS : FM_QAOA_LARGE;
     CHK(run_fused(p, B, mode, phase == 1 ? Wi : 0, bytes, per, grad, B == 1 ? p->d_fstate : nullptr, fill,
                   res.data()));
     for (int b = 0; b < B; ++b) {
@@ -3254,9 +3564,9 @@ static int qaoa_run(qg_plan* p, int B, const qg_term* terms, const int32_t* term
     auto lut_ptr = [&](int j, int i, int dir) -> const double* {
       return phase == 1 ? p->d_lut + (size_t)i * lut_layer + ((size_t)j * 2 + dir) * lut_len * 2 : nullptr;
     };
-    auto hist = [&](int j, int i, int g) {
-      return wsp(p, p->off_hist + (((size_t)j * L + i) * P + g) * p->S);
-    };
+    const int NP = qaoa_passes(p);
+    auto hist_at = [&](int j, int k) { return wsp(p, p->off_hist + ((size_t)j * NP + k) * p->S); };
+    auto hist = [&](int j, int i, int g) { return hist_at(j, i * P + g); };
     auto lam = [&](int j) { return wsp(p, p->off_lam + (size_t)j * 2 * p->S); };
     // every qubit's mixer gate of circuit j, layer i: forward and inverse
     std::vector<GateAB> gab((size_t)nb * L * 2);
@@ -3270,150 +3580,156 @@ static int qaoa_run(qg_plan* p, int B, const qg_term* terms, const int32_t* term
     int nd = 0, row = 0;
     std::vector<std::vector<int>> out_rows((size_t)nb * per_out);
     std::vector<int> cnt(p->nrows, 0);
-    Geo cur_geo;
-    auto begin_pass = [&](const Geo& G0, bool two, int role) {
-      bool tf = false;
-      const Geo G = with_role(G0, p->dtype, role, &tf);
-      cur_geo = G;
-      Launch l;
-      l.desc = nd;
-      l.batch = nb;
-      l.R = G.R;
-      l.K = G.K;
-      l.post = tf;
-      l.threads = G.threads;
-      l.grid = grid_for_pass(p, G, two, tf, phase);
-      // a batched launch fills the device across circuits: fewer workgroups
-      // per circuit, each running more tiles (amortises its prologue); up to
-      // wg_per_cu per CU in all, beyond the resident count, so that the
-      // circuits' tiles spread evenly over the CUs
-      while (l.grid > 1 && (uint64_t)l.grid * nb > (uint64_t)p->wg_per_cu * p->ctx->num_cu) l.grid >>= 1;
-      l.phase = phase;
-      l.two = two;
-      l.kind = 0;
-      p->launches.push_back(l);
-      return l.grid;
-    };
-    auto base_desc = [&](const Geo& G, int j) -> PassDesc& {
-      PassDesc& d = p->h_desc[nd++];
-      desc_geo(d, n, G);
-      d.grid = p->gmax;
-      d.init_tab = p->d_init;
-      d.dterms = p->d_terms + toff[j];
-      d.ndterms = tcnt[j];
-      d.lut_off = Wi;
-      d.part = p->d_part;
-      return d;
-    };
-    const uint32_t phase_flag = phase == 1 ? F_PHASE_LUT : 0u;
-    // With two or more passes per layer the cost phase of layer i + 1 closes
-    // the last pass of layer i (the first layer's opens its first pass), so
-    // the adjoint of that pass takes d/dgamma and undoes the phase in the
-    // natural layout before its reduce-first reductions: psi never has to be
-    // rotated back.  With one pass per layer the phase opens each pass and
-    // the adjoint takes the general form.
-    const bool phase_last = P >= 2;
-    // passes go to the device as they are built (graph replay and profiled
-    // runs launch the whole list at the end); each descriptor splits at most
-    // its circuit's terms
     const bool streamed = !p->use_graph && !p->profile;
-    if (streamed) {
-      size_t per_pass = 0;
-      for (int j = 0; j < nb; ++j) per_pass += (size_t)tcnt[j];
-      CHK(stream_begin(p, per_pass * (size_t)P * L * (grad ? 2 : 1)));
-    }
-    // forward
-    for (int i = 0; i < L; ++i) {
-      // this layer's passes read the phase tables of layers i and i + 1
-      CHK(lut_fill(i + 2));
-      for (int g = 0; g < P; ++g) {
-        const Geo& G = p->geo[g];
-        const bool last = (i == L - 1) && (g == P - 1);
-        const int gr = begin_pass(G, last, last ? ROLE_TWO_FP64 : ROLE_FWD);
-        for (int j = 0; j < nb; ++j) {
-          PassDesc& d = base_desc(cur_geo, j);
-          uint32_t f = F_ROT_A | F_STORE_A | phase_flag;
-          if (g == 0 && (i == 0 || !phase_last)) {
-            f |= (i == 0 && !ini ? F_INIT_TAB : F_LOAD_A) | F_PHASE_PRE;
-            d.phase_gamma = gammas[(c0 + j) * L + i];
-            d.lut = lut_ptr(j, i, 0);
-          } else {
-            f |= F_LOAD_A;
-          }
-          if (phase_last && g == P - 1 && i + 1 < L) {
-            f |= F_PHASE_POST;
-            d.phase_gamma = gammas[(c0 + j) * L + i + 1];
-            d.lut = lut_ptr(j, i + 1, 0);
-          }
-          d.a_in = (i == 0 && g == 0) ? (ini ? (const void*)((char*)p->d_ini_states + (size_t)j * p->S) : nullptr)
-                                      : (g == 0 ? hist(j, i - 1, P - 1) : hist(j, i, g - 1));
-          d.a_out = hist(j, i, g);
-          const GateAB ab = gab[((size_t)j * L + i) * 2];
-          for (int lb = G.own_lo; lb < G.own_hi; ++lb) {
-            d.gtype[lb] = G_X;
-            d.ga[lb] = ab.a;
-            d.gb[lb] = ab.b;
-          }
-          if (last) {
-            f |= F_OBS_DIAG | F_STORE_B;
-            d.b_out = lam(j);
-            d.row_base = row;
-            out_rows[(size_t)j * per_out].push_back(row + G.K);
-            for (int k = 0; k <= kMaxK; ++k) cnt[row + k] = gr;
-            row += kMaxK + 1;
-          }
-          d.flags = f;
-        }
-        if (streamed && p->launches.size() - p->stream_next >= 2) CHK(stream_flush(p));
+    if (p->turn) {
+      TurnRun tr{p, nb, grad, turn_ph, Wi, tcnt.data(), toff.data(), gab.data(), gammas + (size_t)c0 * L};
+      tr.ini = ini ? (const char*)p->d_ini_states : nullptr;
+      CHK(turn_schedule(tr, hist_at, lam, lut_ptr, lut_fill, out_rows, cnt));
+    } else {
+      Geo cur_geo;
+      auto begin_pass = [&](const Geo& G0, bool two, int role) {
+        bool tf = false;
+        const Geo G = with_role(G0, p->dtype, role, &tf);
+        cur_geo = G;
+        Launch l;
+        l.desc = nd;
+        l.batch = nb;
+        l.R = G.R;
+        l.K = G.K;
+        l.post = tf;
+        l.threads = G.threads;
+        l.grid = grid_for_pass(p, G, two, tf, phase);
+        // a batched launch fills the device across circuits: fewer workgroups
+        // per circuit, each running more tiles (amortises its prologue); up to
+        // wg_per_cu per CU in all, beyond the resident count, so that the
+        // circuits' tiles spread evenly over the CUs
+        while (l.grid > 1 && (uint64_t)l.grid * nb > (uint64_t)p->wg_per_cu * p->ctx->num_cu) l.grid >>= 1;
+        l.phase = phase;
+        l.two = two;
+        l.kind = 0;
+        p->launches.push_back(l);
+        return l.grid;
+      };
+      auto base_desc = [&](const Geo& G, int j) -> PassDesc& {
+        PassDesc& d = p->h_desc[nd++];
+        desc_geo(d, n, G);
+        d.grid = p->gmax;
+        d.init_tab = p->d_init;
+        d.dterms = p->d_terms + toff[j];
+        d.ndterms = tcnt[j];
+        d.lut_off = Wi;
+        d.part = p->d_part;
+        return d;
+      };
+      const uint32_t phase_flag = phase == 1 ? F_PHASE_LUT : 0u;
+      // With two or more passes per layer the cost phase of layer i + 1 closes
+      // the last pass of layer i (the first layer's opens its first pass), so
+      // the adjoint of that pass takes d/dgamma and undoes the phase in the
+      // natural layout before its reduce-first reductions: psi never has to be
+      // rotated back.  With one pass per layer the phase opens each pass and
+      // the adjoint takes the general form.
+      const bool phase_last = P >= 2;
+      // passes go to the device as they are built (graph replay and profiled
+      // runs launch the whole list at the end); each descriptor splits at most
+      // its circuit's terms
+      if (streamed) {
+        size_t per_pass = 0;
+        for (int j = 0; j < nb; ++j) per_pass += (size_t)tcnt[j];
+        CHK(stream_begin(p, per_pass * (size_t)P * L * (grad ? 2 : 1)));
       }
-    }
-    if (grad) {
-      for (int i = L - 1; i >= 0; --i) {
-        for (int g = P - 1; g >= 0; --g) {
+      // forward
+      for (int i = 0; i < L; ++i) {
+        // this layer's passes read the phase tables of layers i and i + 1
+        CHK(lut_fill(i + 2));
+        for (int g = 0; g < P; ++g) {
           const Geo& G = p->geo[g];
-          const int gr = begin_pass(G, true, ROLE_REV_HIST);
+          const bool last = (i == L - 1) && (g == P - 1);
+          const int gr = begin_pass(G, last, last ? ROLE_TWO_FP64 : ROLE_FWD);
           for (int j = 0; j < nb; ++j) {
             PassDesc& d = base_desc(cur_geo, j);
-            // the history state is read once here (5345-5352 circuits/s
-            // for the 512-circuit batch with ordinary loads, 5352-5378 with these)
-            uint32_t f = F_LOAD_A | F_ROT_A | F_LOAD_B | F_ROT_B | F_STORE_B | F_REDUCE | F_NT_A | phase_flag;
-            d.a_in = hist(j, i, g);
-            d.b_in = lam(j);
-            d.b_out = lam(j);
-            d.row_base = row;
-            const GateAB ab = gab[((size_t)j * L + i) * 2 + 1];
+            uint32_t f = F_ROT_A | F_STORE_A | phase_flag;
+            if (g == 0 && (i == 0 || !phase_last)) {
+              f |= (i == 0 && !ini ? F_INIT_TAB : F_LOAD_A) | F_PHASE_PRE;
+              d.phase_gamma = gammas[(c0 + j) * L + i];
+              d.lut = lut_ptr(j, i, 0);
+            } else {
+              f |= F_LOAD_A;
+            }
+            if (phase_last && g == P - 1 && i + 1 < L) {
+              f |= F_PHASE_POST;
+              d.phase_gamma = gammas[(c0 + j) * L + i + 1];
+              d.lut = lut_ptr(j, i + 1, 0);
+            }
+            d.a_in = (i == 0 && g == 0) ? (ini ? (const void*)((char*)p->d_ini_states + (size_t)j * p->S) : nullptr)
+                                        : (g == 0 ? hist(j, i - 1, P - 1) : hist(j, i, g - 1));
+            d.a_out = hist(j, i, g);
+            const GateAB ab = gab[((size_t)j * L + i) * 2];
             for (int lb = G.own_lo; lb < G.own_hi; ++lb) {
               d.gtype[lb] = G_X;
               d.ga[lb] = ab.a;
               d.gb[lb] = ab.b;
-              d.own[lb] = 1;
-              out_rows[(size_t)j * per_out + 1 + 2 * i].push_back(row + lb);
             }
-            if (!phase_last && g == 0) {
-              f |= F_DRED_POST | F_PHASE_POST;
-              d.phase_gamma = -gammas[(c0 + j) * L + i];
-              d.lut = lut_ptr(j, i, 1);
-              out_rows[(size_t)j * per_out + 2 + 2 * i].push_back(row + G.K);
-            }
-            if (phase_last && g == P - 1 && i + 1 < L) {
-              // the forward pass ended with the phase of layer i + 1
-              f |= F_PHASE_PRE | F_DRED_PRE;
-              d.phase_gamma = -gammas[(c0 + j) * L + i + 1];
-              d.lut = lut_ptr(j, i + 1, 1);
-              out_rows[(size_t)j * per_out + 2 + 2 * (i + 1)].push_back(row + G.K);
-            }
-            if (phase_last && g == 0 && i == 0) {
-              // the first layer's phase opened this pass: psi is rotated back
-              // to the initial state times that phase (general form), and
-              // lambda is not needed after it
-              f = (f | F_DRED_POST) & ~F_STORE_B;
-              out_rows[(size_t)j * per_out + 2].push_back(row + G.K);
+            if (last) {
+              f |= F_OBS_DIAG | F_STORE_B;
+              d.b_out = lam(j);
+              d.row_base = row;
+              out_rows[(size_t)j * per_out].push_back(row + G.K);
+              for (int k = 0; k <= kMaxK; ++k) cnt[row + k] = gr;
+              row += kMaxK + 1;
             }
             d.flags = f;
-            for (int k = 0; k <= kMaxK; ++k) cnt[row + k] = gr;
-            row += kMaxK + 1;
           }
           if (streamed && p->launches.size() - p->stream_next >= 2) CHK(stream_flush(p));
+        }
+      }
+      if (grad) {
+        for (int i = L - 1; i >= 0; --i) {
+          for (int g = P - 1; g >= 0; --g) {
+            const Geo& G = p->geo[g];
+            const int gr = begin_pass(G, true, ROLE_REV_HIST);
+            for (int j = 0; j < nb; ++j) {
+              PassDesc& d = base_desc(cur_geo, j);
+              // the history state is read once here (5345-5352 circuits/s
+              // for the 512-circuit batch with ordinary loads, 5352-5378 with these)
+              uint32_t f = F_LOAD_A | F_ROT_A | F_LOAD_B | F_ROT_B | F_STORE_B | F_REDUCE | F_NT_A | phase_flag;
+              d.a_in = hist(j, i, g);
+              d.b_in = lam(j);
+              d.b_out = lam(j);
+              d.row_base = row;
+              const GateAB ab = gab[((size_t)j * L + i) * 2 + 1];
+              for (int lb = G.own_lo; lb < G.own_hi; ++lb) {
+                d.gtype[lb] = G_X;
+                d.ga[lb] = ab.a;
+                d.gb[lb] = ab.b;
+                d.own[lb] = 1;
+                out_rows[(size_t)j * per_out + 1 + 2 * i].push_back(row + lb);
+              }
+              if (!phase_last && g == 0) {
+                f |= F_DRED_POST | F_PHASE_POST;
+                d.phase_gamma = -gammas[(c0 + j) * L + i];
+                d.lut = lut_ptr(j, i, 1);
+                out_rows[(size_t)j * per_out + 2 + 2 * i].push_back(row + G.K);
+              }
+              if (phase_last && g == P - 1 && i + 1 < L) {
+                // the forward pass ended with the phase of layer i + 1
+                f |= F_PHASE_PRE | F_DRED_PRE;
+                d.phase_gamma = -gammas[(c0 + j) * L + i + 1];
+                d.lut = lut_ptr(j, i + 1, 1);
+                out_rows[(size_t)j * per_out + 2 + 2 * (i + 1)].push_back(row + G.K);
+              }
+              if (phase_last && g == 0 && i == 0) {
+                // the first layer's phase opened this pass: psi is rotated back
+                // to the initial state times that phase (general form), and
+                // lambda is not needed after it
+                f = (f | F_DRED_POST) & ~F_STORE_B;
+                out_rows[(size_t)j * per_out + 2].push_back(row + G.K);
+              }
+              d.flags = f;
+              for (int k = 0; k <= kMaxK; ++k) cnt[row + k] = gr;
+              row += kMaxK + 1;
+            }
+            if (streamed && p->launches.size() - p->stream_next >= 2) CHK(stream_flush(p));
+          }
         }
       }
     }
@@ -3442,7 +3758,7 @@ static int qaoa_run(qg_plan* p, int B, const qg_term* terms, const int32_t* term
       if (grad)
         for (int k = 0; k < 2 * L; ++k) grad_out[(size_t)(c0 + j) * 2 * L + k] = o[1 + k];
     }
-    p->last_state_ptr = hist(0, L - 1, P - 1);
+    p->last_state_ptr = hist_at(0, NP - 1);
     p->state_sign = false;
     for (int i = 0; i < L; ++i)
       if (n % 2 == 1) p->state_sign ^= gate_flips(betas[(size_t)c0 * L + i], 1.0);

@@ -172,4 +172,47 @@ struct SweepDesc {
   SweepRound r[kMaxRounds + 1];  // and the exchange back to the natural layout
 };
 
+// ---------------------------------------------------------------------------
+// Turning passes of the QAOA circuit (qg_turn.hpp)
+// ---------------------------------------------------------------------------
+// How a kernel evaluates exp(-i gamma D): from a table (integer D), by
+// sincos_reduced, by the library's sincos (angles of 2^26 and more).
+enum TurnPhase { TP_LUT = 0, TP_SINCOS = 1, TP_LARGE = 2 };
+
+constexpr int kMaxTurnRounds = 8;  // two mixer blocks on up to four register windows
+
+// One round: four local bits in registers, the mixer gate of `block` on those in mask.
+struct TurnRound {
+  double a, b;         // shear coefficients (see PassDesc::ga)
+  uint32_t mask;       // register bits that take the gate
+  int32_t block;       // the mixer block (0 or 1) that its reductions belong to
+  int32_t lo;          // the register bits are local bits [lo, lo + 4)
+  uint32_t we[4], re[4];  // the exchange into the round (see SweepRound)
+};
+
+struct TurnDesc {
+  // geometry as in PassDesc
+  int32_t n, K, t, c, p;
+  uint32_t flags;      // PassFlag bits
+  int32_t grid;        // stride of the partial rows
+  int32_t row_base;    // adjoint: row_base + 0, 1: the blocks' mixer sums, + 2: d/dgamma; forward: row_base: E
+  int32_t nr;          // rounds
+  int32_t dq;          // the diagonal operation comes before round dq (nr: after the last)
+  // the diagonal form split by the register bits that the operation meets (as in PassDesc)
+  const DTerm* cterms;
+  int32_t nct;
+  int32_t nht[4];
+  double pwc[16];
+  int32_t lut_off;
+  double phase_gamma;
+  const double* lut;
+  double amp0;         // F_INIT_TAB: every amplitude of the initial state
+  const void* a_in;
+  void* a_out;
+  const void* b_in;
+  void* b_out;
+  double* part;
+  TurnRound r[kMaxTurnRounds + 1];  // and the exchange back to the natural layout
+};
+
 }  // namespace qg

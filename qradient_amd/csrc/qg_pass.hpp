@@ -460,8 +460,8 @@ __device__ __forceinline__ double flipw(double w, uint32_t m) {
   return __longlong_as_double(__double_as_longlong(w) ^ (long long)sb);
 }
 
-template <int R>
-__device__ __forceinline__ void diag_prepare(const PassDesc* __restrict__ d, uint32_t gthr, DiagParts<R>& o) {
+template <int R, class D>
+__device__ __forceinline__ void diag_prepare(const D* __restrict__ d, uint32_t gthr, DiagParts<R>& o) {
   const DTerm* __restrict__ ct = d->cterms;
   const int nc = ldc(&d->nct, 0);
   double c0 = 0.0;
@@ -484,8 +484,8 @@ __device__ __forceinline__ void diag_prepare(const PassDesc* __restrict__ d, uin
   o.c0 = c0;
 }
 
-template <int R>
-__device__ __forceinline__ double diag_value(const PassDesc* __restrict__ d, const DiagParts<R>& o, int a) {
+template <int R, class D>
+__device__ __forceinline__ double diag_value(const D* __restrict__ d, const DiagParts<R>& o, int a) {
   double v = o.c0 + ldc(d->pwc, a);
 #pragma unroll
   for (int k = 0; k < R; ++k) v += ((a >> k) & 1) ? -o.h[k] : o.h[k];
