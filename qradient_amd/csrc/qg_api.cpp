@@ -1555,6 +1555,14 @@ static void plan_sweeps(qg_plan* p) {
   if (p->sweep.size() > p->geo.size() * (size_t)p->L) p->sweep.clear();
 }
 
+// Local bits that number the waves of a workgroup when the registers hold
+// local bits [lo, lo + 4) of K: the thread index's bits from 6 on.
+static uint32_t wave_bits(int K, int lo) {
+  uint32_t m = 0;
+  for (int i = 6; i < K - 4; ++i) m |= 1u << (i < lo ? i : i + 4);
+  return m;
+}
+
 // Room for the sweep descriptors of `circuits` circuits at a time.
 static int ensure_sweeps(qg_plan* p, int circuits) {
   const int need = 2 * (int)p->sweep.size() * circuits;
@@ -1966,7 +1974,7 @@ static int sweep_schedule(qg_plan* p, int nb, const int32_t* axes, const double*
       d.row_base = row;
       const int to_local = s.lo == 0 ? 0 : s.c - s.lo;
       int lo = G.t;
-      bool exchanged = false;
+      bool exchanged = false;  // with a barrier
       // the exchange into a round, as slot offsets: of the registers it is
       // written from, of those it is read into, of the tile bit above
       auto exchange = [&](SweepRound& o) {
@@ -1978,7 +1986,8 @@ static int sweep_schedule(qg_plan* p, int nb, const int32_t* axes, const double*
           o.re[kk] = slot(map(1u << (o.lo + kk)));
         }
         o.off = slot(map(1u << K) & ~(1u << K));
-        exchanged |= o.lo != lo || (o.m1 | o.m2);
+        o.sync = wave_bits(K, lo) != wave_bits(K, o.lo) || (((o.m1 >> 1) | (o.m2 >> 2)) & wave_bits(K, lo)) != 0;
+        exchanged |= o.sync != 0;
         lo = o.lo;
       };
       for (int r = 0; r < NR; ++r) {
@@ -3337,6 +3346,7 @@ static int turn_schedule(const TurnRun& tr, Hist hist, Lam lam, LutPtr lut_ptr, 
         o.we[kk] = slot(1u << (lo + kk));
         o.re[kk] = slot(1u << (o.lo + kk));
       }
+      o.sync = wave_bits(G.K, lo) != wave_bits(G.K, o.lo);
       lo = o.lo;
     }
     const int al = diag ? diag_layout(k, two) : -1;

@@ -147,6 +147,7 @@ struct SweepRound {
   // the exchange into the round: LDS byte offsets of the four register bits
   // it is written from and read into, and of the tile bit above the window
   uint32_t we[4], re[4], off;
+  int32_t sync;        // 0: the exchange stays inside each wave's slots
   int32_t lo;          // the register bits are local bits [lo, lo + 4)
   uint32_t m1, m2;     // nonzero: the index map applied on the way into this round,
                        // new(y) = old(y ^ ((y & m1) >> 1) ^ ((y & m2) >> 2)) in local bits;
@@ -188,6 +189,7 @@ struct TurnRound {
   int32_t block;       // the mixer block (0 or 1) that its reductions belong to
   int32_t lo;          // the register bits are local bits [lo, lo + 4)
   uint32_t we[4], re[4];  // the exchange into the round (see SweepRound)
+  int32_t sync;
 };
 
 struct TurnDesc {

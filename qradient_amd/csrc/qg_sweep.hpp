@@ -214,9 +214,17 @@ __device__ __forceinline__ void run_sweep(const SweepDesc* __restrict__ d, void*
     // The exchange into round rd, from register bits [lo_from, +4), through
     // the round's index map.  Each layout is written to the slots it was read
     // from, so only reads need a barrier before them, and mapped reads one
-    // after them.
+    // after them.  Where both layouts give the same bits to the wave index and
+    // the map leaves those bits alone, a wave only meets its own slots, and
+    // the LDS runs one wave's accesses in order: no barrier at all (adjoint passes of 24 qubits,
+    // complex64: 222 -> 218 us).
     auto exchange = [&](auto with_a, auto with_b, const SweepRound* __restrict__ rd, int lo_from) __attribute__((always_inline)) {
       const uint32_t m1 = ldc(&rd->m1, 0), m2 = ldc(&rd->m2, 0);
+      const bool sync = ldc(&rd->sync, 0) != 0;
+      auto barrier = [&]() __attribute__((always_inline)) {
+        if (sync) __syncthreads();
+        else __builtin_amdgcn_wave_barrier();
+      };
       uint32_t wo[16], ro[16];
       xor_table(wo, ldc(rd->we, 0), ldc(rd->we, 1), ldc(rd->we, 2), ldc(rd->we, 3));
       xor_table(ro, ldc(rd->re, 0), ldc(rd->re, 1), ldc(rd->re, 2), ldc(rd->re, 3));
@@ -227,19 +235,21 @@ __device__ __forceinline__ void run_sweep(const SweepDesc* __restrict__ d, void*
       if constexpr (decltype(with_a)::value) {
 #pragma unroll
         for (int a = 0; a < A; ++a) Stor<LT>::lds_st_a(bw ^ wo[a], xa[a]);
-        __syncthreads();
+        barrier();
 #pragma unroll
         for (int a = 0; a < A; ++a) xa[a] = Stor<LT>::template lds_ld_a<double>(br ^ ro[a]);
-        if (TWO) __syncthreads();
+        if (TWO) barrier();
       }
       if constexpr (TWO && decltype(with_b)::value) {
+        // opaque again: sharing lambda's addresses with psi's keeps them all live
+        asm volatile("" : "+v"(bw), "+v"(br));
 #pragma unroll
         for (int a = 0; a < A; ++a) Stor<LT>::lds_st_a(bw ^ wo[a], xb[a]);
-        __syncthreads();
+        barrier();
 #pragma unroll
         for (int a = 0; a < A; ++a) xb[a] = Stor<LT>::template lds_ld_a<double>(br ^ ro[a]);
       }
-      if (m1 | m2) __syncthreads();
+      if (m1 | m2) barrier();
     };
     int lo = t;
 #pragma unroll 1

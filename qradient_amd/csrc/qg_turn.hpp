@@ -147,8 +147,13 @@ __device__ __forceinline__ void run_turn(const TurnDesc* __restrict__ d, void* l
     int lo = t;
     // The exchange from the layout at hand into round rd's; each layout is
     // written to the slots it was read from, so only reads need a barrier
-    // before them.
+    // before them, and none inside a wave (see qg_sweep.hpp).
     auto exchange = [&](auto with_a, auto with_b, const TurnRound* __restrict__ rd) __attribute__((always_inline)) {
+      const bool sync = ldc(&rd->sync, 0) != 0;
+      auto barrier = [&]() __attribute__((always_inline)) {
+        if (sync) __syncthreads();
+        else __builtin_amdgcn_wave_barrier();
+      };
       uint32_t wo[16], ro[16];
       xor_table(wo, ldc(rd->we, 0), ldc(rd->we, 1), ldc(rd->we, 2), ldc(rd->we, 3));
       xor_table(ro, ldc(rd->re, 0), ldc(rd->re, 1), ldc(rd->re, 2), ldc(rd->re, 3));
@@ -158,15 +163,17 @@ __device__ __forceinline__ void run_turn(const TurnDesc* __restrict__ d, void* l
       if constexpr (decltype(with_a)::value) {
 #pragma unroll
         for (int a = 0; a < A; ++a) Stor<LT>::lds_st_a(bw ^ wo[a], xa[a]);
-        __syncthreads();
+        barrier();
 #pragma unroll
         for (int a = 0; a < A; ++a) xa[a] = Stor<LT>::template lds_ld_a<double>(br ^ ro[a]);
-        if (TWO) __syncthreads();
+        if (TWO) barrier();
       }
       if constexpr (TWO && decltype(with_b)::value) {
+        // opaque again: sharing lambda's addresses with psi's keeps them all live
+        asm volatile("" : "+v"(bw), "+v"(br));
 #pragma unroll
         for (int a = 0; a < A; ++a) Stor<LT>::lds_st_a(bw ^ wo[a], xb[a]);
-        __syncthreads();
+        barrier();
 #pragma unroll
         for (int a = 0; a < A; ++a) xb[a] = Stor<LT>::template lds_ld_a<double>(br ^ ro[a]);
       }
