@@ -25,8 +25,8 @@ hipError_t launch_sweep(int dtype, bool two, const SweepDesc* d, int K, int grid
                         int* occ, int tab);
 hipError_t launch_pass(int dtype, int R, bool two, int phase, bool post, const PassDesc* d, int K, int grid,
                        int batch, int threads, int n, hipStream_t st, int* occ, int tab);
-hipError_t launch_finalize(int nout, const int* ptr, const int* rows, const int* cnt, const double* scale,
-                           const double* part, int stride, double* out, hipStream_t st);
+hipError_t launch_finalize(int nout, const int* ptr, const int2* rows, const double* part, int stride, const double* dot,
+                           double* out, hipStream_t st);
 hipError_t simple_rot1(int dtype, void* v, int n, int b, int type, double c, double s, hipStream_t st);
 hipError_t simple_permute(int dtype, const void* in, void* out, int n, const uint32_t* dmap, hipStream_t st);
 hipError_t simple_diag_phase(int dtype, void* v, int n, const DTerm* dt, int nt, double angle, int cz,
@@ -451,31 +451,30 @@ struct qg_plan {
   uint32_t lad1 = 0, lad2 = 0;  // the ladder map in shift form (gather/scatter)
   uint32_t inv1 = 0, inv2 = 0;  // and its inverse
   double* d_init = nullptr;     // n + 1
-  DTerm* d_terms = nullptr;     // diagonal terms (max_terms)
+  DTerm* d_terms = nullptr;     // diagonal terms, then x / y terms (max_terms of each)
   std::vector<DTerm> h_terms;   // host copy of what d_terms holds for the current run
   std::vector<DTerm> h_cterms;  // the terms split per pass launch (PassDesc::cterms)
   DTerm* d_cterms = nullptr;
   void* d_ini_states = nullptr;  // QAOA: the chunk's initial states (when given)
   size_t ini_cap = 0;            // its size in bytes
   size_t cterm_cap = 0;
-  DTerm* d_xy = nullptr;
+  const DTerm* d_xy = nullptr;  // x / y terms of the current run, behind the diagonal ones in d_terms
   int max_terms = 0;
   double* d_lut = nullptr;
   int lut_len = 0;
   double* d_part = nullptr;
   int gmax = 1, nrows = 0;
-  int* d_fin = nullptr;         // ptr | rows | cnt
+  int* d_fin = nullptr;         // finalize table (see run_finalize)
+  int* h_fin = nullptr;         // pinned
   size_t fin_cap = 0;
   // capacities of the small tables (they only grow, so a plan re-laid out for
   // a shape no larger than one it held before allocates nothing)
   int cap_n = 0;            // d_init (n + 1), h_tabs
   int cap_terms = 0;        // d_terms, d_xy
   size_t cap_part = 0;      // d_part elements (rows x gmax)
-  int cap_nout = 0;         // d_scale, d_out, h_out
+  int cap_nout = 0;         // h_out
   size_t cap_fstate = 0;    // d_fstate bytes
   char* h_tabs = nullptr;   // pinned staging of the initial-state table
-  double* d_scale = nullptr;
-  double* d_out = nullptr;
   double* d_dot = nullptr;      // kDotBlocks + 1
   PassDesc* d_desc = nullptr;
   int ndesc_cap = 0;
@@ -658,9 +657,9 @@ static int ensure_small(qg_plan* p, int ndesc, int nrows, int nout) {
   const bool grow_n = n > p->cap_n || !p->d_init;
   const bool grow_terms = std::max(64, n * n) > p->cap_terms || !p->d_terms;
   const size_t part = (size_t)std::max(1, nrows) * p->gmax;
-  const size_t fin = (size_t)(3 * (nout + 1) + 3 * nrows + 8);
+  const size_t fin = (size_t)(nout + 2 + 2 * nrows);  // a row feeds one output
   const bool grow_part = part > p->cap_part || !p->d_part;
-  const bool grow_out = nout > p->cap_nout || !p->d_out;
+  const bool grow_out = nout > p->cap_nout || !p->h_out;
   const bool grow_fin = fin > p->fin_cap || !p->d_fin;
   const bool grow_desc = ndesc > p->ndesc_cap || !p->d_desc;
   if (grow_n || grow_terms || grow_part || grow_out || grow_fin || grow_desc) {
@@ -680,12 +679,11 @@ static int ensure_small(qg_plan* p, int ndesc, int nrows, int nout) {
   }
   if (grow_terms) {
     (void)hipFree(p->d_terms);
-    (void)hipFree(p->d_xy);
-    p->d_terms = p->d_xy = nullptr;
+    p->d_terms = nullptr;
+    p->d_xy = nullptr;
     p->cap_terms = 0;
     const int mt = std::max(64, n * n);
-    HIPCHK(hipMalloc(&p->d_terms, sizeof(DTerm) * mt));
-    HIPCHK(hipMalloc(&p->d_xy, sizeof(DTerm) * mt));
+    HIPCHK(hipMalloc(&p->d_terms, sizeof(DTerm) * 2 * mt));
     p->cap_terms = mt;
   }
   p->max_terms = p->cap_terms;
@@ -699,20 +697,17 @@ static int ensure_small(qg_plan* p, int ndesc, int nrows, int nout) {
   }
   if (grow_fin) {
     (void)hipFree(p->d_fin);
-    p->d_fin = nullptr;
+    if (p->h_fin) (void)hipHostFree(p->h_fin);
+    p->d_fin = p->h_fin = nullptr;
     p->fin_cap = 0;
     HIPCHK(hipMalloc(&p->d_fin, sizeof(int) * fin));
+    HIPCHK(hipHostMalloc(&p->h_fin, sizeof(int) * fin, hipHostMallocDefault));
     p->fin_cap = fin;
   }
   if (grow_out) {
-    (void)hipFree(p->d_scale);
-    (void)hipFree(p->d_out);
     if (p->h_out) (void)hipHostFree(p->h_out);
-    p->d_scale = p->d_out = nullptr;
     p->h_out = nullptr;
     p->cap_nout = 0;
-    HIPCHK(hipMalloc(&p->d_scale, sizeof(double) * std::max(1, nout)));
-    HIPCHK(hipMalloc(&p->d_out, sizeof(double) * std::max(1, nout)));
     HIPCHK(hipHostMalloc(&p->h_out, sizeof(double) * std::max(1, nout), hipHostMallocDefault));
     p->cap_nout = nout;
   }
@@ -1378,12 +1373,10 @@ static void free_small(qg_plan* p) {
   p->cterm_cap = 0;
   (void)hipFree(p->d_init);
   (void)hipFree(p->d_terms);
-  (void)hipFree(p->d_xy);
   (void)hipFree(p->d_lut);
   (void)hipFree(p->d_part);
   (void)hipFree(p->d_fin);
-  (void)hipFree(p->d_scale);
-  (void)hipFree(p->d_out);
+  if (p->h_fin) (void)hipHostFree(p->h_fin);
   (void)hipFree(p->d_dot);
   (void)hipFree(p->d_desc);
   (void)hipFree(p->d_sweep);
@@ -1415,9 +1408,10 @@ static void free_small(qg_plan* p) {
   p->d_fstate = nullptr;
   p->arena_cap = 0;
   p->d_init = nullptr;
-  p->d_terms = p->d_xy = nullptr;
-  p->d_lut = p->d_part = p->d_scale = p->d_out = p->d_dot = nullptr;
-  p->d_fin = nullptr;
+  p->d_terms = nullptr;
+  p->d_xy = nullptr;
+  p->d_lut = p->d_part = p->d_dot = nullptr;
+  p->d_fin = p->h_fin = nullptr;
   p->d_desc = nullptr;
   p->h_desc = nullptr;
   p->h_out = nullptr;
@@ -2116,29 +2110,39 @@ static int sweep_schedule(qg_plan* p, int nb, const int32_t* axes, const double*
   return flush_rc;
 }
 
-static int upload_finalize(qg_plan* p, const std::vector<std::vector<int>>& out_rows, const std::vector<int>& cnt,
-                           const std::vector<double>& scale) {
+// Sums the partial rows into the outputs and waits for them in p->h_out:
+// output i is the sum of the rows in out_rows[i], row r holding cnt[r] values;
+// output 0 is *dot when given.  The table goes out in one copy from pinned
+// memory, or, while it is small, is read from there by the kernel, which
+// writes the outputs to pinned memory: copies of a few hundred bytes cost 4 us
+// of device time and a gap of 5 to 30 us each (16-qubit grad_run 586 -> 557
+// us, 19-qubit expectation value with x / y terms 249 -> 221 us).
+constexpr size_t kFinReadBytes = 16384;
+
+static int run_finalize(qg_plan* p, const std::vector<std::vector<int>>& out_rows, const std::vector<int>& cnt,
+                        const double* dot = nullptr) {
   const int nout = (int)out_rows.size();
-  std::vector<int> buf;
-  buf.push_back(0);
-  for (int i = 0; i < nout; ++i) buf.push_back(buf.back() + (int)out_rows[i].size());
-  for (int i = 0; i < nout; ++i)
-    for (int r : out_rows[i]) buf.push_back(r);
-  const int rows_off = nout + 1;
-  const int cnt_off = (int)buf.size();
-  for (int r = 0; r < p->nrows; ++r) buf.push_back(r < (int)cnt.size() ? cnt[r] : 0);
-  if (buf.size() > p->fin_cap) {
-    HIPCHK(hipStreamSynchronize(p->ctx->stream));
-    (void)hipFree(p->d_fin);
-    p->d_fin = nullptr;
-    HIPCHK(hipMalloc(&p->d_fin, sizeof(int) * buf.size()));
-    p->fin_cap = buf.size();
+  // ptr[nout + 1], padded to even, then (row, count) pairs
+  const size_t base = ((size_t)nout + 2) & ~(size_t)1;
+  size_t len = base;
+  for (const auto& o : out_rows) len += 2 * o.size();
+  if (len > p->fin_cap || nout > p->cap_nout) return fail(QG_ERR_HIP, "internal: finalize table exceeds its bound");
+  int* t = p->h_fin;
+  size_t at = base;
+  for (int i = 0; i < nout; ++i) {
+    t[i] = (int)((at - base) / 2);
+    for (int r : out_rows[i]) {
+      t[at++] = r;
+      t[at++] = cnt[r];
+    }
   }
-  HIPCHK(hipMemcpyAsync(p->d_fin, buf.data(), sizeof(int) * buf.size(), hipMemcpyHostToDevice, p->ctx->stream));
-  HIPCHK(hipMemcpyAsync(p->d_scale, scale.data(), sizeof(double) * nout, hipMemcpyHostToDevice, p->ctx->stream));
-  HIPCHK(launch_finalize(nout, p->d_fin, p->d_fin + rows_off, p->d_fin + cnt_off, p->d_scale, p->d_part, p->gmax,
-                         p->d_out, p->ctx->stream));
-  // synchronous because the host vectors above die at return
+  t[nout] = (int)((at - base) / 2);
+  const int* tab = t;
+  if (len * sizeof(int) > kFinReadBytes) {
+    HIPCHK(hipMemcpyAsync(p->d_fin, t, sizeof(int) * len, hipMemcpyHostToDevice, p->ctx->stream));
+    tab = p->d_fin;
+  }
+  HIPCHK(launch_finalize(nout, tab, (const int2*)(tab + base), p->d_part, p->gmax, dot, p->h_out, p->ctx->stream));
   HIPCHK(hipStreamSynchronize(p->ctx->stream));
   return QG_OK;
 }
@@ -2184,10 +2188,13 @@ static int run_fused(qg_plan* p, int B, int mode, int lut_w, size_t bytes_per_ci
   const size_t need = (size_t)B * (bytes_per_circuit + 16 * 256 + sizeof(FusedDescH) + sizeof(double) * per_out);
   CHK(ensure_arena(p, need));
   Arena ar{p};
+  // results: written by the kernel to the pinned arena's first bytes (10
+  // qubits, one circuit: 138 -> 124 us against a copy back)
+  double* d_unused = nullptr;
+  double* h_res = ar.take<double>((size_t)B * per_out, &d_unused);
+  const size_t first = ar.used = (ar.used + 255) & ~(size_t)255;
   FusedDescH* d_desc = nullptr;
   FusedDescH* h_desc = ar.take<FusedDescH>(B, &d_desc);
-  double* d_out = nullptr;
-  ar.take<double>((size_t)B * per_out, &d_out);
   for (int b = 0; b < B; ++b) {
     std::memset(&h_desc[b], 0, sizeof(FusedDescH));
     h_desc[b].n = p->n;
@@ -2199,24 +2206,21 @@ static int run_fused(qg_plan* p, int B, int mode, int lut_w, size_t bytes_per_ci
     h_desc[b].inv2 = p->inv2;
     h_desc[b].lut_w = lut_w;
     h_desc[b].init_tab = p->d_init;
-    h_desc[b].out = d_out + (size_t)b * per_out;
+    h_desc[b].out = h_res + (size_t)b * per_out;
     h_desc[b].grad = grad ? 1 : 0;
     h_desc[b].psi_c64 = p->dtype == QG_C64 ? 1 : 0;
     h_desc[b].psi_out = psi_out;
     CHK(fill(b, h_desc[b], ar));
   }
-  HIPCHK(hipMemcpyAsync(p->d_arena, p->h_arena, ar.used, hipMemcpyHostToDevice, c->stream));
+  HIPCHK(hipMemcpyAsync(p->d_arena + first, p->h_arena + first, ar.used - first, hipMemcpyHostToDevice, c->stream));
   HIPCHK(hipEventRecord(c->ev0, c->stream));
   HIPCHK(launch_fused(d_desc, B, p->n, mode, lut_w, c->stream));
   HIPCHK(hipEventRecord(c->ev1, c->stream));
-  const int nout = grad ? per_out : 1;
-  for (int b = 0; b < B && !grad; ++b)
-    HIPCHK(hipMemcpyAsync(out + (size_t)b * per_out, d_out + (size_t)b * per_out, sizeof(double), hipMemcpyDeviceToHost,
-                          c->stream));
-  if (grad)
-    HIPCHK(hipMemcpyAsync(out, d_out, sizeof(double) * (size_t)B * nout, hipMemcpyDeviceToHost, c->stream));
   HIPCHK(hipStreamSynchronize(c->stream));
   HIPCHK(hipEventElapsedTime(&p->last_ms, c->ev0, c->ev1));
+  for (int b = 0; b < B; ++b)
+    std::copy(h_res + (size_t)b * per_out, h_res + (size_t)b * per_out + (grad ? per_out : 1),
+              out + (size_t)b * per_out);
   p->launches.clear();
   return QG_OK;
 }
@@ -2296,12 +2300,17 @@ static int mcclean_run(qg_plan* p, const int32_t* axes, const double* angles, co
   }
   if (!obs.xy.empty() && n > 31) return fail(QG_ERR_UNSUPPORTED, "observables with x/y terms need n <= 31");
   CHK(ensure_workspace(p));
-  if (!obs.diag.empty())
-    HIPCHK(hipMemcpyAsync(p->d_terms, obs.diag.data(), sizeof(DTerm) * obs.diag.size(), hipMemcpyHostToDevice,
-                          c->stream));
-  if (!obs.xy.empty())
-    HIPCHK(hipMemcpyAsync(p->d_xy, obs.xy.data(), sizeof(DTerm) * obs.xy.size(), hipMemcpyHostToDevice,
-                          c->stream));
+  if (!obs.xy.empty()) {
+    // the elementwise observable reads the terms; passes take them split by
+    // their register bits (split_terms)
+    const size_t nd = obs.diag.size(), nx = obs.xy.size();
+    CHK(ensure_stage(p, sizeof(DTerm) * (nd + nx)));
+    DTerm* t = (DTerm*)p->h_stage;
+    std::copy(obs.diag.begin(), obs.diag.end(), t);
+    std::copy(obs.xy.begin(), obs.xy.end(), t + nd);
+    HIPCHK(hipMemcpyAsync(p->d_terms, t, sizeof(DTerm) * (nd + nx), hipMemcpyHostToDevice, c->stream));
+    p->d_xy = p->d_terms + nd;
+  }
   p->h_terms = obs.diag;
   if (ini_state) {
     const size_t N = 1ull << n;
@@ -2361,18 +2370,13 @@ static int mcclean_run(qg_plan* p, const int32_t* axes, const double* angles, co
       }
     }
   }
-  std::vector<double> scale(out_rows.size(), 1.0);
   if (streamed) CHK(stream_flush(p));
   else CHK(run_launches(p, nd));
   HIPCHK(hipEventRecord(c->ev1, c->stream));
   CHK(collect_profile(p));
-  CHK(upload_finalize(p, out_rows, cnt, scale));
+  CHK(run_finalize(p, out_rows, cnt, p->obs_desc < 0 ? p->d_dot + kDotBlocks : nullptr));
   HIPCHK(hipEventElapsedTime(&p->last_ms, c->ev0, c->ev1));
-  const int nout = (int)out_rows.size();
-  HIPCHK(hipMemcpyAsync(p->h_out, p->d_out, sizeof(double) * nout, hipMemcpyDeviceToHost, c->stream));
-  HIPCHK(hipStreamSynchronize(c->stream));
   *E_out = p->h_out[0];
-  if (p->obs_desc < 0) HIPCHK(hipMemcpy(E_out, p->d_dot + kDotBlocks, sizeof(double), hipMemcpyDeviceToHost));
   if (grad) std::memcpy(grad_out, p->h_out + 1, sizeof(double) * L * n);
   return QG_OK;
 }
@@ -2498,9 +2502,6 @@ extern "C" int qg_mcclean_batch_grad_run(qg_plan* p, int B, const int32_t* axes,
     return QG_OK;
   }
   CHK(ensure_workspace(p));
-  if (!obs.diag.empty())
-    HIPCHK(hipMemcpyAsync(p->d_terms, obs.diag.data(), sizeof(DTerm) * obs.diag.size(), hipMemcpyHostToDevice,
-                          c->stream));
   p->h_terms = obs.diag;
   const uint32_t ent_fwd = p->ent == QG_ENT_CNOT ? F_GATHER : F_CZ_PRE;
   const uint32_t ent_rev = p->ent == QG_ENT_CNOT ? F_SCATTER : F_CZ_POST;
@@ -2615,17 +2616,13 @@ extern "C" int qg_mcclean_batch_grad_run(qg_plan* p, int B, const int32_t* axes,
         }
       }
     }
-    std::vector<double> scale(out_rows.size(), 1.0);
     CHK(run_launches(p, nd));
     HIPCHK(hipEventRecord(c->ev1, c->stream));
     CHK(collect_profile(p));
-    CHK(upload_finalize(p, out_rows, cnt, scale));
+    CHK(run_finalize(p, out_rows, cnt));
     float ms = 0.f;
     HIPCHK(hipEventElapsedTime(&ms, c->ev0, c->ev1));
     total_ms += ms;
-    HIPCHK(hipMemcpyAsync(p->h_out, p->d_out, sizeof(double) * (size_t)nb * per_out, hipMemcpyDeviceToHost,
-                          c->stream));
-    HIPCHK(hipStreamSynchronize(c->stream));
     for (int j = 0; j < nb; ++j) {
       const double* o = p->h_out + (size_t)j * per_out;
       E_out[c0 + j] = o[0];
@@ -3390,11 +3387,14 @@ static int turn_schedule(const TurnRun& tr, Hist hist, Lam lam, LutPtr lut_ptr, 
     p->launches.push_back(l);
     // passes go to the device as they are built (graph replay and profiled
     // runs launch the whole list at the end)
-    if (streamed && p->launches.size() - p->stream_next >= 2) CHK(stream_flush(p));
+    // in doubling groups, as single McClean runs (a batch's descriptors: two passes at a time)
+    const size_t due = nb > 8 ? 2 : std::max<size_t>(2, p->stream_next);
+    if (streamed && p->launches.size() - p->stream_next >= due) CHK(stream_flush(p));
     return QG_OK;
   };
   for (int k = 0; k < NP; ++k) {
-    if (passes[k].phase >= 0) CHK(lut_fill(passes[k].phase + 1));
+    // a few circuits' tables go out at once, a batch's layer by layer
+    if (passes[k].phase >= 0) CHK(lut_fill(nb > 8 ? passes[k].phase + 1 : L));
     CHK(launch(k, false));
   }
   for (int k = NP - 1; tr.grad && k >= 0; --k) CHK(launch(k, true));
@@ -3505,12 +3505,10 @@ static int qaoa_run(qg_plan* p, int B, const qg_term* terms, const int32_t* term
   float total_ms = 0.f;
   for (int c0 = 0; c0 < B; c0 += chunk) {
     const int nb = std::min(chunk, B - c0);
-    // terms and phase tables of this chunk, staged in pinned memory and
-    // copied on the stream ahead of the passes
-    const size_t term_bytes = sizeof(DTerm) * (size_t)p->max_terms * nb;
+    // this chunk's phase tables, staged in pinned memory and copied on the
+    // stream ahead of the passes (its terms go out split by register bits)
     const size_t lut_doubles = phase == 1 ? (size_t)nb * 2 * L * lut_len * 2 : 0;
-    CHK(ensure_stage(p, term_bytes + sizeof(double) * lut_doubles));
-    DTerm* tbuf = (DTerm*)p->h_stage;
+    CHK(ensure_stage(p, sizeof(double) * lut_doubles));
     std::vector<int> toff(nb), tcnt(nb);
     p->h_terms.assign((size_t)p->max_terms * nb, DTerm{});
     for (int j = 0; j < nb; ++j) {
@@ -3518,8 +3516,6 @@ static int qaoa_run(qg_plan* p, int B, const qg_term* terms, const int32_t* term
       tcnt[j] = (int)obs[c0 + j].diag.size();
       std::copy(obs[c0 + j].diag.begin(), obs[c0 + j].diag.end(), p->h_terms.begin() + toff[j]);
     }
-    std::memcpy(tbuf, p->h_terms.data(), term_bytes);
-    HIPCHK(hipMemcpyAsync(p->d_terms, tbuf, term_bytes, hipMemcpyHostToDevice, c->stream));
     if (ini) {
       // upload (complex128) and convert to the storage type
       const size_t N = 1ull << n;
@@ -3542,10 +3538,11 @@ static int qaoa_run(qg_plan* p, int B, const qg_term* terms, const int32_t* term
     // the device's passes (about 2.5 ms for 512 circuits, 8 layers, W = 30).
     // cos is even and sin odd (exactly, in the math library), so one sincos
     // per |d| fills four entries.
-    double* lut_host = phase == 1 ? (double*)(p->h_stage + term_bytes) : nullptr;
+    double* lut_host = phase == 1 ? (double*)p->h_stage : nullptr;
     const size_t lut_layer = (size_t)nb * 2 * lut_len * 2;  // doubles per layer
     int lut_filled = 0;
     auto lut_fill = [&](int upto) -> int {
+      const int from = lut_filled;
       for (; phase == 1 && lut_filled < std::min(upto, L); ++lut_filled) {
         const int i = lut_filled;
         double* layer = lut_host + (size_t)i * lut_layer;
@@ -3566,9 +3563,10 @@ static int qaoa_run(qg_plan* p, int B, const qg_term* terms, const int32_t* term
             t1[2 * (Wi - m) + 1] = -sm;
           }
         }
-        HIPCHK(hipMemcpyAsync(p->d_lut + (size_t)i * lut_layer, layer, sizeof(double) * lut_layer,
-                              hipMemcpyHostToDevice, c->stream));
       }
+      if (lut_filled > from)
+        HIPCHK(hipMemcpyAsync(p->d_lut + (size_t)from * lut_layer, lut_host + (size_t)from * lut_layer,
+                              sizeof(double) * lut_layer * (lut_filled - from), hipMemcpyHostToDevice, c->stream));
       return QG_OK;
     };
     auto lut_ptr = [&](int j, int i, int dir) -> const double* {
@@ -3743,7 +3741,6 @@ static int qaoa_run(qg_plan* p, int B, const qg_term* terms, const int32_t* term
         }
       }
     }
-    std::vector<double> scale(out_rows.size(), 1.0);
     if (!grad) {
       for (int j = 0; j < nb; ++j)
         for (int k = 1; k < per_out; ++k) out_rows[(size_t)j * per_out + k].clear();
@@ -3755,13 +3752,10 @@ static int qaoa_run(qg_plan* p, int B, const qg_term* terms, const int32_t* term
     }
     HIPCHK(hipEventRecord(c->ev1, c->stream));
     CHK(collect_profile(p));
-    CHK(upload_finalize(p, out_rows, cnt, scale));
+    CHK(run_finalize(p, out_rows, cnt));
     float ms = 0.f;
     HIPCHK(hipEventElapsedTime(&ms, c->ev0, c->ev1));
     total_ms += ms;
-    const int nout = nb * per_out;
-    HIPCHK(hipMemcpyAsync(p->h_out, p->d_out, sizeof(double) * nout, hipMemcpyDeviceToHost, c->stream));
-    HIPCHK(hipStreamSynchronize(c->stream));
     for (int j = 0; j < nb; ++j) {
       const double* o = p->h_out + (size_t)j * per_out;
       E_out[c0 + j] = o[0];

@@ -16,19 +16,20 @@ hipError_t set_attributes_c64();
 hipError_t set_attributes_c128();
 hipError_t set_attributes_c64x();
 
-// out[i] = scale[i] * sum over the rows r of output i of sum_{w < cnt[r]} part[r*stride + w].
-// One workgroup per output; each thread sums a fixed strided subset, then a
-// fixed-shape tree: the result does not depend on scheduling.
-__global__ __launch_bounds__(256) void k_finalize(int nout, const int* __restrict__ ptr, const int* __restrict__ rows,
-                                                  const int* __restrict__ cnt, const double* __restrict__ scale,
-                                                  const double* __restrict__ part, int stride, double* __restrict__ out) {
+// out[i] = sum over the rows (r, cnt) of output i of sum_{w < cnt} part[r*stride + w];
+// out[0] = *dot when given.  One workgroup per output; each thread sums a fixed
+// strided subset, then a fixed-shape tree: the result does not depend on
+// scheduling.  The table and the outputs may lie in host memory.
+__global__ __launch_bounds__(256) void k_finalize(int nout, const int* __restrict__ ptr, const int2* __restrict__ rows,
+                                                  const double* __restrict__ part, int stride,
+                                                  const double* __restrict__ dot, double* __restrict__ out) {
   __shared__ double red[256];
   const int i = blockIdx.x;
   if (i >= nout) return;
   double s = 0.0;
   for (int k = ptr[i]; k < ptr[i + 1]; ++k) {
-    const int r = rows[k];
-    for (int w = threadIdx.x; w < cnt[r]; w += blockDim.x) s += part[(size_t)r * stride + w];
+    const int2 r = rows[k];
+    for (int w = threadIdx.x; w < r.y; w += blockDim.x) s += part[(size_t)r.x * stride + w];
   }
   red[threadIdx.x] = s;
   __syncthreads();
@@ -36,13 +37,13 @@ __global__ __launch_bounds__(256) void k_finalize(int nout, const int* __restric
     if ((int)threadIdx.x < h) red[threadIdx.x] += red[threadIdx.x + h];
     __syncthreads();
   }
-  if (threadIdx.x == 0) out[i] = scale[i] * red[0];
+  if (threadIdx.x == 0) out[i] = i == 0 && dot ? *dot : red[0];
 }
 
-hipError_t launch_finalize(int nout, const int* ptr, const int* rows, const int* cnt, const double* scale,
-                           const double* part, int stride, double* out, hipStream_t st) {
+hipError_t launch_finalize(int nout, const int* ptr, const int2* rows, const double* part, int stride,
+                           const double* dot, double* out, hipStream_t st) {
   if (nout <= 0) return hipSuccess;
-  hipLaunchKernelGGL(k_finalize, dim3(nout), dim3(256), 0, st, nout, ptr, rows, cnt, scale, part, stride, out);
+  hipLaunchKernelGGL(k_finalize, dim3(nout), dim3(256), 0, st, nout, ptr, rows, part, stride, dot, out);
   return hipGetLastError();
 }
 
