@@ -74,7 +74,13 @@ struct FusedDescH {
   void* psi_out;
 };
 // and of its FusedMode
-enum FusedMode : int32_t { FM_MCCLEAN = 0, FM_QAOA_LUT = 1, FM_QAOA_SINCOS = 2, FM_QAOA_LARGE = 3 };
+enum FusedMode : int32_t {
+  FM_MCCLEAN = 0,
+  FM_QAOA_LUT = 1,
+  FM_QAOA_SINCOS = 2,
+  FM_QAOA_LARGE = 3,
+  FM_QAOA_LUT_LARGE = 4
+};
 constexpr double kSincosMax = 67108864.0;  // phase angles below this take the reduced sincos (qg_math.hpp)
 }  // namespace qg
 
@@ -3466,7 +3472,8 @@ static int qaoa_run(qg_plan* p, int B, const qg_term* terms, const int32_t* term
       HIPCHK(hipMalloc(&p->d_fstate, ((size_t)16) << n));
       p->cap_fstate = (size_t)16 << n;
     }
-    const int mode = turn_ph == TP_LUT ? FM_QAOA_LUT : turn_ph == TP_SINCOS ? FM_QAOA_SINCOS : FM_QAOA_LARGE;
+    const bool large = !(gmax * W < kSincosMax);
+    const int mode = phase == 1 ? (large ? FM_QAOA_LUT_LARGE : FM_QAOA_LUT) : large ? FM_QAOA_LARGE : FM_QAOA_SINCOS;
     CHK(run_fused(p, B, mode, phase == 1 ? Wi : 0, bytes, per, grad, B == 1 ? p->d_fstate : nullptr, fill,
                   res.data()));
     for (int b = 0; b < B; ++b) {

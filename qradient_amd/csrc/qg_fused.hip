@@ -1,7 +1,7 @@
 // Whole-circuit grad_run for states that fit one workgroup (n <= 13).
 //
 // One workgroup runs one circuit end to end: the 2^n amplitudes stay in
-// registers (16 per thread) and LDS for every layer of the forward sweep,
+// registers (16 or 8 per thread) and LDS for every layer of the forward sweep,
 // the observable and the adjoint sweep, so nothing but the parameters and the
 // results crosses HBM.  psi is uncomputed alongside lambda in FP64 (no
 // history: unitary FP64 uncompute drifts by ~1e-15 per layer), so complex64
@@ -22,22 +22,30 @@
 //                       bits with v_permlane16/32_swap: no LDS, no wait
 //   layout 2 (n >= 10)  index bits 0-3 in registers: an LDS exchange inside
 //                       each wave, so no barrier
-//   layout 3 (n >= 11)  the wave bits in registers: an LDS exchange across
+//   layout 3 (n >= 12)  the wave bits in registers: an LDS exchange across
 //                       waves
 //
 // and the ladder's permutation (or the plain way back) is the exchange into
 // layout 0 of the next layer: three LDS round trips a layer where a stage of
-// four bits at a time needs five.  A layout is written to the slots it was
-// read from, so only reads across waves need a barrier.  Up to 11 qubits psi
-// and lambda have a buffer each and share their barriers; above, they take
-// turns in one buffer, which leaves room for a second workgroup on the CU at
-// 12 qubits.  Rotations are the in-place shears of the pass kernels, which
-// need no second copy of the state: the earlier form (direct 2x2 products, all
-// gate types joined by branches) spilled 259 registers.
+// four bits at a time needs five.  10 and 11 qubits would have one and two
+// waves that way and wait alone for every instruction; they hold 8 amplitudes
+// per thread (registers: the top 3 bits; bits 0-2, then 3-5, exchanged inside
+// the waves; the wave bits) in two and four waves: 97 -> 76 us and 124 -> 94
+// us for 10 layers.  At 12 qubits the same form took 126 us against 174 for
+// one circuit but 119 against 110 for a batch of 512, which fills the CUs
+// either way, so 12 qubits keep 16 per thread.
+//
+// A layout is written to the slots it was read from, so only reads across
+// waves need a barrier.  Up to 11 qubits psi and lambda have a buffer each and
+// share their barriers; above, they take turns in one buffer, which leaves
+// room for a second workgroup on the CU at 12 qubits.  Rotations are the
+// in-place shears of the pass kernels, which need no second copy of the state:
+// the earlier form (direct 2x2 products, all gate types joined by branches)
+// spilled 259 registers.
 //
 // Measured (kernel time, MI355X; before -> now): 10 qubits x 10 layers
-// 209 -> 98 us, 13 x 20 959 -> 435 us, 64 QAOA circuits of 12 qubits x 4
-// layers 476 -> 85 us.  At 13 qubits the two waves of a SIMD issue vector
+// 209 -> 76 us, 13 x 20 959 -> 435 us, 64 QAOA circuits of 12 qubits x 4
+// layers 476 -> 70 us.  At 13 qubits the two waves of a SIMD issue vector
 // instructions in 55% of its cycles; the rest waits on LDS and barriers.
 #include "qg_math.hpp"
 #include "qg_pass.hpp"
@@ -75,12 +83,12 @@ struct Layout {
 
 template <int N>
 struct Shape {
-  static constexpr int R = N < kRegBits ? N : kRegBits;
+  static constexpr int R = N < kRegBits ? N : N == 10 || N == 11 ? 3 : kRegBits;
   static constexpr int T = N - R;              // thread bits
   static constexpr int NT = 1 << T;            // threads
   static constexpr int W = T > 6 ? T - 6 : 0;  // wave bits
   // stages per layer, each with its layout
-  static constexpr int NS = N >= 11 ? 4 : N == 10 ? 3 : T == 0 ? 1 : T <= 4 ? 2 : 3;
+  static constexpr int NS = N >= 10 ? 4 : T == 0 ? 1 : T <= 4 ? 2 : 3;
   static constexpr bool TWO_BUF = N <= 11;     // psi and lambda have an LDS buffer each
 };
 
@@ -96,19 +104,32 @@ constexpr Layout layout(int s) {
     for (int j = 0; j < T; ++j) o.thr[j] = j < lo ? j : j + R;
     return o;
   }
-  for (int k = 0; k < 4; ++k) o.reg[k] = T + k;
+  for (int k = 0; k < R; ++k) o.reg[k] = T + k;
   for (int j = 0; j < T; ++j) o.thr[j] = j;
-  if (s == 1) {
+  // lanes are ordered so that the first four cover the four low slot bits
+  // under the swizzle (no bank conflicts)
+  if constexpr (R == 3) {
+    if (s < 3) {
+      for (int k = 0; k < 3; ++k) o.reg[k] = 3 * (s - 1) + k;
+      const int lanes[2][2][6] = {{{3, 4, 5, 9, 7, 8}, {3, 4, 5, 9, 8, 10}}, {{0, 1, 2, 7, 8, 9}, {0, 1, 2, 10, 8, 9}}};
+      for (int j = 0; j < 6; ++j) o.thr[j] = lanes[s - 1][N - 10][j];
+    } else {
+      // the wave bits into registers, filled up with bits 5 and 4
+      for (int k = 0; k < 3; ++k) o.reg[k] = k < W ? 6 + k : 5 - (k - W);
+      const int lanes[2][6] = {{0, 1, 2, 3, 7, 8}, {0, 1, 2, 3, 4, 8}};
+      for (int j = 0; j < 6; ++j) o.thr[j] = lanes[N - 10][j];
+      for (int k = 0; k < W; ++k) o.thr[6 + k] = 9 + k;
+    }
+  } else if (s == 1) {
     o.reg[0] = 4;
     o.reg[1] = 5;
     o.thr[4] = T;
     o.thr[5] = T + 1;
   } else if (s == 2) {
-    // lanes: the six bits 4, 5, T .. T + 3, ordered so that the first four
-    // cover the four low slot bits under the swizzle (no bank conflicts)
+    // lanes: the six bits 4, 5, T .. T + 3
     for (int k = 0; k < 4; ++k) o.reg[k] = k;
-    const int lanes[4][6] = {{4, 5, 6, 7, 8, 9}, {4, 5, 10, 7, 8, 9}, {4, 5, 10, 11, 8, 9}, {4, 5, 10, 11, 9, 12}};
-    for (int j = 0; j < 6; ++j) o.thr[j] = lanes[N - 10][j];
+    const int lanes[2][6] = {{4, 5, 10, 11, 8, 9}, {4, 5, 10, 11, 9, 12}};
+    for (int j = 0; j < 6; ++j) o.thr[j] = lanes[N - 12][j];
   } else {
     // wave bits into registers, register bits into the waves
     for (int k = 0; k < W; ++k) {
@@ -130,10 +151,14 @@ constexpr bool gates_here(int s, int k) {
   return true;
 }
 
-// LDS slot of index j: every four bits from bit 4 up are XORed into the low
-// four, so that 16 consecutive lanes of every layout above fall on 16
-// different slots modulo 16 (16-byte slots, 64 banks).
-__host__ __device__ constexpr uint32_t fslot(uint32_t j) { return j ^ (((j >> 4) ^ (j >> 8) ^ (j >> 12)) & 15u); }
+// LDS slot of index j: the bits from 4 up are folded into the low four, so
+// that 16 consecutive lanes of every layout above fall on 16 different slots
+// modulo 16 (16-byte slots, 64 banks).
+template <int N>
+__host__ __device__ constexpr uint32_t fslot(uint32_t j) {
+  if constexpr (Shape<N>::R == 3) return j ^ (((j >> 4) ^ (j >> 7) ^ (j >> 10)) & 15u);
+  else return j ^ (((j >> 4) ^ (j >> 8) ^ (j >> 12)) & 15u);
+}
 
 template <int N, int S>
 __device__ __forceinline__ uint32_t thread_index(uint32_t tid) {
@@ -173,7 +198,7 @@ __device__ __forceinline__ void put(const Cd (&x)[1 << Shape<N>::R], uint32_t ba
   asm volatile("" : "+v"(base));
   static_for<(1 << Shape<N>::R)>([&](auto ac) __attribute__((always_inline)) {
     constexpr int a = decltype(ac)::value;
-    constexpr uint32_t c = fslot(reg_index<N, S>(a)) << 4;
+    constexpr uint32_t c = fslot<N>(reg_index<N, S>(a)) << 4;
     Stor<double>::lds_st_a(base ^ c, x[a]);
   });
 }
@@ -182,7 +207,7 @@ __device__ __forceinline__ void get(Cd (&x)[1 << Shape<N>::R], uint32_t base) {
   asm volatile("" : "+v"(base));  // opaque (see put)
   static_for<(1 << Shape<N>::R)>([&](auto ac) __attribute__((always_inline)) {
     constexpr int a = decltype(ac)::value;
-    constexpr uint32_t c = fslot(reg_index<N, S>(a)) << 4;
+    constexpr uint32_t c = fslot<N>(reg_index<N, S>(a)) << 4;
     x[a] = Stor<double>::template lds_ld_a<double>(base ^ c);
   });
 }
@@ -192,7 +217,7 @@ __device__ __forceinline__ void get_map(Cd (&x)[1 << Shape<N>::R], uint32_t base
   asm volatile("" : "+v"(base));  // opaque (see put)
   static_for<(1 << Shape<N>::R)>([&](auto ac) __attribute__((always_inline)) {
     constexpr int a = decltype(ac)::value;
-    const uint32_t c = __builtin_amdgcn_readfirstlane(fslot(ladder_of(reg_index<N, 0>(a), m1, m2)) << 4);
+    const uint32_t c = __builtin_amdgcn_readfirstlane(fslot<N>(ladder_of(reg_index<N, 0>(a), m1, m2)) << 4);
     x[a] = Stor<double>::template lds_ld_a<double>(base ^ c);
   });
 }
@@ -237,11 +262,17 @@ __device__ __forceinline__ void layout_0_to_1(Cd (&x)[16]) {
 // (integer-valued C), by the reduced sincos, or, for angles past its range,
 // by the library's.  Kernels of their own: the code of one in another cost the
 // others registers.
-enum FusedMode : int32_t { FM_MCCLEAN = 0, FM_QAOA_LUT = 1, FM_QAOA_SINCOS = 2, FM_QAOA_LARGE = 3 };
+enum FusedMode : int32_t {
+  FM_MCCLEAN = 0,
+  FM_QAOA_LUT = 1,
+  FM_QAOA_SINCOS = 2,
+  FM_QAOA_LARGE = 3,     // angles past sincos_reduced
+  FM_QAOA_LUT_LARGE = 4  // the same, from a table
+};
 
 template <int N, int MODE>
 struct Fused {
-  static constexpr bool QAOA = MODE != FM_MCCLEAN;
+  static constexpr bool QAOA = MODE != FM_MCCLEAN, TABLE = MODE == FM_QAOA_LUT || MODE == FM_QAOA_LUT_LARGE;
   static constexpr int R = Shape<N>::R, A = 1 << R, T = Shape<N>::T, NT = Shape<N>::NT, NS = Shape<N>::NS;
   static constexpr int NW = (NT + 63) / 64;
   static constexpr int WIDTH = NT < 64 ? NT : 64;
@@ -256,10 +287,10 @@ struct Fused {
   uint32_t b0, b1, b2, b3;  // byte addresses of the thread's amplitude 0 in each layout
 
   __device__ __forceinline__ Fused(const FusedDesc& d_, uint32_t t) : d(d_), tid(t) {
-    b0 = fslot(thread_index<N, 0>(t)) << 4;
-    b1 = NS > 1 ? fslot(thread_index<N, (NS > 1 ? 1 : 0)>(t)) << 4 : 0u;
-    b2 = NS > 2 ? fslot(thread_index<N, (NS > 2 ? 2 : 0)>(t)) << 4 : 0u;
-    b3 = NS > 3 ? fslot(thread_index<N, (NS > 3 ? 3 : 0)>(t)) << 4 : 0u;
+    b0 = fslot<N>(thread_index<N, 0>(t)) << 4;
+    b1 = NS > 1 ? fslot<N>(thread_index<N, (NS > 1 ? 1 : 0)>(t)) << 4 : 0u;
+    b2 = NS > 2 ? fslot<N>(thread_index<N, (NS > 2 ? 2 : 0)>(t)) << 4 : 0u;
+    b3 = NS > 3 ? fslot<N>(thread_index<N, (NS > 3 ? 3 : 0)>(t)) << 4 : 0u;
   }
   template <int S>
   __device__ __forceinline__ uint32_t base(int buf) const {
@@ -273,7 +304,7 @@ struct Fused {
   // layout S -> S + 1, of psi and (TWO) lambda
   template <int S, bool TWO>
   __device__ __forceinline__ void next(Cd (&psi)[A], Cd (&lam)[A]) const {
-    if constexpr (N >= 10 && S == 0) {
+    if constexpr (N >= 10 && R == 4 && S == 0) {
       layout_0_to_1(psi);
       if constexpr (TWO) layout_0_to_1(lam);
     } else {
@@ -298,7 +329,7 @@ struct Fused {
   // the last layout -> layout 0, through the ladder map (MAP) or straight
   template <bool MAP, bool TWO>
   __device__ __forceinline__ void back(Cd (&psi)[A], Cd (&lam)[A], uint32_t m1, uint32_t m2) const {
-    const uint32_t mb = MAP ? fslot(ladder_of(thread_index<N, 0>(tid), m1, m2)) << 4 : b0;
+    const uint32_t mb = MAP ? fslot<N>(ladder_of(thread_index<N, 0>(tid), m1, m2)) << 4 : b0;
     auto rd = [&](Cd (&x)[A], int buf) __attribute__((always_inline)) {
       if constexpr (MAP) get_map<N>(x, mb + (TWO_BUF ? buf * BUF : 0u), m1, m2);
       else get<N, 0>(x, base<0>(buf));
@@ -397,7 +428,8 @@ struct Fused {
     lds_point<MANY>();  // the previous layer's reads are done
     for (int k = (int)tid; k <= w; k += NT) {
       double sn, cs;
-      sincos_phase(g * (double)k, &sn, &cs);
+      if constexpr (MODE == FM_QAOA_LUT) sincos_reduced(g * (double)k, &sn, &cs);
+      else sincos_phase(g * (double)k, &sn, &cs);
       lut[2 * (w + k)] = cs;
       lut[2 * (w + k) + 1] = -sn;
       lut[2 * (w - k)] = cs;
@@ -421,7 +453,7 @@ struct Fused {
       }
       psi[a] = cmul(ph, psi[a]);
     };
-    if constexpr (MODE == FM_QAOA_LUT) {
+    if constexpr (TABLE) {
       fill_lut(g, lds);
       const double* lut = lds_d(lds, LUT) + 2 * d.lut_w;
 #pragma unroll
@@ -446,11 +478,11 @@ struct Fused {
       uint32_t bx = b0;
       asm volatile("" : "+v"(bx));
 #pragma unroll
-      for (int a = 0; a < A; ++a) Stor<double>::lds_st_a(bx ^ (fslot(reg_index<N, 0>(a)) << 4), Cd{g * D[a], 0.0});
+      for (int a = 0; a < A; ++a) Stor<double>::lds_st_a(bx ^ (fslot<N>(reg_index<N, 0>(a)) << 4), Cd{g * D[a], 0.0});
       lds_point<false>();
 #pragma unroll 1
       for (uint32_t a = 0; a < (uint32_t)A; ++a) {
-        const uint32_t at = bx ^ (fslot(a << T) << 4);
+        const uint32_t at = bx ^ (fslot<N>(a << T) << 4);
         double sn, cs;
         sincos(Stor<double>::template lds_ld_a<double>(at).re, &sn, &cs);
         Stor<double>::lds_st_a(at, Cd{cs, -sn});
@@ -458,7 +490,7 @@ struct Fused {
       lds_point<false>();
 #pragma unroll
       for (int a = 0; a < A; ++a) {
-        mul(a, Stor<double>::template lds_ld_a<double>(bx ^ (fslot(reg_index<N, 0>(a)) << 4)));
+        mul(a, Stor<double>::template lds_ld_a<double>(bx ^ (fslot<N>(reg_index<N, 0>(a)) << 4)));
         __builtin_amdgcn_sched_barrier(0);
       }
       lds_point<false>();
@@ -514,10 +546,10 @@ struct Fused {
 #pragma unroll 1
       for (int k = 0; k < d.nxy; ++k) {
         const DTerm t = ldc(d.xy, k);
-        const uint32_t px = b0 ^ (fslot(1u << t.a) << 4);
+        const uint32_t px = b0 ^ (fslot<N>(1u << t.a) << 4);
         static_for<A>([&](auto ac) __attribute__((always_inline)) {
           constexpr int a = decltype(ac)::value;
-          constexpr uint32_t c = fslot(reg_index<N, 0>(a)) << 4;
+          constexpr uint32_t c = fslot<N>(reg_index<N, 0>(a)) << 4;
           const Cd p = Stor<double>::template lds_ld_a<double>(px ^ c);
           if (t.b == 0) {
             lam[a].re += t.w * p.re;
@@ -598,7 +630,7 @@ void k_fused(const FusedDesc* __restrict__ descs) {
 template <int N, int MODE>
 static hipError_t launch_n(const FusedDesc* d, int batch, int lut_w, hipStream_t st, bool st_attr) {
   const int w = st_attr ? kLutMax / 2 : lut_w;
-  const size_t lds = (size_t)Fused<N, MODE>::LUT + (MODE == FM_QAOA_LUT ? 16 * (size_t)(2 * w + 1) : 0);
+  const size_t lds = (size_t)Fused<N, MODE>::LUT + (Fused<N, MODE>::TABLE ? 16 * (size_t)(2 * w + 1) : 0);
   if (st_attr)
     return lds <= 65536 ? hipSuccess
                         : hipFuncSetAttribute(reinterpret_cast<const void*>(&k_fused<N, MODE>),
@@ -614,6 +646,7 @@ static hipError_t launch_mode(const FusedDesc* d, int batch, int mode, int lut_w
     case FM_QAOA_LUT: return launch_n<N, FM_QAOA_LUT>(d, batch, lut_w, st, st_attr);
     case FM_QAOA_SINCOS: return launch_n<N, FM_QAOA_SINCOS>(d, batch, lut_w, st, st_attr);
     case FM_QAOA_LARGE: return launch_n<N, FM_QAOA_LARGE>(d, batch, lut_w, st, st_attr);
+    case FM_QAOA_LUT_LARGE: return launch_n<N, FM_QAOA_LUT_LARGE>(d, batch, lut_w, st, st_attr);
   }
   return hipErrorInvalidValue;
 }
@@ -629,14 +662,14 @@ static hipError_t launch_any(const FusedDesc* d, int batch, int n, int mode, int
 
 // lut_w: the largest lut_w of the batch (FM_QAOA_LUT).
 hipError_t launch_fused(const void* descs, int batch, int n, int mode, int lut_w, hipStream_t st) {
-  if (mode == FM_QAOA_LUT && (lut_w < 0 || 2 * lut_w + 1 > kLutMax)) return hipErrorInvalidValue;
+  if ((mode == FM_QAOA_LUT || mode == FM_QAOA_LUT_LARGE) && (lut_w < 0 || 2 * lut_w + 1 > kLutMax)) return hipErrorInvalidValue;
   return launch_any((const FusedDesc*)descs, batch, n, mode, lut_w, st, false);
 }
 
 hipError_t set_fused_attributes() {
   hipError_t e = hipSuccess;
   for (int n = 1; n <= kFusedMaxN && e == hipSuccess; ++n)
-    for (int mode = FM_MCCLEAN; mode <= FM_QAOA_LARGE && e == hipSuccess; ++mode)
+    for (int mode = FM_MCCLEAN; mode <= FM_QAOA_LUT_LARGE && e == hipSuccess; ++mode)
       e = launch_any(nullptr, 0, n, mode, 0, nullptr, true);
   return e;
 }

@@ -52,3 +52,31 @@
       "+v"(x[M[10]].re), "+v"(x[M[10]].im), "+v"(x[M[11]].re), "+v"(x[M[11]].im), "+v"(x[M[12]].re), \
       "+v"(x[M[12]].im), "+v"(x[M[13]].re), "+v"(x[M[13]].im), "+v"(x[M[14]].re), "+v"(x[M[14]].im), \
       "+v"(x[M[15]].re), "+v"(x[M[15]].im)
+
+// The same for 8 amplitudes per thread: pairs %0..%15, type %16, %17 = a, %18 = b.
+#define QG8_PAIRS(M, op) M(op, 0, 1, 2, 3) M(op, 4, 5, 6, 7) M(op, 8, 9, 10, 11) M(op, 12, 13, 14, 15)
+#define QG8_X1(op, r0, i0, r1, i1) QG_GF(op, r0, "%17", i1) QG_GF(op, i0, "-%17", r1)
+#define QG8_X2(op, r0, i0, r1, i1) QG_GF(op, i1, "-%18", r0) QG_GF(op, r1, "%18", i0)
+#define QG8_Y1(op, r0, i0, r1, i1) QG_GF(op, r0, "-%17", r1) QG_GF(op, i0, "-%17", i1)
+#define QG8_Y2(op, r0, i0, r1, i1) QG_GF(op, r1, "%18", r0) QG_GF(op, i1, "%18", i0)
+#define QG8_Z1(op, r0, i0, r1, i1) QG_GF(op, r0, "%17", i0) QG_GF(op, r1, "-%17", i1)
+#define QG8_Z2(op, r0, i0, r1, i1) QG_GF(op, i0, "-%18", r0) QG_GF(op, i1, "%18", r1)
+
+#define QG8_GATE_ASM(op)                                                                  \
+  "s_cmp_eq_u32 %16, 1\n\t"                                                               \
+  "s_cbranch_scc1 1f\n\t"                                                                 \
+  "s_cmp_eq_u32 %16, 2\n\t"                                                               \
+  "s_cbranch_scc1 2f\n\t"                                                                 \
+  "s_cmp_eq_u32 %16, 3\n\t"                                                               \
+  "s_cbranch_scc1 3f\n\t"                                                                 \
+  "s_branch 4f\n"                                                                         \
+  "1:\n\t" QG8_PAIRS(QG8_X1, op) QG8_PAIRS(QG8_X2, op) QG8_PAIRS(QG8_X1, op) "s_branch 4f\n" \
+  "2:\n\t" QG8_PAIRS(QG8_Y1, op) QG8_PAIRS(QG8_Y2, op) QG8_PAIRS(QG8_Y1, op) "s_branch 4f\n" \
+  "3:\n\t" QG8_PAIRS(QG8_Z1, op) QG8_PAIRS(QG8_Z2, op) QG8_PAIRS(QG8_Z1, op) "\n"           \
+  "4:\n\t"
+
+#define QG8_GATE_OPERANDS(x, M)                                                                   \
+  "+v"(x[M[0]].re), "+v"(x[M[0]].im), "+v"(x[M[1]].re), "+v"(x[M[1]].im), "+v"(x[M[2]].re),        \
+      "+v"(x[M[2]].im), "+v"(x[M[3]].re), "+v"(x[M[3]].im), "+v"(x[M[4]].re), "+v"(x[M[4]].im),     \
+      "+v"(x[M[5]].re), "+v"(x[M[5]].im), "+v"(x[M[6]].re), "+v"(x[M[6]].im), "+v"(x[M[7]].re),     \
+      "+v"(x[M[7]].im)

@@ -593,6 +593,11 @@ __device__ __forceinline__ void gate_bit_s(Cx<T> (&x)[1 << R], int type, double 
     }
     return;
   }
+  if constexpr (R == 3 && std::is_same<T, double>::value) {
+    constexpr PairOrder po = pair_order(KK);  // its first half: the amplitudes below 8
+    asm(QG8_GATE_ASM("v_fma_f64") : QG8_GATE_OPERANDS(x, po.m) : "s"(type), "s"(ad), "s"(bd) : "scc");
+    return;
+  }
   const T a = (T)ad, b = (T)bd, na = (T)(-ad), nb = (T)(-bd);
   if (type == G_X) {
 #pragma unroll

@@ -86,3 +86,20 @@ def test_ini_states(gpu, p):
     ini = rs.standard_normal(1 << 15) + 1j * rs.standard_normal(1 << 15)
     ini /= np.linalg.norm(ini)
     _check(15, p, 'complex128', 'real', batch=2, ini=ini)
+
+
+@pytest.mark.parametrize('n', [2, 9, 10, 11, 12, 13])
+def test_large_angles_from_a_table(gpu, n):
+    """Whole-circuit runs with integer weights and angles past 2^26: the
+    table's arguments are the oracle's products, so the bar is the usual one
+    times the libraries' sincos (1e-12 covers both)."""
+    from qradient_amd.batch import QaoaBatch
+    rs = np.random.RandomState(n)
+    zz = np.full((n, n), None)
+    for i in range(n - 1):
+        zz[i, i + 1] = 1.0
+    betas, gammas = rs.uniform(0, 3, (1, 3)), np.array([[1.0e8, -2.5e8, 0.7]])
+    E, g = QaoaBatch(n, 3, 1).grad_run([{'zz': zz}], betas, gammas)
+    Eo, go = sv.qaoa_grad_run_adjoint(n, {'zz': zz}, betas[0], gammas[0])
+    assert abs(E[0] - Eo) <= 1e-12 * n
+    assert rel_err(np.asarray(g[0]).reshape(-1), np.asarray(go).reshape(-1)) <= 1e-12
