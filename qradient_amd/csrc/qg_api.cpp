@@ -21,18 +21,18 @@ hipError_t set_sweep_attributes();
 hipError_t set_turn_attributes();
 hipError_t launch_turn(int dtype, bool two, int ph, const TurnDesc* d, int K, int grid, int batch, int n,
                        hipStream_t st, int* occ, int tab);
-hipError_t launch_sweep(int dtype, bool two, const SweepDesc* d, int K, int grid, int batch, int n, hipStream_t st,
-                        int* occ, int tab);
+hipError_t launch_sweep(int dtype, bool two, bool obs, const SweepDesc* d, int K, int grid, int batch, int n,
+                        hipStream_t st, int* occ, int tab);
 hipError_t launch_pass(int dtype, int R, bool two, int phase, bool post, const PassDesc* d, int K, int grid,
                        int batch, int threads, int n, hipStream_t st, int* occ, int tab);
 hipError_t launch_finalize(int nout, const int* ptr, const int2* rows, const double* part, int stride, const double* dot,
-                           double* out, hipStream_t st);
+                           int ndot, double* out, hipStream_t st);
 hipError_t simple_rot1(int dtype, void* v, int n, int b, int type, double c, double s, hipStream_t st);
 hipError_t simple_permute(int dtype, const void* in, void* out, int n, const uint32_t* dmap, hipStream_t st);
 hipError_t simple_diag_phase(int dtype, void* v, int n, const DTerm* dt, int nt, double angle, int cz,
                              hipStream_t st);
 hipError_t simple_obs_apply(int dtype, const void* in, void* out, int n, const DTerm* dt, int ndt, const DTerm* xy,
-                            int nxy, hipStream_t st);
+                            int nxy, double* part, int* blocks, hipStream_t st);
 hipError_t simple_dot(int dtype, const void* a, const void* b, int n, int mode, double* part, double* out,
                       hipStream_t st);
 hipError_t simple_init(int dtype, void* v, int n, const double* tab, hipStream_t st);
@@ -481,7 +481,7 @@ struct qg_plan {
   int cap_nout = 0;         // h_out
   size_t cap_fstate = 0;    // d_fstate bytes
   char* h_tabs = nullptr;   // pinned staging of the initial-state table
-  double* d_dot = nullptr;      // kDotBlocks + 1
+  double* d_dot = nullptr;      // kObsBlocks
   PassDesc* d_desc = nullptr;
   int ndesc_cap = 0;
   // pinned staging
@@ -523,7 +523,8 @@ struct qg_plan {
   // McClean with x / y observable terms on the pass kernels: lambda = O psi
   // and E = Re<psi|lambda> by the elementwise kernels (a kind-1 launch)
   const void* gen_in = nullptr;
-  void* gen_out = nullptr;
+  void* gen_out = nullptr;  // NULL: E only
+  int gen_blocks = 0;       // partial sums of E in d_dot
   int gen_ndiag = 0, gen_nxy = 0;
   int obs_desc = -1;     // McClean: descriptor whose row K holds E
   int adj_desc = -1;     // McClean: first adjoint descriptor
@@ -607,7 +608,7 @@ static int grid_for_pass(const qg_plan* p, const Geo& g, bool two, bool post, in
 // per-thread sums outlive a tile).
 static int grid_for_sweep(const qg_plan* p, int K, bool two) {
   int occ = 0;
-  if (launch_sweep(kdtype(p, two), two, nullptr, K, 0, 1, p->n, nullptr, &occ, 0) != hipSuccess || occ < 1) occ = 1;
+  if (launch_sweep(kdtype(p, two), two, false, nullptr, K, 0, 1, p->n, nullptr, &occ, 0) != hipSuccess || occ < 1) occ = 1;
   const uint64_t ntiles = 1ull << (p->n - K);
   const uint64_t target = (uint64_t)p->ctx->num_cu * occ * kWgOversub;
   uint64_t grid = 1;
@@ -717,7 +718,7 @@ static int ensure_small(qg_plan* p, int ndesc, int nrows, int nout) {
     HIPCHK(hipHostMalloc(&p->h_out, sizeof(double) * std::max(1, nout), hipHostMallocDefault));
     p->cap_nout = nout;
   }
-  if (!p->d_dot) HIPCHK(hipMalloc(&p->d_dot, sizeof(double) * (kDotBlocks + 1)));
+  if (!p->d_dot) HIPCHK(hipMalloc(&p->d_dot, sizeof(double) * kObsBlocks));
   if (grow_desc) {
     (void)hipFree(p->d_desc);
     if (p->h_desc) (void)hipHostFree(p->h_desc);
@@ -1061,23 +1062,20 @@ static void drop_graph(qg_plan* p) {
   p->gsig.clear();
 }
 
-// lambda = O psi with x / y terms (k_obs_apply) and E = Re<psi|lambda> into
-// d_dot[kDotBlocks]: the observable step of a McClean run whose observable
-// the pass kernels' diagonal form cannot carry.
+// lambda = O psi with x / y terms (gradient runs only) and E's partial sums
+// into d_dot: the observable step of a McClean run whose observable the pass
+// kernels' diagonal form cannot carry.
 static hipError_t launch_generic_obs(qg_plan* p) {
-  hipError_t e = simple_obs_apply(p->dtype, p->gen_in, p->gen_out, p->n, p->d_terms, p->gen_ndiag, p->d_xy,
-                                  p->gen_nxy, p->ctx->stream);
-  if (e == hipSuccess)
-    e = simple_dot(p->dtype, p->gen_in, p->gen_out, p->n, 0, p->d_dot, p->d_dot + kDotBlocks, p->ctx->stream);
-  return e;
+  return simple_obs_apply(p->dtype, p->gen_in, p->gen_out, p->n, p->d_terms, p->gen_ndiag, p->d_xy, p->gen_nxy,
+                          p->d_dot, &p->gen_blocks, p->ctx->stream);
 }
 
 static hipError_t launch_one(qg_plan* p, const Launch& l) {
   if (l.kind == 1) return launch_generic_obs(p);
   if (l.kind != 0) return hipSuccess;
   if (l.sweep)
-    return launch_sweep(kdtype(p, l.two), l.two, p->d_sweep + l.desc, l.K, l.grid, l.batch, p->n, p->ctx->stream,
-                        nullptr, l.tab);
+    return launch_sweep(kdtype(p, l.two), l.two, l.post, p->d_sweep + l.desc, l.K, l.grid, l.batch, p->n,
+                        p->ctx->stream, nullptr, l.tab);
   if (l.turn)
     return launch_turn(p->dtype == QG_C64 ? 1 : 0, l.two, l.phase, p->d_turn + l.desc, l.K, l.grid, l.batch, p->n,
                        p->ctx->stream, nullptr, l.tab);
@@ -1531,6 +1529,7 @@ static int mcclean_geometry(qg_plan* p) {
 //    steps (1761 | 2132);
 //  - beyond, the state streams from memory in whole 64-byte lines: c = 3, 4
 //    steps (25 qubits 12.6 ms against 13.5 ms).
+constexpr size_t kFoldObs = (size_t)32 << 20;      // bytes (see sweep_schedule)
 constexpr size_t kCachedState = (size_t)64 << 20;  // bytes; two of them fit the 256 MiB cache
 
 static void plan_sweeps(qg_plan* p) {
@@ -1574,8 +1573,9 @@ static int ensure_sweeps(qg_plan* p, int circuits) {
   p->d_sweep = nullptr;
   p->h_sweep = nullptr;
   p->sweep_cap = 0;
-  HIPCHK(hipMalloc(&p->d_sweep, sizeof(SweepDesc) * need));
-  HIPCHK(hipHostMalloc(&p->h_sweep, sizeof(SweepDesc) * need, hipHostMallocDefault));
+  // and a slot for the observable's DiagForm behind them
+  HIPCHK(hipMalloc(&p->d_sweep, sizeof(SweepDesc) * (need + 1)));
+  HIPCHK(hipHostMalloc(&p->h_sweep, sizeof(SweepDesc) * (need + 1), hipHostMallocDefault));
   p->sweep_cap = need;
   return QG_OK;
 }
@@ -1794,7 +1794,7 @@ static int mcclean_schedule(qg_plan* p, const int32_t* axes, const double* angle
     l.kind = 1;
     p->launches.push_back(l);
     p->gen_in = cur;
-    p->gen_out = lam[0];
+    p->gen_out = grad ? lam[0] : nullptr;
     p->gen_ndiag = (int)obs.diag.size();
     p->gen_nxy = (int)obs.xy.size();
   }
@@ -1898,6 +1898,71 @@ static void bond_masks(uint32_t b1, uint32_t b2, bool inverse, int shift, uint32
   *m2 = put((first << 1) & (second << 2));
 }
 
+// The diagonal form of one circuit split by register bits (see split_terms).
+struct DiagSplit {
+  size_t off;
+  int nct, nht[4];
+  double pwc[16];
+};
+
+static void diag_split(const DTerm* terms, int nt, const int (&rpos)[4], std::vector<DTerm>& out, DiagSplit& s) {
+  auto regk = [&](int b) {
+    for (int k = 0; k < 4; ++k)
+      if (rpos[k] == b) return k;
+    return -1;
+  };
+  auto sgn = [](int a, int k) { return ((a >> k) & 1) ? -1.0 : 1.0; };
+  s.off = out.size();
+  s.nct = 0;
+  for (int k = 0; k < 4; ++k) s.nht[k] = 0;
+  for (int a = 0; a < 16; ++a) s.pwc[a] = 0.0;
+  for (int i = 0; i < nt; ++i) {
+    const DTerm& t = terms[i];
+    const int ka = regk(t.a), kb = t.b >= 0 ? regk(t.b) : -1;
+    if (ka < 0 && kb < 0) {
+      out.push_back({(int32_t)((1u << t.a) | (t.b >= 0 ? 1u << t.b : 0u)), 0, t.w});
+      s.nct++;
+    } else if (t.b < 0 || (ka >= 0 && kb >= 0)) {
+      for (int a = 0; a < 16; ++a) s.pwc[a] += t.w * sgn(a, ka) * (t.b < 0 ? 1.0 : sgn(a, kb));
+    }
+  }
+  for (int k = 0; k < 4; ++k)
+    for (int i = 0; i < nt; ++i) {
+      const DTerm& t = terms[i];
+      if (t.b < 0) continue;
+      const int ka = regk(t.a), kb = regk(t.b);
+      if ((ka < 0) == (kb < 0) || (ka >= 0 ? ka : kb) != k) continue;
+      out.push_back({(int32_t)(1u << (ka >= 0 ? t.b : t.a)), 0, t.w});
+      s.nht[k]++;
+    }
+}
+
+// Copies a split into a descriptor (whose terms lie at off in the plan's table).
+template <class D>
+static void set_split(const qg_plan* p, D& d, const DiagSplit& s) {
+  d.cterms = p->d_cterms + s.off;
+  d.nct = s.nct;
+  std::copy(s.nht, s.nht + 4, d.nht);
+  std::copy(s.pwc, s.pwc + 16, d.pwc);
+}
+
+// Global bits of local bits [lo, lo + 4) of a pass.
+static void register_bits(const Geo& G, int lo, int (&rpos)[4]) {
+  for (int k = 0; k < 4; ++k) {
+    const int l = lo + k;
+    rpos[k] = l < G.c ? l : G.p + (l - G.c);
+  }
+}
+
+// Sends the split terms built so far (stream_begin has made room for them).
+static int send_splits(qg_plan* p) {
+  if (p->h_cterms.empty()) return QG_OK;
+  std::memcpy(p->h_cstage, p->h_cterms.data(), sizeof(DTerm) * p->h_cterms.size());
+  HIPCHK(hipMemcpyAsync(p->d_cterms, p->h_cstage, sizeof(DTerm) * p->h_cterms.size(), hipMemcpyHostToDevice,
+                        p->ctx->stream));
+  return QG_OK;
+}
+
 // Builds the launches of one McClean run (nb circuits: circuit j's parameters
 // at axes + j * L * n and angles + j * L * n) from the plan's multi-layer
 // passes.  out_rows and cnt: the finalize tables (1 + L * n outputs per
@@ -1940,10 +2005,17 @@ static int sweep_schedule(qg_plan* p, int nb, const int32_t* axes, const double*
       src = wsp(p, p->off_prep);
     }
   }
+  // The first adjoint pass forms lambda and E where the observable's own read
+  // and write of the state cost more than a kernel variant that runs once per
+  // call (its code is cold every time): grad_run at 23 qubits, complex128, 9
+  // layers 1997 -> 1950 us, 27 qubits, 10 layers 32.3 -> 31.3 ms, but at 16
+  // qubits 556 -> 571 us.
+  const bool fold = grad && diag_obs && p->S >= kFoldObs;
   // one launch of pass k; fill(j, d) sets circuit j's states
   auto launch = [&](int k, bool two, auto fill) {
     due();
     const PlanPass& s = p->sweep[k];
+    const bool seed = two && fold && k == NP - 1;  // forms lambda and E
     const int K = p->sweep_for[3];
     const Geo G = s.lo == 0 ? make_geo(K, K, n, 0, K) : make_geo(K, s.c, s.lo, s.c, K);
     const int NR = (int)s.rounds.size();
@@ -1957,6 +2029,7 @@ static int sweep_schedule(qg_plan* p, int nb, const int32_t* axes, const double*
     l.grid = grid_for_sweep(p, K, two);
     l.phase = 0;
     l.two = two;
+    l.post = seed;
     l.kind = 0;
     for (int j = 0; j < nb; ++j) {
       SweepDesc& d = p->h_sweep[ns++];
@@ -2022,7 +2095,8 @@ static int sweep_schedule(qg_plan* p, int nb, const int32_t* axes, const double*
       d.r[NR].lo = G.t;
       d.r[NR].m1 = d.r[NR].m2 = d.r[NR].cz = 0;
       exchange(d.r[NR]);
-      uint32_t f = two ? F_LOAD_A | F_LOAD_B : 0u;
+      uint32_t f = two ? F_LOAD_A | (seed ? F_OBS_DIAG : F_LOAD_B) : 0u;
+      if (seed) d.obs = (const DiagForm*)(p->d_sweep + p->sweep_cap);
       if (!cz && (s.rounds[0].b1 | s.rounds[0].b2)) {
         // the bonds before the first round: on the load, or undone on the store
         f |= two ? F_SCATTER : F_GATHER;
@@ -2036,6 +2110,10 @@ static int sweep_schedule(qg_plan* p, int nb, const int32_t* axes, const double*
       if (two) {
         for (int i = 0; i < 4 * NR; ++i) cnt[row + i] = l.grid;
         row += 4 * NR;
+        if (seed) {
+          out_rows[(size_t)j * per_out].push_back(row);
+          cnt[row++] = l.grid;
+        }
       }
     }
     l.tab = (p->h_sweep[l.desc].flags & F_INIT_TAB) ? (int)sizeof(double) * (n + 1) : 0;
@@ -2050,9 +2128,10 @@ static int sweep_schedule(qg_plan* p, int nb, const int32_t* axes, const double*
       d.flags |= F_STORE_A | (cur[j] ? F_LOAD_A | (nt ? F_NT_A : 0u) : (uint32_t)F_INIT_TAB);
       cur[j] = d.a_out;
     });
-  // lambda = O psi and E: a pass of its own, or the elementwise kernels (x / y terms)
+  // lambda = O psi and E: the first adjoint pass (below), a pass of its own,
+  // or the elementwise kernel (x / y terms)
   due();
-  if (diag_obs) {
+  if (diag_obs && !fold) {
     const Geo og = obs_geo(n);
     Launch l;
     l.desc = nd;
@@ -2080,7 +2159,7 @@ static int sweep_schedule(qg_plan* p, int nb, const int32_t* axes, const double*
       row += kMaxK + 1;
     }
     p->launches.push_back(l);
-  } else {
+  } else if (!diag_obs) {
     Launch l;
     l.desc = -1;
     l.R = l.K = l.threads = l.grid = l.phase = l.tab = 0;
@@ -2088,15 +2167,28 @@ static int sweep_schedule(qg_plan* p, int nb, const int32_t* axes, const double*
     l.kind = 1;
     p->launches.push_back(l);
     p->gen_in = cur[0];
-    p->gen_out = lam(0);
+    p->gen_out = grad ? lam(0) : nullptr;
     p->gen_ndiag = (int)obs.diag.size();
     p->gen_nxy = (int)obs.xy.size();
   }
   p->last_state_ptr = (void*)cur[0];
   // adjoint sweep; lambda is updated in place, psi read from the history or
   // taken back in place from the nearest checkpoint
+  if (fold) {
+    // the copy waits for no one here: the device still runs forward passes
+    const PlanPass& s = p->sweep[NP - 1];
+    const int K = p->sweep_for[3];
+    int rpos[4];
+    register_bits(s.lo == 0 ? make_geo(K, K, n, 0, K) : make_geo(K, s.c, s.lo, s.c, K), K - 4, rpos);
+    if (!streamed) CHK(stream_begin(p, std::max<size_t>(1, obs.diag.size())));
+    DiagSplit split;
+    diag_split(obs.diag.data(), (int)obs.diag.size(), rpos, p->h_cterms, split);
+    CHK(send_splits(p));
+    DiagForm* form = (DiagForm*)(p->h_sweep + p->sweep_cap);
+    set_split(p, *form, split);
+    HIPCHK(hipMemcpyAsync(p->d_sweep + p->sweep_cap, form, sizeof(DiagForm), hipMemcpyHostToDevice, p->ctx->stream));
+  }
   if (grad) {
-    std::vector<const void*> psi(cur);
     for (int k = NP - 1; k >= 0; --k)
       launch(k, true, [&](int j, SweepDesc& d) {
         d.b_in = lam(j);
@@ -2118,7 +2210,7 @@ static int sweep_schedule(qg_plan* p, int nb, const int32_t* axes, const double*
 
 // Sums the partial rows into the outputs and waits for them in p->h_out:
 // output i is the sum of the rows in out_rows[i], row r holding cnt[r] values;
-// output 0 is *dot when given.  The table goes out in one copy from pinned
+// with ndot, output 0 is the sum of ndot values in d_dot.  The table goes out in one copy from pinned
 // memory, or, while it is small, is read from there by the kernel, which
 // writes the outputs to pinned memory: copies of a few hundred bytes cost 4 us
 // of device time and a gap of 5 to 30 us each (16-qubit grad_run 586 -> 557
@@ -2126,7 +2218,7 @@ static int sweep_schedule(qg_plan* p, int nb, const int32_t* axes, const double*
 constexpr size_t kFinReadBytes = 16384;
 
 static int run_finalize(qg_plan* p, const std::vector<std::vector<int>>& out_rows, const std::vector<int>& cnt,
-                        const double* dot = nullptr) {
+                        int ndot = 0) {
   const int nout = (int)out_rows.size();
   // ptr[nout + 1], padded to even, then (row, count) pairs
   const size_t base = ((size_t)nout + 2) & ~(size_t)1;
@@ -2148,7 +2240,7 @@ static int run_finalize(qg_plan* p, const std::vector<std::vector<int>>& out_row
     HIPCHK(hipMemcpyAsync(p->d_fin, t, sizeof(int) * len, hipMemcpyHostToDevice, p->ctx->stream));
     tab = p->d_fin;
   }
-  HIPCHK(launch_finalize(nout, tab, (const int2*)(tab + base), p->d_part, p->gmax, dot, p->h_out, p->ctx->stream));
+  HIPCHK(launch_finalize(nout, tab, (const int2*)(tab + base), p->d_part, p->gmax, p->d_dot, ndot, p->h_out, p->ctx->stream));
   HIPCHK(hipStreamSynchronize(p->ctx->stream));
   return QG_OK;
 }
@@ -2356,7 +2448,7 @@ static int mcclean_run(qg_plan* p, const int32_t* axes, const double* angles, co
     for (int k = 0; k <= kMaxK; ++k) cnt[d.row_base + k] = l.grid;
   }
   if (!sweeps) {
-    // E: row K of the observable pass (none with x / y terms: from d_dot)
+    // E: row K of the observable pass (with x / y terms: from d_dot)
     if (p->obs_desc >= 0) {
       const PassDesc& d = p->h_desc[p->obs_desc];
       out_rows[0].push_back(d.row_base + d.K);
@@ -2380,7 +2472,7 @@ static int mcclean_run(qg_plan* p, const int32_t* axes, const double* angles, co
   else CHK(run_launches(p, nd));
   HIPCHK(hipEventRecord(c->ev1, c->stream));
   CHK(collect_profile(p));
-  CHK(run_finalize(p, out_rows, cnt, p->obs_desc < 0 ? p->d_dot + kDotBlocks : nullptr));
+  CHK(run_finalize(p, out_rows, cnt, p->obs_desc < 0 ? p->gen_blocks : 0));
   HIPCHK(hipEventElapsedTime(&p->last_ms, c->ev0, c->ev1));
   *E_out = p->h_out[0];
   if (grad) std::memcpy(grad_out, p->h_out + 1, sizeof(double) * L * n);
@@ -3184,45 +3276,6 @@ struct TurnRun {
   const char* ini = nullptr;  // initial states in the storage type (null: |+>^n)
 };
 
-// The diagonal form of one circuit split by register bits (see split_terms).
-struct TurnSplit {
-  size_t off;
-  int nct, nht[4];
-  double pwc[16];
-};
-
-static void turn_split(const DTerm* terms, int nt, const int (&rpos)[4], std::vector<DTerm>& out, TurnSplit& s) {
-  auto regk = [&](int b) {
-    for (int k = 0; k < 4; ++k)
-      if (rpos[k] == b) return k;
-    return -1;
-  };
-  auto sgn = [](int a, int k) { return ((a >> k) & 1) ? -1.0 : 1.0; };
-  s.off = out.size();
-  s.nct = 0;
-  for (int k = 0; k < 4; ++k) s.nht[k] = 0;
-  for (int a = 0; a < 16; ++a) s.pwc[a] = 0.0;
-  for (int i = 0; i < nt; ++i) {
-    const DTerm& t = terms[i];
-    const int ka = regk(t.a), kb = t.b >= 0 ? regk(t.b) : -1;
-    if (ka < 0 && kb < 0) {
-      out.push_back({(int32_t)((1u << t.a) | (t.b >= 0 ? 1u << t.b : 0u)), 0, t.w});
-      s.nct++;
-    } else if (t.b < 0 || (ka >= 0 && kb >= 0)) {
-      for (int a = 0; a < 16; ++a) s.pwc[a] += t.w * sgn(a, ka) * (t.b < 0 ? 1.0 : sgn(a, kb));
-    }
-  }
-  for (int k = 0; k < 4; ++k)
-    for (int i = 0; i < nt; ++i) {
-      const DTerm& t = terms[i];
-      if (t.b < 0) continue;
-      const int ka = regk(t.a), kb = regk(t.b);
-      if ((ka < 0) == (kb < 0) || (ka >= 0 ? ka : kb) != k) continue;
-      out.push_back({(int32_t)(1u << (ka >= 0 ? t.b : t.a)), 0, t.w});
-      s.nht[k]++;
-    }
-}
-
 // Builds (and, unless the plan replays graphs or profiles, launches) the
 // turning passes of a run; out_rows and cnt as in qaoa_run.
 template <class Hist, class Lam, class LutPtr, class LutFill>
@@ -3282,22 +3335,15 @@ static int turn_schedule(const TurnRun& tr, Hist hist, Lam lam, LutPtr lut_ptr, 
   size_t bound = 0;
   for (int j = 0; j < nb; ++j) bound += (size_t)tr.tcnt[j];
   CHK(stream_begin(p, std::max<size_t>(1, bound * at.size())));
-  std::vector<TurnSplit> split((size_t)nb * at.size());
+  std::vector<DiagSplit> split((size_t)nb * at.size());
   for (size_t a = 0; a < at.size(); ++a) {
     const Geo& G = p->geo[at[a].first];
     int rpos[4];
-    for (int k = 0; k < 4; ++k) {
-      const int l = at[a].second + k;
-      rpos[k] = l < G.c ? l : G.p + (l - G.c);
-    }
+    register_bits(G, at[a].second, rpos);
     for (int j = 0; j < nb; ++j)
-      turn_split(p->h_terms.data() + tr.toff[j], tr.tcnt[j], rpos, p->h_cterms, split[a * nb + j]);
+      diag_split(p->h_terms.data() + tr.toff[j], tr.tcnt[j], rpos, p->h_cterms, split[a * nb + j]);
   }
-  if (!p->h_cterms.empty()) {
-    std::memcpy(p->h_cstage, p->h_cterms.data(), sizeof(DTerm) * p->h_cterms.size());
-    HIPCHK(hipMemcpyAsync(p->d_cterms, p->h_cstage, sizeof(DTerm) * p->h_cterms.size(), hipMemcpyHostToDevice,
-                          p->ctx->stream));
-  }
+  CHK(send_splits(p));
   int nd = 0, row = 0;
   auto launch = [&](int k, bool two) -> int {
     const Pass& ps = passes[k];
@@ -3357,11 +3403,8 @@ static int turn_schedule(const TurnRun& tr, Hist hist, Lam lam, LutPtr lut_ptr, 
       TurnDesc& d = p->h_turn[nd++];
       d = base;
       if (al >= 0) {
-        const TurnSplit& s = split[(size_t)al * nb + j];
-        d.cterms = p->d_cterms + s.off;
-        d.nct = s.nct;
-        std::copy(s.nht, s.nht + 4, d.nht);
-        std::copy(s.pwc, s.pwc + 16, d.pwc);
+        const DiagSplit& s = split[(size_t)al * nb + j];
+        set_split(p, d, s);
       }
       if (ps.phase >= 0) {
         d.phase_gamma = (two ? -1.0 : 1.0) * tr.gammas[(size_t)j * L + ps.phase];
@@ -4152,7 +4195,7 @@ extern "C" int qg_state_multiply_observable(qg_state* s, const qg_term* terms, i
   HIPCHK(hipSetDevice(s->ctx->device));
   ObsSplit o;
   CHK(state_upload_obs(s, terms, nterms, o));
-  HIPCHK(simple_obs_apply(s->dtype, s->v, s->tmp, s->n, s->d_terms, (int)o.diag.size(), s->d_xy, (int)o.xy.size(),
+  HIPCHK(simple_obs_apply(s->dtype, s->v, s->tmp, s->n, s->d_terms, (int)o.diag.size(), s->d_xy, (int)o.xy.size(), nullptr, nullptr,
                           s->ctx->stream));
   std::swap(s->v, s->tmp);
   HIPCHK(hipStreamSynchronize(s->ctx->stream));
@@ -4164,7 +4207,7 @@ extern "C" int qg_state_expec_val(qg_state* s, const qg_term* terms, int nterms,
   HIPCHK(hipSetDevice(s->ctx->device));
   ObsSplit o;
   CHK(state_upload_obs(s, terms, nterms, o));
-  HIPCHK(simple_obs_apply(s->dtype, s->v, s->tmp, s->n, s->d_terms, (int)o.diag.size(), s->d_xy, (int)o.xy.size(),
+  HIPCHK(simple_obs_apply(s->dtype, s->v, s->tmp, s->n, s->d_terms, (int)o.diag.size(), s->d_xy, (int)o.xy.size(), nullptr, nullptr,
                           s->ctx->stream));
   HIPCHK(simple_dot(s->dtype, s->v, s->tmp, s->n, 0, s->d_dot, s->d_dot + kDotBlocks, s->ctx->stream));
   HIPCHK(hipMemcpyAsync(out, s->d_dot + kDotBlocks, sizeof(double), hipMemcpyDeviceToHost, s->ctx->stream));

@@ -17,12 +17,12 @@ hipError_t set_attributes_c128();
 hipError_t set_attributes_c64x();
 
 // out[i] = sum over the rows (r, cnt) of output i of sum_{w < cnt} part[r*stride + w];
-// out[0] = *dot when given.  One workgroup per output; each thread sums a fixed
+// with ndot, out[0] = the sum of dot[0, ndot).  One workgroup per output; each thread sums a fixed
 // strided subset, then a fixed-shape tree: the result does not depend on
 // scheduling.  The table and the outputs may lie in host memory.
 __global__ __launch_bounds__(256) void k_finalize(int nout, const int* __restrict__ ptr, const int2* __restrict__ rows,
                                                   const double* __restrict__ part, int stride,
-                                                  const double* __restrict__ dot, double* __restrict__ out) {
+                                                  const double* __restrict__ dot, int ndot, double* __restrict__ out) {
   __shared__ double red[256];
   const int i = blockIdx.x;
   if (i >= nout) return;
@@ -31,19 +31,21 @@ __global__ __launch_bounds__(256) void k_finalize(int nout, const int* __restric
     const int2 r = rows[k];
     for (int w = threadIdx.x; w < r.y; w += blockDim.x) s += part[(size_t)r.x * stride + w];
   }
+  if (i == 0)
+    for (int w = threadIdx.x; w < ndot; w += blockDim.x) s += dot[w];
   red[threadIdx.x] = s;
   __syncthreads();
   for (int h = blockDim.x / 2; h > 0; h >>= 1) {
     if ((int)threadIdx.x < h) red[threadIdx.x] += red[threadIdx.x + h];
     __syncthreads();
   }
-  if (threadIdx.x == 0) out[i] = i == 0 && dot ? *dot : red[0];
+  if (threadIdx.x == 0) out[i] = red[0];
 }
 
 hipError_t launch_finalize(int nout, const int* ptr, const int2* rows, const double* part, int stride,
-                           const double* dot, double* out, hipStream_t st) {
+                           const double* dot, int ndot, double* out, hipStream_t st) {
   if (nout <= 0) return hipSuccess;
-  hipLaunchKernelGGL(k_finalize, dim3(nout), dim3(256), 0, st, nout, ptr, rows, part, stride, dot, out);
+  hipLaunchKernelGGL(k_finalize, dim3(nout), dim3(256), 0, st, nout, ptr, rows, part, stride, dot, ndot, out);
   return hipGetLastError();
 }
 

@@ -67,6 +67,7 @@ struct PTerm {
 constexpr int kTermsPerLaunch = 16;  // terms measured per pass over the state (general kernel)
 constexpr int kDiagTermsPerLaunch = 24;  // diagonal (Z / ZZ / identity) terms per pass of the mask kernel
 constexpr int kTermPartRows = kDiagTermsPerLaunch;  // partial rows a term launch may write
+constexpr int kObsBlocks = 4096;    // workgroups of an observable pass with x / y terms (partial sums of E)
 constexpr int kTermBlocks = 2048;    // workgroups of a term pass (partials per term)
 constexpr int kSampleBlock = 1024;   // positions per block of the basis sampler
 
@@ -156,6 +157,14 @@ struct SweepRound {
                        // applies: before its gates forward, after them in the adjoint
 };
 
+// A diagonal form split by four register bits (as in PassDesc).
+struct DiagForm {
+  const DTerm* cterms;
+  int32_t nct;
+  int32_t nht[4];
+  double pwc[16];
+};
+
 struct SweepDesc {
   // geometry as in PassDesc; hi: the global bit just above the window (32: none)
   int32_t n, K, t, c, p, hi;
@@ -170,6 +179,8 @@ struct SweepDesc {
   void* b_out;
   const double* init_tab;  // n + 1 entries when F_INIT_TAB
   double* part;
+  // F_OBS_DIAG (adjoint): lambda = D psi is formed here, E goes into row row_base + 4 nr
+  const DiagForm* obs;
   SweepRound r[kMaxRounds + 1];  // and the exchange back to the natural layout
 };
 

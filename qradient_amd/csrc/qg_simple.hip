@@ -85,28 +85,47 @@ __global__ void k_diag_phase(typename V2<S>::T* v, uint32_t N, const DTerm* __re
   v[x].y = (S)im;
 }
 
-// out = O in, O = D(x) + sum_k w_k P_k (P in {X, Y} on global bit b_k).
+// O in, O = D(x) + sum_k w_k P_k (P in {X, Y} on global bit b_k): stored to
+// out when given, and with part also part[block] = this block's share of
+// Re<in|O in>, in a fixed order.  Bound by the reads of in (one per x / y
+// term, mostly from the caches).  One pass instead of applying O, a dot product
+// of both vectors and a sum of its parts; expectation values store nothing (a
+// 19-qubit, 12-layer run, complex128: 174 -> 165 us on the device).
 template <class S>
-__global__ void k_obs_apply(const typename V2<S>::T* __restrict__ in, typename V2<S>::T* __restrict__ out,
-                            uint32_t N, const DTerm* __restrict__ dt, int ndt, const DTerm* __restrict__ xy, int nxy) {
-  const uint32_t x = blockIdx.x * blockDim.x + threadIdx.x;
-  if (x >= N) return;
-  const double D = diag_at(dt, ndt, x);
-  double re = D * (double)in[x].x, im = D * (double)in[x].y;
-  for (int k = 0; k < nxy; ++k) {
-    const int b = xy[k].a;
-    const double w = xy[k].w;
-    const uint32_t y = x ^ (1u << b);
-    const double pr = in[y].x, pi = in[y].y;
-    if (xy[k].b == 0) {  // X
-      re += w * pr; im += w * pi;
-    } else {             // Y: (Y v)_x = -i v_y if bit 0, +i v_y if bit 1
-      const double sg = ((x >> b) & 1u) ? 1.0 : -1.0;
-      re += w * (-sg * pi); im += w * (sg * pr);
+__global__ __launch_bounds__(256) void k_obs(const typename V2<S>::T* __restrict__ in, typename V2<S>::T* __restrict__ out,
+                                             uint32_t N, const DTerm* __restrict__ dt, int ndt,
+                                             const DTerm* __restrict__ xy, int nxy, double* __restrict__ part) {
+  double acc = 0.0;
+  const uint64_t step = (uint64_t)gridDim.x * blockDim.x;
+  for (uint64_t at = blockIdx.x * blockDim.x + threadIdx.x; at < N; at += step) {
+    const uint32_t x = (uint32_t)at;
+    const double D = diag_at(dt, ndt, x);
+    const double vr = in[x].x, vi = in[x].y;
+    double re = D * vr, im = D * vi;
+    for (int k = 0; k < nxy; ++k) {
+      const int b = xy[k].a;
+      const double w = xy[k].w;
+      const uint32_t y = x ^ (1u << b);
+      const double pr = in[y].x, pi = in[y].y;
+      if (xy[k].b == 0) {  // X
+        re += w * pr; im += w * pi;
+      } else {             // Y: (Y v)_x = -i v_y if bit 0, +i v_y if bit 1
+        const double sg = ((x >> b) & 1u) ? 1.0 : -1.0;
+        re += w * (-sg * pi); im += w * (sg * pr);
+      }
     }
+    if (out) {
+      out[x].x = (S)re;
+      out[x].y = (S)im;
+    }
+    acc += vr * re + vi * im;
   }
-  out[x].x = (S)re;
-  out[x].y = (S)im;
+  if (!part) return;
+  __shared__ double red[4];
+  const double w = wave_sum(acc, 64);
+  if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = w;
+  __syncthreads();
+  if (threadIdx.x == 0) part[blockIdx.x] = ((red[0] + red[1]) + red[2]) + red[3];
 }
 
 // part[block] = sum over this block's elements of Re(conj(a) b) (mode 0),
@@ -513,12 +532,16 @@ hipError_t simple_diag_phase(int dtype, void* v, int n, const DTerm* dt, int nt,
   return hipGetLastError();
 }
 
+// out = O in (or nothing with out NULL).  With part, *blocks receives the
+// number of partial sums of <in|O in> in part (at most kObsBlocks).
 hipError_t simple_obs_apply(int dtype, const void* in, void* out, int n, const DTerm* dt, int ndt, const DTerm* xy,
-                            int nxy, hipStream_t st) {
+                            int nxy, double* part, int* blocks, hipStream_t st) {
   if (n < 1 || n > kSimpleMaxN) return hipErrorInvalidValue;
   const uint32_t N = (uint32_t)(1ull << n);
-  QG_DT_SWITCH(dtype, hipLaunchKernelGGL(k_obs_apply<S>, grid_for(N, 256), dim3(256), 0, st,
-                                         (const typename V2<S>::T*)in, (typename V2<S>::T*)out, N, dt, ndt, xy, nxy));
+  const dim3 grid = part ? dim3(std::min<uint32_t>((N + 255) / 256, kObsBlocks)) : grid_for(N, 256);
+  if (blocks) *blocks = (int)grid.x;
+  QG_DT_SWITCH(dtype, hipLaunchKernelGGL(k_obs<S>, grid, dim3(256), 0, st, (const typename V2<S>::T*)in,
+                                         (typename V2<S>::T*)out, N, dt, ndt, xy, nxy, part));
   return hipGetLastError();
 }
 

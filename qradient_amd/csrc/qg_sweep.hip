@@ -4,29 +4,38 @@
 
 namespace qg {
 
-// dtype as in launch_pass: 0 complex128, 1 complex64, 2 complex64 with FP64 LDS tiles.
-hipError_t launch_sweep(int dtype, bool two, const SweepDesc* d, int K, int grid, int batch, int n, hipStream_t st,
-                        int* occ, int tab) {
+namespace {
+
+// Calls f with the kernel variant's template arguments.
+template <class F>
+hipError_t sweep_variant(int dtype, bool two, bool big, bool obs, F&& f) {
+  auto with_mode = [&](auto s, auto b) {
+    if (!two) return f(s, std::false_type{}, b, std::false_type{});
+    return obs ? f(s, std::true_type{}, b, std::true_type{}) : f(s, std::true_type{}, b, std::false_type{});
+  };
+  auto with_big = [&](auto s) { return big ? with_mode(s, std::true_type{}) : with_mode(s, std::false_type{}); };
+  return dtype == 0 ? with_big(double{}) : dtype == 1 ? with_big(float{}) : with_big(F32L64{});
+}
+
+}  // namespace
+
+// dtype as in launch_pass: 0 complex128, 1 complex64, 2 complex64 with FP64
+// LDS tiles.  obs: an adjoint pass that forms lambda.
+hipError_t launch_sweep(int dtype, bool two, bool obs, const SweepDesc* d, int K, int grid, int batch, int n,
+                        hipStream_t st, int* occ, int tab) {
   if (K < kSweepMinK || K > kSweepMaxK || K > n) return hipErrorInvalidValue;
-  const bool big = (n + (dtype == 0 ? 4 : 3)) > 32;
-  switch (dtype * 2 + (two ? 1 : 0)) {
-    case 0: return launch_sweep_t<double, false>(d, K, grid, batch, big, st, occ, tab);
-    case 1: return launch_sweep_t<double, true>(d, K, grid, batch, big, st, occ, tab);
-    case 2: return launch_sweep_t<float, false>(d, K, grid, batch, big, st, occ, tab);
-    case 3: return launch_sweep_t<float, true>(d, K, grid, batch, big, st, occ, tab);
-    case 4: return launch_sweep_t<F32L64, false>(d, K, grid, batch, big, st, occ, tab);
-    case 5: return launch_sweep_t<F32L64, true>(d, K, grid, batch, big, st, occ, tab);
-  }
-  return hipErrorInvalidValue;
+  return sweep_variant(dtype, two, (n + (dtype == 0 ? 4 : 3)) > 32, obs, [&](auto s, auto tw, auto b, auto o) {
+    return launch_sweep_t<decltype(s), decltype(tw)::value, decltype(b)::value, decltype(o)::value>(d, K, grid, batch,
+                                                                                                   st, occ, tab);
+  });
 }
 
 hipError_t set_sweep_attributes() {
-  hipError_t e = set_sweep_attr_t<double, false>();
-  if (e == hipSuccess) e = set_sweep_attr_t<double, true>();
-  if (e == hipSuccess) e = set_sweep_attr_t<float, false>();
-  if (e == hipSuccess) e = set_sweep_attr_t<float, true>();
-  if (e == hipSuccess) e = set_sweep_attr_t<F32L64, false>();
-  if (e == hipSuccess) e = set_sweep_attr_t<F32L64, true>();
+  hipError_t e = hipSuccess;
+  for (int v = 0; v < 24 && e == hipSuccess; ++v)
+    e = sweep_variant(v / 8, v & 1, v & 2, v & 4, [](auto s, auto tw, auto b, auto o) {
+      return set_sweep_attr_t<decltype(s), decltype(tw)::value, decltype(b)::value, decltype(o)::value>();
+    });
   return e;
 }
 

@@ -26,7 +26,8 @@
 // output) and lambda, taking each reduction Im<lam|P_q|psi> (the reference's
 // gradient entries, mc_clean.py:68-76) where its bit is in registers.  psi is
 // rotated back inside the tile and not stored (history mode), or stored
-// (checkpoint mode).
+// (checkpoint mode).  The adjoint of the circuit's last pass forms lambda =
+// D psi and E itself where the observable is diagonal (OBS).
 //
 // Bound: the vector ALU.  A round costs 4 x 48 FMAs per thread and state and
 // an exchange of about 130 instructions (with FP32 tiles half of them
@@ -93,7 +94,7 @@ __host__ __device__ inline size_t sweep_lds_bytes(int dtype, int K, bool two, in
          (size_t)tab_bytes;
 }
 
-template <class S, bool TWO, bool BIG>
+template <class S, bool TWO, bool BIG, bool OBS>
 __device__ __forceinline__ void run_sweep(const SweepDesc* __restrict__ d, void* lds, uint32_t tid_in, uint32_t blk,
                                           uint32_t nblk) {
   constexpr int R = 4, A = 16;
@@ -173,9 +174,12 @@ __device__ __forceinline__ void run_sweep(const SweepDesc* __restrict__ d, void*
     if constexpr (TWO) {
 #pragma unroll
       for (int a = 0; a < A; ++a)
-        rb[a] = BIG ? Stor<G>::template ld_big<G>(d->b_in, adr[a]) : Stor<G>::template ld_o<G>(d->b_in, adr[a]);
+        rb[a] = OBS   ? Cx<G>{(G)0, (G)0}
+                : BIG ? Stor<G>::template ld_big<G>(d->b_in, adr[a])
+                      : Stor<G>::template ld_o<G>(d->b_in, adr[a]);
     }
   };
+  double energy = 0.0;  // OBS: this thread's share of E
   if (PF && rounds > 0) fetch(tile_of(0));
 #pragma unroll 1
   for (uint32_t r = 0; r < rounds; ++r) {
@@ -199,7 +203,19 @@ __device__ __forceinline__ void run_sweep(const SweepDesc* __restrict__ d, void*
 #pragma unroll
       for (int a = 0; a < A; ++a) xa[a] = {(double)ra[a].re, (double)ra[a].im};
     }
-    if constexpr (TWO) {
+    if constexpr (OBS) {
+      const DiagForm* __restrict__ form = d->obs;
+      DiagParts<R> dp;
+      diag_prepare<R>(form, gthr, dp);
+#pragma unroll
+      for (int a = 0; a < A; ++a) {
+        const double D = diag_value<R>(form, dp, a);
+        xb[a] = {D * xa[a].re, D * xa[a].im};
+        energy += xa[a].re * xb[a].re + xa[a].im * xb[a].im;
+        asm volatile("" : "+v"(energy));  // one amplitude at a time (register pressure)
+        __builtin_amdgcn_sched_barrier(0);
+      }
+    } else if constexpr (TWO) {
 #pragma unroll
       for (int a = 0; a < A; ++a) xb[a] = {(double)rb[a].re, (double)rb[a].im};
     }
@@ -332,42 +348,45 @@ __device__ __forceinline__ void run_sweep(const SweepDesc* __restrict__ d, void*
       d->part[(size_t)(d->row_base + (int)i) * d->grid + blk] = v;
     }
   }
+  if constexpr (OBS) {
+    double* red = reinterpret_cast<double*>(lds);  // the tile is done with
+    const double w = wave_sum(energy, 64);
+    if ((tid_in & 63u) == 0u) red[tid_in >> 6] = w;
+    __syncthreads();
+    if (tid_in == 0) {
+      double v = 0.0;
+      for (uint32_t i = 0; i < nthr / 64; ++i) v += red[i];
+      d->part[(size_t)(d->row_base + nr * 4) * d->grid + blk] = v;
+    }
+  }
 }
 
 // blockIdx.y selects one of gridDim.y consecutive descriptors (batched
 // circuits).  Three waves per SIMD where the LDS tiles allow it (FP32 tiles):
 // the complex64 adjoint at 24 qubits took 262 us per pass with 177 registers
 // (two waves) and 222 us with 168.
-template <class S, bool TWO, bool BIG>
+template <class S, bool TWO, bool BIG, bool OBS>
 __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(kernel_dtype<S>() == 1 ? 3 : 2)))
 void k_sweep(const SweepDesc* __restrict__ d) {
   extern __shared__ __align__(16) char lds_dyn[];
-  run_sweep<S, TWO, BIG>(d + blockIdx.y, lds_dyn, threadIdx.x, blockIdx.x, gridDim.x);
+  run_sweep<S, TWO, BIG, OBS>(d + blockIdx.y, lds_dyn, threadIdx.x, blockIdx.x, gridDim.x);
 }
 
 // With occ != NULL nothing is launched: *occ receives the workgroups per CU.
-template <class S, bool TWO>
-hipError_t launch_sweep_t(const SweepDesc* d, int K, int grid, int batch, bool big, hipStream_t st, int* occ, int tab) {
+template <class S, bool TWO, bool BIG, bool OBS>
+hipError_t launch_sweep_t(const SweepDesc* d, int K, int grid, int batch, hipStream_t st, int* occ, int tab) {
   const int threads = 1 << (K - 4);
   const size_t lds = sweep_lds_bytes(kernel_dtype<S>(), K, TWO, tab);
-  if (occ) {
-    if (big) return hipOccupancyMaxActiveBlocksPerMultiprocessor(occ, k_sweep<S, TWO, true>, threads, lds);
-    return hipOccupancyMaxActiveBlocksPerMultiprocessor(occ, k_sweep<S, TWO, false>, threads, lds);
-  }
-  if (big) hipLaunchKernelGGL((k_sweep<S, TWO, true>), dim3(grid, batch), dim3(threads), lds, st, d);
-  else hipLaunchKernelGGL((k_sweep<S, TWO, false>), dim3(grid, batch), dim3(threads), lds, st, d);
+  if (occ) return hipOccupancyMaxActiveBlocksPerMultiprocessor(occ, k_sweep<S, TWO, BIG, OBS>, threads, lds);
+  hipLaunchKernelGGL((k_sweep<S, TWO, BIG, OBS>), dim3(grid, batch), dim3(threads), lds, st, d);
   return hipGetLastError();
 }
 
-template <class S, bool TWO>
+template <class S, bool TWO, bool BIG, bool OBS>
 hipError_t set_sweep_attr_t() {
-  const int lds = (int)sweep_lds_bytes(kernel_dtype<S>(), kSweepMaxK, TWO, 8 * (kMaxQubits + 1));
-  hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(&k_sweep<S, TWO, false>),
-                                     hipFuncAttributeMaxDynamicSharedMemorySize, lds);
-  if (e == hipSuccess)
-    e = hipFuncSetAttribute(reinterpret_cast<const void*>(&k_sweep<S, TWO, true>),
-                            hipFuncAttributeMaxDynamicSharedMemorySize, lds);
-  return e;
+  return hipFuncSetAttribute(reinterpret_cast<const void*>(&k_sweep<S, TWO, BIG, OBS>),
+                             hipFuncAttributeMaxDynamicSharedMemorySize,
+                             (int)sweep_lds_bytes(kernel_dtype<S>(), kSweepMaxK, TWO, 8 * (kMaxQubits + 1)));
 }
 
 }  // namespace qg

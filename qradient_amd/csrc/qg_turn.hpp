@@ -20,11 +20,11 @@
 // phase.  The circuit's last pass forms lambda = D psi itself.  psi is never
 // stored.
 //
-// Bound: the FP64 vector ALU (gates and reductions) with the LDS exchanges,
-// whose conversions cost as much as the gates, then HBM.  256 circuits of 20
-// qubits, 8 layers, complex64: 46.5 -> 32.6 ms (9 + 9 passes instead of 16 +
-// 16); one circuit of 17 qubits, 6 layers, complex128, real weights:
-// 541 -> 274 us.
+// Bound: the vector ALU (gates, reductions, and the FP64 <-> FP32 conversions
+// of the exchanges), then HBM: 84 GB of states would take 18 ms at the copy
+// rate.  256 circuits of 20 qubits, 8 layers, complex64: 46.5 -> 32.0 ms (9 + 9
+// passes instead of 16 + 16); one circuit of 17 qubits, 6 layers, complex128,
+// real weights: 541 -> 251 us.
 #pragma once
 #include "qg_math.hpp"
 #include "qg_sweep.hpp"
