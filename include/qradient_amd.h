@@ -272,7 +272,7 @@ int qg_plan_last_ms(const qg_plan* plan, double* ms);
 int qg_plan_set_profiling(qg_plan* plan, int on);
 /* Per-launch device times (ms) of the profiled runs of the current series,
  * run after run, and their kind (0 forward pass, 1 reverse two-state pass,
- * 2 forward pass fused with the observable, 3 another launch); *count
+ * 2 the observable's pass, 3 another launch); *count
  * receives the launch count, at most cap are written.  The times are read
  * from the events here, so profiled runs pay only for the event records. */
 int qg_plan_pass_times(const qg_plan* plan, int cap, float* ms, int* kinds, int* count);
@@ -282,9 +282,12 @@ int qg_plan_pass_times(const qg_plan* plan, int cap, float* ms, int* kinds, int*
  * of the forward and adjoint passes (r_fwd = r_rev = 4).  The plan is laid out
  * again (its pass count, memory mode and workspace size may change; a
  * caller-supplied workspace that is too small is an error).  Used by the
- * autotuner.  Default: the fewest passes per layer that 13 local bits allow,
- * with the smallest kmax (>= 11 for QG_C64, >= 12 for QG_C128) that keeps it;
- * kmax 13 for QG_C64 states of 4 GiB and more (n >= 29). */
+ * autotuner.  With kmax in 10..13 and kmax - cmin >= 4 a pass runs several
+ * layers on its tile, otherwise one.  Default for such passes: kmax 11, cmin 2
+ * below 20 qubits, else kmax 12 and cmin 2 (states up to 64 MiB) or 3; passes
+ * of one layer: the fewest per layer that 13 local bits allow, with the
+ * smallest kmax (>= 11 for QG_C64, >= 12 for QG_C128) that keeps it, 13 for
+ * QG_C64 states of 4 GiB and more (n >= 29). */
 int qg_plan_tune(qg_plan* plan, int kmax, int cmin, int r_fwd, int r_rev);
 /* on = 1 (default): circuits with n <= kmax run whole in one workgroup each
  * (one launch per call, FP64 throughout); on = 0 uses the pass kernels. */

@@ -364,7 +364,7 @@ __device__ __forceinline__ void run_sweep(const SweepDesc* __restrict__ d, void*
 // blockIdx.y selects one of gridDim.y consecutive descriptors (batched
 // circuits).  Three waves per SIMD where the LDS tiles allow it (FP32 tiles):
 // the complex64 adjoint at 24 qubits took 262 us per pass with 177 registers
-// (two waves) and 222 us with 168.
+// (two waves) and takes 222 us with at most 168.
 template <class S, bool TWO, bool BIG, bool OBS>
 __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(kernel_dtype<S>() == 1 ? 3 : 2)))
 void k_sweep(const SweepDesc* __restrict__ d) {
