@@ -151,8 +151,12 @@ __device__ __forceinline__ void run_turn(const TurnDesc* __restrict__ d, void* l
     auto exchange = [&](auto with_a, auto with_b, const TurnRound* __restrict__ rd) __attribute__((always_inline)) {
       const bool sync = ldc(&rd->sync, 0) != 0;
       auto barrier = [&]() __attribute__((always_inline)) {
-        if (sync) __syncthreads();
-        else __builtin_amdgcn_wave_barrier();
+        if (sync) {
+          __syncthreads();
+        } else {
+          __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");  // the compiler keeps the order, no instruction
+          __builtin_amdgcn_wave_barrier();
+        }
       };
       uint32_t wo[16], ro[16];
       xor_table(wo, ldc(rd->we, 0), ldc(rd->we, 1), ldc(rd->we, 2), ldc(rd->we, 3));
