@@ -118,7 +118,9 @@ struct PassDesc {
   // map(v) = v ^ ((v & lad1) >> 1) ^ ((v & lad2) >> 2)
   uint32_t lad1, lad2;
   const double* init_tab;// n + 1 entries when F_INIT_TAB
-  const DTerm* dterms;   // diagonal quadratic form (global bit positions a, b)
+  // diagonal quadratic form, named by its place in the plan's table: the host
+  // splits it there, the passes read cterms
+  const DTerm* dterms;
   int32_t ndterms;
   // The same terms split by the launch's register bits (filled by the host):
   // cterms[0, nct) have no register bit, then nht[k] terms pair register bit
