@@ -693,7 +693,8 @@ static int ensure_small(qg_plan* p, int ndesc, int nrows, int nout) {
     HIPCHK(hipMalloc(&p->d_terms, sizeof(DTerm) * 2 * mt));
     p->cap_terms = mt;
   }
-  p->max_terms = p->cap_terms;
+  // a QAOA plan's limit is its Hamiltonian's term count (qaoa_layout), which sizes its d_terms
+  if (p->kind == PK_MCCLEAN) p->max_terms = p->cap_terms;
   if (grow_part) {
     (void)hipFree(p->d_part);
     p->d_part = nullptr;
@@ -3878,9 +3879,7 @@ extern "C" int qg_qaoa_shift_sample(qg_plan* p, const qg_term* terms, int nterms
   HIPCHK(hipMalloc(&ob.p, sizeof(ShiftOp) * ops.size()));
   HIPCHK(hipMemcpy(ob.p, ops.data(), sizeof(ShiftOp) * ops.size(), hipMemcpyHostToDevice));
   const ShiftOp* d_ops = (const ShiftOp*)ob.p;
-  if (nterms)
-    HIPCHK(hipMemcpy(p->d_terms, obs.diag.data(), sizeof(DTerm) * nterms, hipMemcpyHostToDevice));
-  p->h_terms = obs.diag;
+  p->h_terms = obs.diag;  // the passes take them split by register bits (split_terms)
   DevBuf lb;
   if (phase == 1) {
     // exp(-i gamma k), k = -W .. W, per layer
