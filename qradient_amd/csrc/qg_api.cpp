@@ -650,7 +650,8 @@ static int grid_max(const qg_plan* p) {
         gm = std::max(gm, grid_for_pass(p, G, role != ROLE_FWD, false, phase));
         gm = std::max(gm, grid_for_pass(p, G, true, true, phase));
       }
-  if (!p->sweep.empty()) gm = std::max(gm, grid_for_sweep(p, p->sweep_for[3], true));
+  if (!p->sweep.empty())
+    for (int two = 0; two < 2; ++two) gm = std::max(gm, grid_for_sweep(p, p->sweep_for[3], two));
   if (p->turn)
     for (int v = 0; v < 6; ++v) gm = std::max(gm, grid_for_turn(p, p->geo[0].K, v & 1, v / 2));
   return gm;
