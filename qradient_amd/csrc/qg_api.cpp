@@ -555,6 +555,13 @@ static int kdtype(const qg_plan* p, bool two) {
   return (p->dtype == QG_C64 && (two ? p->lds64_adj : p->lds64)) ? 2 : p->dtype;
 }
 
+// The same for multi-layer passes, whose forward passes exchange FP64 values
+// unless FP32 tiles were asked for (the default of one-layer passes of circuits
+// that are not long: see mcclean_geometry and qg_sweep.hpp).
+static int sweep_dtype(const qg_plan* p, bool two) {
+  return two ? kdtype(p, true) : p->dtype == QG_C64 && p->lds64_req != 0 ? 2 : p->dtype;
+}
+
 static size_t lds_bytes_of(int dtype, int K, int threads) {  // the larger (adjoint) variant
   return (size_t)(1u << K) * (dtype == QG_C64 ? 8 : 16) + (size_t)((threads + 63) / 64) * (kMaxK + 1) * 8 +
          (dtype == QG_C64 ? (size_t)K * threads * 8 : 0);
@@ -608,7 +615,7 @@ static int grid_for_pass(const qg_plan* p, const Geo& g, bool two, bool post, in
 // per-thread sums outlive a tile).
 static int grid_for_sweep(const qg_plan* p, int K, bool two) {
   int occ = 0;
-  if (launch_sweep(kdtype(p, two), two, false, nullptr, K, 0, 1, p->n, nullptr, &occ, 0) != hipSuccess || occ < 1) occ = 1;
+  if (launch_sweep(sweep_dtype(p, two), two, false, nullptr, K, 0, 1, p->n, nullptr, &occ, 0) != hipSuccess || occ < 1) occ = 1;
   const uint64_t ntiles = 1ull << (p->n - K);
   const uint64_t target = (uint64_t)p->ctx->num_cu * occ * kWgOversub;
   uint64_t grid = 1;
@@ -1076,7 +1083,7 @@ static hipError_t launch_one(qg_plan* p, const Launch& l) {
   if (l.kind == 1) return launch_generic_obs(p);
   if (l.kind != 0) return hipSuccess;
   if (l.sweep)
-    return launch_sweep(kdtype(p, l.two), l.two, l.post, p->d_sweep + l.desc, l.K, l.grid, l.batch, p->n,
+    return launch_sweep(sweep_dtype(p, l.two), l.two, l.post, p->d_sweep + l.desc, l.K, l.grid, l.batch, p->n,
                         p->ctx->stream, nullptr, l.tab);
   if (l.turn)
     return launch_turn(p->dtype == QG_C64 ? 1 : 0, l.two, l.phase, p->d_turn + l.desc, l.K, l.grid, l.batch, p->n,
@@ -1162,7 +1169,7 @@ static int run_launches(qg_plan* p, int ndesc, int first_desc = 0) {
   if (p->use_graph && !p->profile) {
     std::vector<int64_t> sig;
     sig.reserve(p->launches.size() * 12 + 8);
-    sig.push_back(kdtype(p, false) * 4 + kdtype(p, true));
+    sig.push_back((kdtype(p, false) * 4 + kdtype(p, true)) * 4 + sweep_dtype(p, false));
     sig.push_back(p->n);
     sig.push_back((int64_t)(intptr_t)p->d_desc);
     sig.push_back((int64_t)(intptr_t)p->d_sweep);
@@ -1472,10 +1479,12 @@ static int mcclean_geometry(qg_plan* p) {
     }
   }
   p->S = (size_t)(1ull << n) * (p->dtype == QG_C64 ? 8 : 16);
-  // complex64 states are rounded at every LDS transpose of a pass with FP32
-  // tiles; beyond about 200 passes these roundings would take the gradient
-  // past a 1e-6 relative error, so long circuits use FP64 tiles (rounding
-  // once per pass, at the store)
+  // complex64 states are rounded at every LDS transpose of a one-layer pass
+  // with FP32 tiles; beyond about 200 such passes these roundings would take
+  // the gradient past a 1e-6 relative error, so long circuits use FP64 tiles
+  // (rounding once per pass, at the store).  Multi-layer forward passes round
+  // only at the store by default (24 qubits, 66 layers, just below the line:
+  // 4.7e-7; 70 layers: 4.9e-7)
   p->lds64 = p->dtype == QG_C64 && n >= 4 && (p->lds64_req >= 1 || (p->lds64_req < 0 && P * L > 200));
   p->lds64_adj = p->lds64 && (p->lds64_req == 1 || (p->lds64_req < 0 && kLds64Adjoint));
   const size_t hist_bytes = (size_t)(P * L + 4) * p->S;
@@ -2053,7 +2062,7 @@ static int sweep_schedule(qg_plan* p, int nb, const int32_t* axes, const double*
       // the exchange into a round, as slot offsets: of the registers it is
       // written from, of those it is read into, of the tile bit above
       auto exchange = [&](SweepRound& o) {
-        const int sh = kdtype(p, two) == 1 ? 3 : 4;
+        const int dt = sweep_dtype(p, two), sh = dt == 1 || sweep_halves(dt, two) ? 3 : 4;
         auto slot = [&](uint32_t x) { return (x ^ ((x >> 4) & (sh == 3 ? 31u : 15u))) << sh; };
         auto map = [&](uint32_t x) { return x ^ ((x & o.m1) >> 1) ^ ((x & o.m2) >> 2); };
         for (int kk = 0; kk < 4; ++kk) {

@@ -142,6 +142,9 @@ struct PassDesc {
 constexpr int kMaxRounds = 14;   // rounds of a multi-layer pass
 constexpr int kSweepMinK = 10;   // local bits of one: whole waves of 16 amplitudes per lane
 constexpr int kSweepMaxK = 13;
+// Whether a multi-layer pass exchanges FP64 values half an amplitude at a time,
+// through slots of 8 bytes (dtype 2: complex64 states, FP64 tiles).
+constexpr bool sweep_halves(int dtype, bool two) { return dtype == 2 && !two; }
 
 // One round: four local bits in registers, a rotation on each.
 struct SweepRound {

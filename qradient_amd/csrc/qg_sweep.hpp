@@ -29,13 +29,25 @@
 // (checkpoint mode).  The adjoint of the circuit's last pass forms lambda =
 // D psi and E itself where the observable is diagonal (OBS).
 //
+// A complex64 forward pass (F32L64) keeps tiles of 8 bytes an amplitude: it moves
+// the FP64 real parts through them and then the imaginary parts, so psi is
+// rounded where it is stored and nowhere else; the adjoint rounds both states to
+// FP32 at every exchange, as a pass of one layer does.  A pass of several layers
+// has up to 14 exchanges, which in FP32 make a forward circuit less accurate than
+// one layer at a time: geometric mean of the gradient's error over seeds, one
+// layer at a time | FP32 forward exchanges | now: 18 qubits, 12 layers 1.78e-7 |
+// 1.94e-7 | 1.20e-7; 24 qubits, 40 layers 6.14e-7 | 6.26e-7 | 3.87e-7; 25 qubits,
+// 10 layers 1.83e-8 | 2.29e-8 | 1.15e-8.  It costs 1 to 3% of a gradient run (16
+// qubits 553 -> 557 us, 24 qubits, 40 layers 10.65 -> 10.90 ms).  The adjoint's psi
+// in halves too costs another 3 to 5% and leaves these errors as they are (24
+// qubits, with FP32 forward exchanges: 6.26e-7 either way).
+//
 // Bound: the vector ALU.  A round costs 4 x 48 FMAs per thread and state and
-// an exchange of about 130 instructions (with FP32 tiles half of them
-// conversions); the adjoint adds 4 x 32 FMAs of reductions.  The four sums of
-// a round are reduced across the wave together: two lane swaps fold four
-// values into one register, so they cost 21 instructions instead of 88.
-// Measured at 24 qubits, complex64, per layer: forward 145 -> 86 us,
-// adjoint 288 -> 200 us.
+// an exchange of about 130 instructions (in FP32 half of them conversions); the
+// adjoint adds 4 x 32 FMAs of reductions.  The four sums of a round are reduced
+// across the wave together: two lane swaps fold four values into one register,
+// so they cost 21 instructions instead of 88.  Measured at 24 qubits, complex64,
+// per layer: forward 145 -> 86 us (92 with FP64 exchanges), adjoint 288 -> 200 us.
 #pragma once
 #include "qg_pass.hpp"
 
@@ -88,10 +100,18 @@ __device__ __forceinline__ int wave_sum4_slot(uint32_t tid) {  // the value whos
   return (int)(((r & 1u) << 1) | (r >> 1));
 }
 
+// One FP64 value by absolute LDS address.
+__device__ __forceinline__ void lds_st_d(uint32_t addr, double v) {
+  *(__attribute__((address_space(3))) double*)(uintptr_t)addr = v;
+}
+__device__ __forceinline__ double lds_ld_d(uint32_t addr) {
+  return *(const __attribute__((address_space(3))) double*)(uintptr_t)addr;
+}
+
 // LDS bytes of a pass: the tile, the per-wave sums and the initial-state table.
 __host__ __device__ inline size_t sweep_lds_bytes(int dtype, int K, bool two, int tab_bytes) {
-  return (size_t)(1u << K) * (dtype == 1 ? 8 : 16) + (two ? (size_t)(1u << (K - 4)) / 64 * kMaxRounds * 4 * 8 : 0) +
-         (size_t)tab_bytes;
+  return (size_t)(1u << K) * (dtype == 1 || sweep_halves(dtype, two) ? 8 : 16) +
+         (two ? (size_t)(1u << (K - 4)) / 64 * kMaxRounds * 4 * 8 : 0) + (size_t)tab_bytes;
 }
 
 template <class S, bool TWO, bool BIG, bool OBS>
@@ -101,15 +121,18 @@ __device__ __forceinline__ void run_sweep(const SweepDesc* __restrict__ d, void*
   typedef typename Store<S>::G G;   // HBM element type
   typedef typename Store<S>::L LT;  // LDS tile element type
   constexpr int GSH = sizeof(G) == 4 ? 3 : 4;
-  constexpr int SH = sizeof(LT) == 4 ? 3 : 4;
   constexpr bool PF = !TWO;  // the next tile's loads in flight while this one is worked on
+  // the exchange moves FP64 halves of an amplitude (see above)
+  constexpr bool HALVES = sweep_halves(kernel_dtype<S>(), TWO);
+  typedef typename std::conditional<HALVES, float, LT>::type SL;  // whose complex values fill an LDS slot
+  constexpr int SH = sizeof(SL) == 4 ? 3 : 4;
   warm_lines<(int)sizeof(SweepDesc)>(d);
   const int n = d->n, K = d->K, t = d->t, c = d->c, p = d->p;
   const uint32_t flags = d->flags;
   const uint32_t ntiles = 1u << (n - K);
   const uint32_t nthr = blockDim.x;
   const int nr = d->nr;
-  double* wacc = reinterpret_cast<double*>(reinterpret_cast<char*>(lds) + (sizeof(LT) * 2u << K));
+  double* wacc = reinterpret_cast<double*>(reinterpret_cast<char*>(lds) + (1u << (K + SH)));
   double* itab = wacc + (TWO ? (nthr / 64) * kMaxRounds * 4 : 0);
   if constexpr (TWO) {
     for (uint32_t i = tid_in; i < (nthr / 64) * kMaxRounds * 4; i += nthr) wacc[i] = 0.0;
@@ -248,11 +271,24 @@ __device__ __forceinline__ void run_sweep(const SweepDesc* __restrict__ d, void*
       uint32_t wo[16], ro[16];
       xor_table(wo, ldc(rd->we, 0), ldc(rd->we, 1), ldc(rd->we, 2), ldc(rd->we, 3));
       xor_table(ro, ldc(rd->re, 0), ldc(rd->re, 1), ldc(rd->re, 2), ldc(rd->re, 3));
-      uint32_t bw = lds_addr(lds) + (swz<LT>(lidx<R>(tid, 0, lo_from)) << SH);
+      uint32_t bw = lds_addr(lds) + (swz<SL>(lidx<R>(tid, 0, lo_from)) << SH);
       uint32_t br = lds_addr(lds) +
-                    ((swz<LT>(ladder_of(lidx<R>(tid, 0, ldc(&rd->lo, 0)), m1, m2)) << SH) ^ (above ? ldc(&rd->off, 0) : 0u));
+                    ((swz<SL>(ladder_of(lidx<R>(tid, 0, ldc(&rd->lo, 0)), m1, m2)) << SH) ^ (above ? ldc(&rd->off, 0) : 0u));
       asm volatile("" : "+v"(bw), "+v"(br));  // opaque (see lds_transpose)
-      if constexpr (decltype(with_a)::value) {
+      if constexpr (HALVES) {
+        // real parts, then imaginary parts, unrounded, through the same slots
+        auto half = [&](double Cd::*part) __attribute__((always_inline)) {
+#pragma unroll
+          for (int a = 0; a < A; ++a) lds_st_d(bw ^ wo[a], xa[a].*part);
+          barrier();
+#pragma unroll
+          for (int a = 0; a < A; ++a) xa[a].*part = lds_ld_d(br ^ ro[a]);
+        };
+        half(&Cd::re);
+        barrier();
+        asm volatile("" : "+v"(bw), "+v"(br));  // opaque again: shared addresses would all stay live
+        half(&Cd::im);
+      } else if constexpr (decltype(with_a)::value) {
 #pragma unroll
         for (int a = 0; a < A; ++a) Stor<LT>::lds_st_a(bw ^ wo[a], xa[a]);
         barrier();
@@ -366,11 +402,12 @@ __device__ __forceinline__ void run_sweep(const SweepDesc* __restrict__ d, void*
 }
 
 // blockIdx.y selects one of gridDim.y consecutive descriptors (batched
-// circuits).  Three waves per SIMD where the LDS tiles allow it (FP32 tiles):
+// circuits).  Three waves per SIMD where the LDS tiles allow it (8-byte slots):
 // the complex64 adjoint at 24 qubits took 262 us per pass with 177 registers
 // (two waves) and takes 222 us with at most 168.
 template <class S, bool TWO, bool BIG, bool OBS>
-__global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(kernel_dtype<S>() == 1 ? 3 : 2)))
+__global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(
+    kernel_dtype<S>() == 1 || sweep_halves(kernel_dtype<S>(), TWO) ? 3 : 2)))
 void k_sweep(const SweepDesc* __restrict__ d) {
   extern __shared__ __align__(16) char lds_dyn[];
   run_sweep<S, TWO, BIG, OBS>(d + blockIdx.y, lds_dyn, threadIdx.x, blockIdx.x, gridDim.x);
