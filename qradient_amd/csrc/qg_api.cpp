@@ -492,7 +492,7 @@ struct qg_plan {
   // multi-layer passes of a McClean plan (qg_sweep.hpp)
   std::vector<PlanPass> sweep;
   int sweep_rounds = 0;     // rounds of all of them
-  int sweep_for[5] = {0, 0, 0, 0, 0};  // n, L, entangler, local bits, contiguous bits it was planned for
+  int sweep_for[6] = {0, 0, 0, 0, 0, 0};  // n, L, entangler, local bits, contiguous bits, steps it was planned for
   SweepDesc* d_sweep = nullptr;
   SweepDesc* h_sweep = nullptr;
   int sweep_cap = 0;
@@ -1526,9 +1526,10 @@ static int mcclean_geometry(qg_plan* p) {
 // waves or of 1024 threads.
 //
 // The tile (K local bits, c of them the low bits that make the runs of
-// contiguous amplitudes) and the steps (layers) that a pass may run on it,
-// unless the tile was chosen by the caller.  Device us of a gradient run, 20
-// layers, complex64 | complex128:
+// contiguous amplitudes), unless it was chosen by the caller, and the steps
+// (layers) that a pass may run on it: functions of the shape and the tile
+// options, so that a plan does not depend on what it held before.  Device us of
+// a gradient run, 20 layers, complex64 | complex128:
 //  - below 20 qubits a pass takes as long as its chain of rounds, and tiles
 //    of 2^12 are fewer than the CUs: K = 11, c = 2, 4 steps (16 qubits 502 |
 //    479, 19 qubits 684 | 694) against K = 12, c = 3 (523 | 539, 756 | 799);
@@ -1544,23 +1545,24 @@ constexpr size_t kFoldObs = (size_t)32 << 20;      // bytes (see sweep_schedule)
 constexpr size_t kCachedState = (size_t)64 << 20;  // bytes; two of them fit the 256 MiB cache
 
 static void plan_sweeps(qg_plan* p) {
-  int K = p->kmax, c = p->cmin, steps = 4;
+  int K = p->kmax, c = p->cmin;
   if (p->kmax_auto) {
     K = p->n < 20 ? 11 : 12;
     if (p->S <= kCachedState) c = 2;
-    if (p->n >= 20 && c == 2) steps = 6;
   }
-  const int key[5] = {p->n, p->L, p->ent, K, c};
+  const int steps = p->n >= 20 && p->S <= kCachedState && K == 12 && c == 2 ? 6 : 4;
+  const int key[6] = {p->n, p->L, p->ent, K, c, steps};
   if (p->n <= kFusedMaxN || K < kSweepMinK || K > kSweepMaxK || c < 1 || K - c < 4) {
     p->sweep.clear();
     p->sweep_rounds = 0;
     return;
   }
-  if (!p->sweep.empty() && std::equal(key, key + 5, p->sweep_for)) return;
-  p->sweep = SweepPlanner(p->n, p->L, p->ent == QG_ENT_CZ, K, c).plan(steps);
-  p->sweep_rounds = 0;
-  for (const PlanPass& s : p->sweep) p->sweep_rounds += (int)s.rounds.size();
-  std::copy(key, key + 5, p->sweep_for);
+  if (p->sweep.empty() || !std::equal(key, key + 6, p->sweep_for)) {
+    p->sweep = SweepPlanner(p->n, p->L, p->ent == QG_ENT_CZ, K, c).plan(steps);
+    p->sweep_rounds = 0;
+    for (const PlanPass& s : p->sweep) p->sweep_rounds += (int)s.rounds.size();
+    std::copy(key, key + 6, p->sweep_for);
+  }
   // the layout holds one state per single-layer pass
   if (p->sweep.size() > p->geo.size() * (size_t)p->L) p->sweep.clear();
 }
