@@ -1575,9 +1575,13 @@ static uint32_t wave_bits(int K, int lo) {
   return m;
 }
 
-// Room for the sweep descriptors of `circuits` circuits at a time.
+// Room for the sweep descriptors of `circuits` circuits at a time.  A plan that
+// can be re-laid out takes the bound of plan_sweeps instead of its own number,
+// which is larger for some smaller shapes (40 layers, complex128: 22 qubits 24
+// passes, 19 qubits 29): so a smaller shape never needs more.
 static int ensure_sweeps(qg_plan* p, int circuits) {
-  const int need = 2 * (int)p->sweep.size() * circuits;
+  const size_t passes = p->mc_batch || p->sweep.empty() ? p->sweep.size() : p->geo.size() * (size_t)p->L;
+  const int need = 2 * (int)passes * circuits;
   if (need <= p->sweep_cap) return QG_OK;
   HIPCHK(hipStreamSynchronize(p->ctx->stream));
   drop_graph(p);
@@ -1595,9 +1599,12 @@ static int ensure_sweeps(qg_plan* p, int circuits) {
 
 // Partial rows of one circuit: of the single-layer passes (shifted circuits
 // and plans without multi-layer passes), or of the multi-layer ones and the
-// observable's pass.
+// observable's pass (plans that can be re-laid out: their bound for the shape,
+// as in ensure_sweeps).
 static int mcclean_rows(const qg_plan* p) {
-  return std::max(((int)p->geo.size() * p->L + 1) * (kMaxK + 1), 4 * p->sweep_rounds + kMaxK + 1);
+  int rounds = p->sweep_rounds;
+  if (!p->mc_batch && !p->sweep.empty()) rounds = std::max(rounds, sweep_round_bound(p->n, p->L));
+  return std::max(((int)p->geo.size() * p->L + 1) * (kMaxK + 1), 4 * rounds + kMaxK + 1);
 }
 
 // mcclean_geometry plus the partial-row stride and the small device tables.

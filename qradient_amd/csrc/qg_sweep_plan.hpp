@@ -25,6 +25,11 @@ struct PlanPass {
   std::vector<PlanRound> rounds;
 };
 
+// A bound on the rounds of all passes of a circuit on its default tile (a round
+// holds four rotations; at most 1.52 slots go to each, at 29 qubits).  It grows
+// with n and L, while a larger shape's own rounds can be fewer than a smaller's.
+inline int sweep_round_bound(int n, int L) { return (25 * n * L / 16 + 3) / 4; }
+
 // The circuit as three events per bit and layer: the bond of the first group,
 // the bond of the second (passed over where the end bits have none), the
 // rotation.  Bond k belongs to qubits n-2-k and n-1-k; the odd bonds act first
