@@ -9,11 +9,13 @@
 - QAOA batch shape (``tune_qaoa``): tile shape, circuits resident at once
   (``chunk``) and workgroups per CU of a batched launch (``wg_per_cu``).
 
-The tuner times each candidate on the device and caches the fastest per
-workload key in a JSON file (``$QRADIENT_AMD_TUNE_CACHE``, default
-``~/.cache/qradient_amd/tune.json``).  Lookups fall back to
-``tune_defaults.json`` beside this file: shapes measured on MI355X and
-committed with the package, so a fresh machine starts from them.
+The tuner times the untuned plan and each candidate on the device and caches
+the fastest per workload key in a JSON file (``$QRADIENT_AMD_TUNE_CACHE``,
+default ``~/.cache/qradient_amd/tune.json``).  The file names the generation of
+the kernels its shapes were timed on (``KERNELS``); entries of another
+generation are not used.  Lookups fall back to ``tune_defaults.json`` beside
+this file: shapes measured on MI355X and committed with the package, so a fresh
+machine starts from them.
 """
 import ctypes
 import json
@@ -26,6 +28,10 @@ from . import _native
 
 DEFAULTS_PATH = os.path.join(os.path.dirname(os.path.abspath(__file__)), 'tune_defaults.json')
 
+# Raised when the passes change so much that shapes timed before say nothing
+# (2: several layers per McClean pass, turning QAOA passes).
+KERNELS = 2
+
 DEFAULT = {'kmax': 13, 'cmin': 3, 'r_fwd': 4, 'r_rev': 4}
 
 
@@ -34,17 +40,26 @@ def _passes(n, kmax, cmin):
 
 
 def default_shape(n, dtype):
-    """The library's untuned shape: the fewest passes per layer 13 local bits
-    allow, with the smallest tile (>= 11 bits for complex64, 12 for
-    complex128) that keeps that count; 13 bits for complex64 states of 4 GiB
-    and more (n >= 29)."""
-    if dtype == 'complex64' and n >= 29:
-        return dict(DEFAULT, kmax=13)
+    """The tile of the library's untuned plan: past 13 qubits that of its
+    multi-layer passes (11 local bits below 20 qubits, else 12; 2 contiguous
+    bits while the state is at most 64 MiB, else 3).  Smaller circuits run whole
+    in one workgroup and have no tile; theirs is that of the single-layer
+    passes they take with an initial state."""
+    if n > 13:
+        cached_state = (16 if dtype == 'complex128' else 8) << n <= 64 << 20
+        return dict(DEFAULT, kmax=11 if n < 20 else 12, cmin=2 if cached_state else 3)
     best = _passes(n, 13, 3)
     for kmax in range(11 if dtype == 'complex64' else 12, 13):
         if _passes(n, kmax, 3) == best:
             return dict(DEFAULT, kmax=kmax)
     return dict(DEFAULT)
+
+
+def untuned_shape(n, dtype):
+    """The entry of a workload that runs fastest as the library lays it out.  A
+    plan set to its tile is not quite the same: a tile chosen by the caller is
+    that of the single-layer passes too, and so of the memory mode."""
+    return dict(default_shape(n, dtype), untuned=True)
 
 
 def cache_path():
@@ -61,7 +76,8 @@ def _read(path):
 
 
 def _load_cache():
-    return _read(cache_path())
+    c = _read(cache_path())
+    return c if c.get('kernels') == KERNELS else {}
 
 
 def _save_cache(c):
@@ -88,6 +104,7 @@ def lookup(k):
 
 def _store(k, v):
     c = _load_cache()
+    c['kernels'] = KERNELS
     c[k] = v
     _save_cache(c)
 
@@ -108,12 +125,18 @@ def candidates(dtype):
 
 
 def apply(plan, shape):
+    """Sets a tile of ``candidates`` or of the cache; an ``untuned`` one leaves a
+    fresh plan as it is."""
+    if shape.get('untuned'):
+        return
     _native.call('qg_plan_tune', plan, int(shape['kmax']), int(shape['cmin']), int(shape['r_fwd']),
                  int(shape['r_rev']))
 
 
 def tune_mcclean(n, L, dtype='complex64', entangler='cnot', shapes=None, reps=2, seed=0, device=0, store=True):
-    """Time every candidate shape on a seeded circuit; return (best, [(shape, ms)])."""
+    """Time the untuned plan and every candidate shape on a seeded circuit;
+    return (best, [(shape, ms)]).  A candidate is taken only if it is more than
+    2% faster than the untuned plan."""
     ctx = _native.Context.default(device)
     rs = np.random.RandomState(seed)
     axes = np.ascontiguousarray((3 * rs.rand(L, n)).astype(np.int32))
@@ -121,7 +144,7 @@ def tune_mcclean(n, L, dtype='complex64', entangler='cnot', shapes=None, reps=2,
     terms = [(_native.TERM_ZZ, i, i + 1, float(w)) for i, w in enumerate(rs.standard_normal(n - 1))]
     arr, k = _native.terms_array(terms)
     results = []
-    for shape in (shapes or candidates(dtype)):
+    for shape in [untuned_shape(n, dtype)] + list(shapes or candidates(dtype)):
         h = ctypes.c_void_p()
         _native.call('qg_mcclean_plan', ctx.handle, n, L, _native.DTYPES[dtype], _native.ENTANGLERS[entangler], 0,
                      ctypes.byref(h))
@@ -142,9 +165,9 @@ def tune_mcclean(n, L, dtype='complex64', entangler='cnot', shapes=None, reps=2,
             results.append((shape, best))
         finally:
             _native.load().qg_plan_destroy(h)
-    if not results:
-        return default_shape(n, dtype), results
-    best = min(results, key=lambda r: r[1])[0]
+    best, ms = min(results, key=lambda r: r[1])
+    if ms > 0.98 * results[0][1]:
+        best = results[0][0]
     if store:
         _store(key('mcclean', n, L, dtype, entangler), best)
     return best, results
