@@ -228,6 +228,12 @@ int qg_qaoa_expec_val_ini(qg_plan* plan, int B, const qg_term* terms, const int3
 int qg_qaoa_shift_sample(qg_plan* plan, const qg_term* terms, int nterms, const double* betas, const double* gammas,
                          const double* ini_state, const qg_term* mterms, int nm, double* expec, int shots,
                          const double* u, int32_t* idx);
+/* The shifted circuits [first, first + count) of that order only (count < 0:
+ * the rest): u and idx hold count * shots entries.  With many shots the draws
+ * of all circuits need not be in memory at once.  expec may be NULL. */
+int qg_qaoa_shift_sample_part(qg_plan* plan, const qg_term* terms, int nterms, const double* betas,
+                              const double* gammas, const double* ini_state, const qg_term* mterms, int nm,
+                              double* expec, int64_t first, int64_t count, int shots, const double* u, int32_t* idx);
 
 /* Lays a McClean plan out again for another circuit shape: n qubits, L
  * layers, ckpt_every as for qg_mcclean_plan; dtype, entangler, context and

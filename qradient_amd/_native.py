@@ -75,6 +75,8 @@ SIGNATURES = {
     'qg_qaoa_grad_run_ini': [_vp, _i, _tp, _ip, _dp, _dp, _dp, _dp, _dp],
     'qg_qaoa_expec_val_ini': [_vp, _i, _tp, _ip, _dp, _dp, _dp, _dp],
     'qg_qaoa_shift_sample': [_vp, _tp, _i, _dp, _dp, _dp, _tp, _i, _dp, _i, _dp, _ip],
+    'qg_qaoa_shift_sample_part': [_vp, _tp, _i, _dp, _dp, _dp, _tp, _i, _dp, ctypes.c_int64, ctypes.c_int64, _i, _dp,
+                                  _ip],
     'qg_plan_reshape': [_vp, _i, _i, _i],
     'qg_plan_workspace_size': [_vp, ctypes.POINTER(ctypes.c_size_t)],
     'qg_plan_set_workspace': [_vp, _vp, ctypes.c_size_t],

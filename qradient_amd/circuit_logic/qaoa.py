@@ -15,6 +15,10 @@ from .. import _native
 from ..physical_components import Gates
 from .base import ParametrizedCircuit, draw_uniforms, sample_projectors
 
+# Shots of shifted circuits that are in memory at once (20 bytes each on the
+# host): with more, the circuits are drawn and run in groups.
+SHOT_GROUP = 1 << 24
+
 
 class Qaoa(ParametrizedCircuit):
     def __init__(self, qubit_number, observable, layer_number, **kwargs):
@@ -105,19 +109,25 @@ class Qaoa(ParametrizedCircuit):
         # draws in the reference's order: E's shots, then per layer each
         # component's two circuits and each qubit's
         u_E = None if exact_expec_val else draw_uniforms(len(terms), shots)
-        u = draw_uniforms(L * 2 * (k + n), shots)
-        if shots == 0:
-            u = np.zeros((u.shape[0], 1))  # no shots: E alone, the estimates are nan
         m_arr, m = _native.terms_array(terms)
         expec = np.empty(m + 1)
-        idx = np.empty(u.shape, dtype=np.int32)
-        _native.call('qg_qaoa_shift_sample', self._get_plan(), arr, k, _native.dptr(betas), _native.dptr(gammas), ini,
-                     m_arr, m, _native.dptr(expec), u.shape[1], _native.dptr(u), _native.iptr(idx))
+        total = L * 2 * (k + n)
+        o = np.empty(total)
+        group = max(1, SHOT_GROUP // max(1, shots))
+        for first in range(0, total, group):
+            u = draw_uniforms(min(group, total - first), shots)
+            if shots == 0:
+                u = np.zeros((u.shape[0], 1))  # no shots: E alone, the estimates are nan
+            idx = np.empty(u.shape, dtype=np.int32)
+            _native.call('qg_qaoa_shift_sample_part', self._get_plan(), arr, k, _native.dptr(betas),
+                         _native.dptr(gammas), ini, m_arr, m, None if first else _native.dptr(expec), first,
+                         u.shape[0], u.shape[1], _native.dptr(u), _native.iptr(idx))
+            o[first:first + u.shape[0]] = C[idx[:, :shots]].mean(axis=1)
         if exact_expec_val:
             E = np.float64((w * expec[:m]).sum())
         else:
             E = sample_projectors(.5 * (expec[m] + expec[:m]), w, shots, uniforms=u_E)
-        o = C[idx[:, :shots]].mean(axis=1).reshape(L, k + n, 2)
+        o = o.reshape(L, k + n, 2)
         diff = o[:, :, 0] - o[:, :, 1]
         grad = np.empty((L, 2), dtype='double')
         for i in range(L):

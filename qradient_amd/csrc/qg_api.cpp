@@ -3846,12 +3846,14 @@ static int qaoa_run(qg_plan* p, int B, const qg_term* terms, const int32_t* term
 // the classical Hamiltonian) and RX(+-pi/2) on qubit q after the mixer.  The
 // unshifted circuit keeps both of a layer's states; the shifted copies of one
 // state run the rest of the circuit together, every pass one launch with one
-// descriptor (push_forward), and are sampled together.
-extern "C" int qg_qaoa_shift_sample(qg_plan* p, const qg_term* terms, int nterms, const double* betas,
-                                    const double* gammas, const double* ini_state, const qg_term* mterms, int nm,
-                                    double* expec, int shots, const double* u, int32_t* idx) {
+// descriptor (push_forward), and are sampled together.  Only the shifted
+// circuits [first, first + count) are run (count < 0: all from first on).
+extern "C" int qg_qaoa_shift_sample_part(qg_plan* p, const qg_term* terms, int nterms, const double* betas,
+                                         const double* gammas, const double* ini_state, const qg_term* mterms, int nm,
+                                         double* expec, int64_t first, int64_t count, int shots, const double* u,
+                                         int32_t* idx) {
   if (!p || p->kind != PK_QAOA) return fail(QG_ERR_INVALID, "not a QAOA plan");
-  if (!betas || !gammas || !expec || !u || !idx || nterms < 0 || (nterms > 0 && !terms))
+  if (!betas || !gammas || !u || !idx || nterms < 0 || (nterms > 0 && !terms))
     return fail(QG_ERR_INVALID, "NULL argument");
   if (shots < 1) return fail(QG_ERR_INVALID, "shots must be >= 1");
   const int n = p->n, L = p->L, P = (int)p->geo.size();
@@ -3874,13 +3876,17 @@ extern "C" int qg_qaoa_shift_sample(qg_plan* p, const qg_term* terms, int nterms
   // states: the history (after each phase and each mixer), the initial state
   // when given, and the copies of a batch
   const int per_layer = 2 * (nterms + n);
+  const int64_t total = (int64_t)L * per_layer;
+  if (count < 0) count = total - first;
+  if (first < 0 || first > total || count > total - first)
+    return fail(QG_ERR_INVALID, "the circuit has " + std::to_string(total) + " shifted circuits");
   const int most = std::min(shift_batch(n), 2 * std::max(nterms, n));
   const size_t S = p->S;
   CHK(ensure_shift(p, (size_t)(2 * L + 1 + most) * S));
   auto hist = [&](int k) { return (void*)(p->d_shift + (size_t)k * S); };
   char* copies = p->d_shift + (size_t)(2 * L + 1) * S;
   SampleBufs b;
-  CHK(sample_setup(n, nullptr, (int64_t)L * per_layer * shots, u, most, b));
+  CHK(sample_setup(n, nullptr, count * shots, u, most, b));
   // the shift operations of a layer (the same for every layer)
   std::vector<ShiftOp> ops((size_t)per_layer);
   for (int j = 0; j < nterms; ++j)
@@ -3973,20 +3979,31 @@ extern "C" int qg_qaoa_shift_sample(qg_plan* p, const qg_term* terms, int nterms
   }
   for (int i = 0; i < L; ++i)
     for (int kind = 0; kind < 2; ++kind) {
-      const int first = kind == 0 ? 0 : 2 * nterms, all = kind == 0 ? 2 * nterms : 2 * n;
-      for (int s = 0; s < all; s += most) {
-        const int count = std::min(most, all - s);
-        HIPCHK(simple_shift_copies(p->dtype, hist(2 * i + kind), copies, n, d_ops + first + s, count, c->stream));
-        if (kind == 0) CHK(emit(copies, copies, count, i, false, true));
-        for (int j = i + 1; j < L; ++j) CHK(emit(copies, copies, count, j, true, true));
-        const size_t at = ((size_t)i * per_layer + first + s) * shots;
-        HIPCHK(simple_sample_basis(p->dtype, copies, n, nullptr, b.u + at, shots, b.idx + at, b.mass, count,
-                                   c->stream));
+      // circuits [s0, s1) of this state's, of which op0 is the first's operation
+      const int op0 = kind == 0 ? 0 : 2 * nterms, all = kind == 0 ? 2 * nterms : 2 * n;
+      const int64_t g0 = (int64_t)i * per_layer + op0;
+      const int s0 = (int)std::min<int64_t>(all, std::max<int64_t>(0, first - g0));
+      const int s1 = (int)std::max<int64_t>(0, std::min<int64_t>(all, first + count - g0));
+      for (int s = s0; s < s1; s += most) {
+        const int m = std::min(most, s1 - s);
+        HIPCHK(simple_shift_copies(p->dtype, hist(2 * i + kind), copies, n, d_ops + op0 + s, m, c->stream));
+        if (kind == 0) CHK(emit(copies, copies, m, i, false, true));
+        for (int j = i + 1; j < L; ++j) CHK(emit(copies, copies, m, j, true, true));
+        const size_t at = (size_t)(g0 + s - first) * shots;
+        HIPCHK(simple_sample_basis(p->dtype, copies, n, nullptr, b.u + at, shots, b.idx + at, b.mass, m, c->stream));
       }
     }
-  CHK(term_expec(c, p->dtype, hist(2 * L - 1), n, mterms, nm, expec));
-  HIPCHK(hipMemcpy(idx, b.idx, (size_t)L * per_layer * shots * 4, hipMemcpyDeviceToHost));
+  if (expec) CHK(term_expec(c, p->dtype, hist(2 * L - 1), n, mterms, nm, expec));
+  else HIPCHK(hipStreamSynchronize(c->stream));
+  HIPCHK(hipMemcpy(idx, b.idx, (size_t)count * shots * 4, hipMemcpyDeviceToHost));
   return QG_OK;
+}
+
+extern "C" int qg_qaoa_shift_sample(qg_plan* p, const qg_term* terms, int nterms, const double* betas,
+                                    const double* gammas, const double* ini_state, const qg_term* mterms, int nm,
+                                    double* expec, int shots, const double* u, int32_t* idx) {
+  if (!expec) return fail(QG_ERR_INVALID, "NULL argument");
+  return qg_qaoa_shift_sample_part(p, terms, nterms, betas, gammas, ini_state, mterms, nm, expec, 0, -1, shots, u, idx);
 }
 
 extern "C" int qg_qaoa_grad_run(qg_plan* p, int B, const qg_term* terms, const int32_t* term_off,
