@@ -2882,6 +2882,21 @@ static int ensure_shift(qg_plan* p, size_t bytes) {
   return QG_OK;
 }
 
+// Frees shifted circuits' scratch past this size at the end of a call: the
+// batches of copies stay (at most 128 MiB of two buffers), a large circuit's
+// stored states do not, so that its gradient runs find the memory they had.
+constexpr size_t kShiftKeep = (size_t)512 << 20;
+struct ShiftTrim {
+  qg_plan* p;
+  ~ShiftTrim() {
+    if (p->shift_cap <= kShiftKeep) return;
+    (void)hipStreamSynchronize(p->ctx->stream);
+    (void)hipFree(p->d_shift);
+    p->d_shift = nullptr;
+    p->shift_cap = 0;
+  }
+};
+
 // Shifted circuits run this many amplitudes at a time (all circuits of a
 // launch together): enough tiles to fill the device, and states that the
 // memory-side cache holds.  From 22 qubits on they run one by one, as one
@@ -3882,6 +3897,7 @@ extern "C" int qg_qaoa_shift_sample_part(qg_plan* p, const qg_term* terms, int n
     return fail(QG_ERR_INVALID, "the circuit has " + std::to_string(total) + " shifted circuits");
   const int most = std::min(shift_batch(n), 2 * std::max(nterms, n));
   const size_t S = p->S;
+  ShiftTrim trim{p};
   CHK(ensure_shift(p, (size_t)(2 * L + 1 + most) * S));
   auto hist = [&](int k) { return (void*)(p->d_shift + (size_t)k * S); };
   char* copies = p->d_shift + (size_t)(2 * L + 1) * S;
