@@ -905,35 +905,31 @@ static void desc_geo(PassDesc& d, int n, const Geo& g) {
   }
 }
 
-// U = cos(phi) I - i sin(phi) P with phi = sign * angle / 2.  phi is reduced
-// modulo pi to [-pi/2, pi/2]; each reduction multiplies U by -1, a global sign
-// the kernels drop (returns true when it did, so the caller can track the
-// parity for the returned state vector).
-static bool gate_flips(double angle, double sign) {
-  const double phi0 = sign * 0.5 * angle;
-  const double phi = std::remainder(phi0, M_PI);
-  return std::fabs(std::remainder((phi0 - phi) / M_PI, 2.0)) > 0.5;
-}
-
-static bool set_gate(PassDesc& d, int lb, int axis, double angle, double sign) {
-  const double phi0 = sign * 0.5 * angle;
-  const double phi = std::remainder(phi0, M_PI);
-  const bool flipped = gate_flips(angle, sign);
-  const double c = std::cos(phi), s = std::sin(phi);
-  d.gtype[lb] = axis == 0 ? G_X : axis == 1 ? G_Y : G_Z;
-  d.ga[lb] = s / (1.0 + c);
-  d.gb[lb] = s;
-  return flipped;
-}
-
-// The (ga, gb) pair set_gate stores for a gate of this angle and sign.
+// U = cos(phi) I - i sin(phi) P with phi = sign * angle / 2, as shears by
+// a = tan(phi / 2) and b = sin(phi).  |phi| is kept to at most pi / 2 by taking
+// -U where cos(phi) < 0: a global sign the kernels drop (gate_flips, so the
+// caller can track the parity for the returned state vector).  The sign is taken
+// from the cosine and sine of phi itself, which the library reduces exactly:
+// a remainder modulo the rounded pi moves phi by 1.2e-16 per multiple (10 qubits,
+// 10 layers, angles within a period: gradient error 1.75e-15 against 1.3e-15; an
+// angle of 1e8: 2e-9).
 struct GateAB {
   double a, b;
 };
+static bool gate_flips(double angle, double sign) { return std::cos(sign * 0.5 * angle) < 0.0; }
+
 static GateAB gate_ab(double angle, double sign) {
-  const double phi = std::remainder(sign * 0.5 * angle, M_PI);
-  const double c = std::cos(phi), s = std::sin(phi);
+  const double phi = sign * 0.5 * angle;
+  const double c0 = std::cos(phi), s0 = std::sin(phi);
+  const double c = std::fabs(c0), s = c0 < 0.0 ? -s0 : s0;
   return {s / (1.0 + c), s};
+}
+
+static void set_gate(PassDesc& d, int lb, int axis, double angle, double sign) {
+  const GateAB g = gate_ab(angle, sign);
+  d.gtype[lb] = axis == 0 ? G_X : axis == 1 ? G_Y : G_Z;
+  d.ga[lb] = g.a;
+  d.gb[lb] = g.b;
 }
 
 // Pinned staging for per-call tables, grown as needed; the previous call's
