@@ -471,16 +471,16 @@ struct qg_plan {
   double* d_part = nullptr;
   int gmax = 1, nrows = 0;
   int* d_fin = nullptr;         // finalize table (see run_finalize)
-  int* h_fin = nullptr;         // pinned
+  int* h_fin = nullptr;         // pinned (see h_tabs)
   size_t fin_cap = 0;
   // capacities of the small tables (they only grow, so a plan re-laid out for
   // a shape no larger than one it held before allocates nothing)
-  int cap_n = 0;            // d_init (n + 1), h_tabs
+  int cap_n = 0;            // d_init (n + 1), the table at h_tabs
   int cap_terms = 0;        // d_terms, d_xy
   size_t cap_part = 0;      // d_part elements (rows x gmax)
   int cap_nout = 0;         // h_out
   size_t cap_fstate = 0;    // d_fstate bytes
-  char* h_tabs = nullptr;   // pinned staging of the initial-state table
+  char* h_tabs = nullptr;   // pinned staging of the initial-state table; h_out and h_fin lie behind it
   double* d_dot = nullptr;      // kObsBlocks
   PassDesc* d_desc = nullptr;
   int ndesc_cap = 0;
@@ -676,7 +676,7 @@ static int ensure_small(qg_plan* p, int ndesc, int nrows, int nout) {
   const bool grow_part = part > p->cap_part || !p->d_part;
   const bool grow_out = nout > p->cap_nout || !p->h_out;
   const bool grow_fin = fin > p->fin_cap || !p->d_fin;
-  const bool grow_desc = ndesc > p->ndesc_cap || !p->d_desc;
+  const bool grow_desc = ndesc > p->ndesc_cap;
   if (grow_n || grow_terms || grow_part || grow_out || grow_fin || grow_desc) {
     // the tables being replaced may still be read by queued work
     HIPCHK(hipStreamSynchronize(p->ctx->stream));
@@ -684,12 +684,9 @@ static int ensure_small(qg_plan* p, int ndesc, int nrows, int nout) {
   }
   if (grow_n) {
     (void)hipFree(p->d_init);
-    if (p->h_tabs) (void)hipHostFree(p->h_tabs);
     p->d_init = nullptr;
-    p->h_tabs = nullptr;
     p->cap_n = 0;
     HIPCHK(hipMalloc(&p->d_init, sizeof(double) * (n + 1)));
-    HIPCHK(hipHostMalloc(&p->h_tabs, sizeof(double) * (n + 1), hipHostMallocDefault));
     p->cap_n = n;
   }
   if (grow_terms) {
@@ -713,19 +710,25 @@ static int ensure_small(qg_plan* p, int ndesc, int nrows, int nout) {
   }
   if (grow_fin) {
     (void)hipFree(p->d_fin);
-    if (p->h_fin) (void)hipHostFree(p->h_fin);
-    p->d_fin = p->h_fin = nullptr;
+    p->d_fin = nullptr;
     p->fin_cap = 0;
     HIPCHK(hipMalloc(&p->d_fin, sizeof(int) * fin));
-    HIPCHK(hipHostMalloc(&p->h_fin, sizeof(int) * fin, hipHostMallocDefault));
     p->fin_cap = fin;
   }
-  if (grow_out) {
-    if (p->h_out) (void)hipHostFree(p->h_out);
+  if (grow_n || grow_out || grow_fin) {
+    // one pinned allocation for the three: a pair of hipHostMalloc and
+    // hipHostFree takes 24 us whatever the size, a small hipMalloc 1.3 us
+    const int out = std::max(std::max(1, nout), p->cap_nout);
+    if (p->h_tabs) (void)hipHostFree(p->h_tabs);
+    p->h_tabs = nullptr;
     p->h_out = nullptr;
+    p->h_fin = nullptr;
     p->cap_nout = 0;
-    HIPCHK(hipHostMalloc(&p->h_out, sizeof(double) * std::max(1, nout), hipHostMallocDefault));
-    p->cap_nout = nout;
+    HIPCHK(hipHostMalloc(&p->h_tabs, sizeof(double) * (p->cap_n + 1 + out) + sizeof(int) * p->fin_cap,
+                         hipHostMallocDefault));
+    p->h_out = (double*)p->h_tabs + p->cap_n + 1;
+    p->h_fin = (int*)(p->h_out + out);
+    p->cap_nout = out;
   }
   if (!p->d_dot) HIPCHK(hipMalloc(&p->d_dot, sizeof(double) * kObsBlocks));
   if (grow_desc) {
@@ -734,8 +737,8 @@ static int ensure_small(qg_plan* p, int ndesc, int nrows, int nout) {
     p->d_desc = nullptr;
     p->h_desc = nullptr;
     p->ndesc_cap = 0;
-    HIPCHK(hipMalloc(&p->d_desc, sizeof(PassDesc) * std::max(1, ndesc)));
-    HIPCHK(hipHostMalloc(&p->h_desc, sizeof(PassDesc) * std::max(1, ndesc), hipHostMallocDefault));
+    HIPCHK(hipMalloc(&p->d_desc, sizeof(PassDesc) * ndesc));
+    HIPCHK(hipHostMalloc(&p->h_desc, sizeof(PassDesc) * ndesc, hipHostMallocDefault));
     p->ndesc_cap = ndesc;
   }
   p->nout = nout;
@@ -1385,7 +1388,6 @@ static void free_small(qg_plan* p) {
   (void)hipFree(p->d_lut);
   (void)hipFree(p->d_part);
   (void)hipFree(p->d_fin);
-  if (p->h_fin) (void)hipHostFree(p->h_fin);
   (void)hipFree(p->d_dot);
   (void)hipFree(p->d_desc);
   (void)hipFree(p->d_sweep);
@@ -1399,7 +1401,6 @@ static void free_small(qg_plan* p) {
   p->h_turn = nullptr;
   p->turn_cap = 0;
   if (p->h_desc) (void)hipHostFree(p->h_desc);
-  if (p->h_out) (void)hipHostFree(p->h_out);
   if (p->h_arena) (void)hipHostFree(p->h_arena);
   if (p->h_stage) (void)hipHostFree(p->h_stage);
   if (p->h_cstage) (void)hipHostFree(p->h_cstage);
@@ -3216,7 +3217,7 @@ static int qaoa_layout(qg_plan* p) {
   p->off_lam = (size_t)p->chunk * NP * p->S;
   p->ws_bytes = p->off_lam + (size_t)p->chunk * 2 * p->S;
   p->gmax = grid_max(p);
-  const int ndesc = p->turn ? 1 : p->chunk * 2 * NP;
+  const int ndesc = p->turn ? 0 : p->chunk * 2 * NP;
   p->nrows = p->turn ? p->chunk * (3 * NP + 1) : p->chunk * (NP + 1) * (kMaxK + 1);
   if (p->turn) CHK(ensure_turn(p, p->chunk * 2 * NP));
   CHK(ensure_small(p, ndesc, p->nrows, p->chunk * (1 + 2 * L)));
