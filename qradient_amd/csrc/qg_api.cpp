@@ -133,6 +133,7 @@ struct qg_ctx {
   // pinned host mirror of the device scratch of qg_mcclean_grad_run_noalloc
   // (tables staged here, copied with one H2D; results copied back here)
   unsigned char* noalloc_host = nullptr;
+  SweepPlans sweeps;  // planned multi-layer passes
 };
 
 extern "C" int qg_ctx_create(int device, void* stream, qg_ctx** out) {
@@ -492,7 +493,7 @@ struct qg_plan {
   // multi-layer passes of a McClean plan (qg_sweep.hpp)
   std::vector<PlanPass> sweep;
   int sweep_rounds = 0;     // rounds of all of them
-  int sweep_for[6] = {0, 0, 0, 0, 0, 0};  // n, L, entangler, local bits, contiguous bits, steps it was planned for
+  SweepKey sweep_for{};     // what it was planned for
   SweepDesc* d_sweep = nullptr;
   SweepDesc* h_sweep = nullptr;
   int sweep_cap = 0;
@@ -1548,17 +1549,17 @@ static void plan_sweeps(qg_plan* p) {
     if (p->S <= kCachedState) c = 2;
   }
   const int steps = p->n >= 20 && p->S <= kCachedState && K == 12 && c == 2 ? 6 : 4;
-  const int key[6] = {p->n, p->L, p->ent, K, c, steps};
+  const SweepKey key = {p->n, p->L, p->ent == QG_ENT_CZ, K, c, steps};
   if (p->n <= kFusedMaxN || K < kSweepMinK || K > kSweepMaxK || c < 1 || K - c < 4) {
     p->sweep.clear();
     p->sweep_rounds = 0;
     return;
   }
-  if (p->sweep.empty() || !std::equal(key, key + 6, p->sweep_for)) {
-    p->sweep = SweepPlanner(p->n, p->L, p->ent == QG_ENT_CZ, K, c).plan(steps);
+  if (p->sweep.empty() || key != p->sweep_for) {
+    p->sweep = p->ctx->sweeps.get(key);
     p->sweep_rounds = 0;
     for (const PlanPass& s : p->sweep) p->sweep_rounds += (int)s.rounds.size();
-    std::copy(key, key + 6, p->sweep_for);
+    p->sweep_for = key;
   }
   // the layout holds one state per single-layer pass
   if (p->sweep.size() > p->geo.size() * (size_t)p->L) p->sweep.clear();

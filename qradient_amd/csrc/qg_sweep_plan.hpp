@@ -3,7 +3,11 @@
 // function of the circuit's shape, never of its angles.
 #pragma once
 #include <algorithm>
+#include <array>
 #include <cstdint>
+#include <list>
+#include <mutex>
+#include <utility>
 #include <vector>
 
 #include "qg_internal.h"
@@ -206,6 +210,52 @@ class SweepPlanner {
       s = q;
     }
   }
+};
+
+// What a planned circuit depends on: qubits, layers, CZ ladder (else CNOT), local
+// bits, contiguous bits, steps.
+typedef std::array<int, 6> SweepKey;
+
+// The plans last asked for, shared by the plans of a context: a plan that is laid
+// out for the shapes of a request stream, or made anew for a circuit of a known
+// shape, does not plan again (30 qubits, 100 layers 0.63 ms a layout, 24 qubits,
+// 40 layers 0.15 ms, against 0.02 ms without planning).  Holds at most kPlans
+// plans and kRounds rounds (4 MiB); safe to use from several threads.
+class SweepPlans {
+ public:
+  static constexpr size_t kPlans = 64, kRounds = 65536;
+
+  std::vector<PlanPass> get(const SweepKey& k) {
+    {
+      std::lock_guard<std::mutex> lock(m_);
+      for (auto it = held_.begin(); it != held_.end(); ++it)
+        if (it->first == k) {
+          held_.splice(held_.begin(), held_, it);
+          return it->second;
+        }
+    }
+    std::vector<PlanPass> p = SweepPlanner(k[0], k[1], k[2] != 0, k[3], k[4]).plan(k[5]);
+    std::lock_guard<std::mutex> lock(m_);
+    held_.emplace_front(k, p);
+    rounds_ += rounds_of(p);
+    while (held_.size() > kPlans || rounds_ > kRounds) {
+      rounds_ -= rounds_of(held_.back().second);
+      held_.pop_back();
+    }
+    return p;
+  }
+  size_t plans() const { return held_.size(); }
+  size_t rounds() const { return rounds_; }
+
+ private:
+  static size_t rounds_of(const std::vector<PlanPass>& p) {
+    size_t r = 0;
+    for (const PlanPass& s : p) r += s.rounds.size();
+    return r;
+  }
+  std::mutex m_;
+  std::list<std::pair<SweepKey, std::vector<PlanPass>>> held_;  // the last asked for first
+  size_t rounds_ = 0;
 };
 
 }  // namespace qg
