@@ -2539,7 +2539,8 @@ static int mcclean_batch_layout(qg_plan* p) {
   p->gmax = grid_max(p);
   const int ch = n > kFusedMaxN ? p->chunk : 1;
   p->nrows = ch * mcclean_rows(p);
-  CHK(ensure_small(p, ch * 2 * P * L, p->nrows, ch * (1 + L * n)));
+  // multi-layer passes: the observable's pass alone takes a PassDesc per circuit
+  CHK(ensure_small(p, p->sweep.empty() ? ch * 2 * P * L : ch, p->nrows, ch * (1 + L * n)));
   CHK(ensure_sweeps(p, ch));
   if (!ladder_shift_form(n, 1, &p->lad1, &p->lad2) || !ladder_shift_form(n, 0, &p->inv1, &p->inv2))
     return fail(QG_ERR_INVALID, "ladder map not in shift form");
