@@ -2446,7 +2446,17 @@ static int mcclean_run(qg_plan* p, const int32_t* axes, const double* angles, co
   if (streamed) CHK(stream_begin(p, std::max<size_t>(1, obs.diag.size())));
   std::vector<std::vector<int>> out_rows(grad ? 1 + L * n : 1);
   std::vector<int> cnt(p->nrows, 0);
-  const bool sweeps = !layered && !p->sweep.empty();
+  // A value alone, without x / y terms: the last single-layer pass also takes
+  // E, which multi-layer passes leave to one more read of the state.  That
+  // read shows from 2^25 amplitudes on where there are no fewer passes, or one
+  // fewer and the single-layer tile holds 13 bits.  run_expec_val, one layer,
+  // us, multi-layer | single-layer: complex64 25 qubits 508 | 434, 26 1058 |
+  // 955, 27 2093 | 2350, 28 4282 | 3646; complex128 25 749 | 725, 28 5615 |
+  // 5308, but 24 328 | 357.  Two layers, complex64: 29 qubits 14566 | 13462, 30
+  // 31423 | 31948; 27 qubits, tiles of 11 bits, 3322 | 4064.
+  const bool in_last = !grad && obs.xy.empty() && n >= 25 &&
+                       p->sweep.size() + (p->kmax_auto && p->kmax > 12) >= p->geo.size() * (size_t)L;
+  const bool sweeps = !layered && !in_last && !p->sweep.empty();
   if (sweeps) {
     p->state_sign = false;
     for (int k = 0; k < L * n; ++k) p->state_sign ^= gate_flips(angles[k], 1.0);
