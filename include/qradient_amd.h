@@ -72,7 +72,10 @@ const char* qg_last_error(void);
 int qg_version(void);
 
 /* Context: one HIP device and one stream (NULL: the library creates a
- * default-priority stream).  The stream argument is a hipStream_t. */
+ * default-priority stream).  The stream argument is a hipStream_t.
+ * qg_ctx_destroy gives up the caller's hold: plans and states made from the
+ * context stay valid, and it is freed with the last of them (a given
+ * stream must live as long). */
 int qg_ctx_create(int device, void* stream, qg_ctx** out);
 int qg_ctx_destroy(qg_ctx* ctx);
 int qg_ctx_synchronize(qg_ctx* ctx);

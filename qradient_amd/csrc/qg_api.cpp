@@ -4,6 +4,7 @@
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
+#include <atomic>
 #include <cmath>
 #include <cstdio>
 #include <cstring>
@@ -134,7 +135,26 @@ struct qg_ctx {
   // (tables staged here, copied with one H2D; results copied back here)
   unsigned char* noalloc_host = nullptr;
   SweepPlans sweeps;  // planned multi-layer passes
+  // the creator's reference and one per plan and state: these may be destroyed
+  // after qg_ctx_destroy (an interpreter that ends picks the order itself)
+  std::atomic<int> refs{1};
 };
+
+static qg_ctx* ctx_retain(qg_ctx* c) {
+  c->refs.fetch_add(1, std::memory_order_relaxed);
+  return c;
+}
+
+static void ctx_release(qg_ctx* c) {
+  if (c->refs.fetch_sub(1, std::memory_order_acq_rel) != 1) return;
+  (void)hipSetDevice(c->device);
+  if (c->stream) (void)hipStreamSynchronize(c->stream);
+  if (c->ev0) (void)hipEventDestroy(c->ev0);
+  if (c->ev1) (void)hipEventDestroy(c->ev1);
+  if (c->own_stream && c->stream) (void)hipStreamDestroy(c->stream);
+  if (c->noalloc_host) (void)hipHostFree(c->noalloc_host);
+  delete c;
+}
 
 extern "C" int qg_ctx_create(int device, void* stream, qg_ctx** out) {
   if (!out) return fail(QG_ERR_INVALID, "qg_ctx_create: out is NULL");
@@ -188,14 +208,7 @@ extern "C" int qg_ctx_create(int device, void* stream, qg_ctx** out) {
 }
 
 extern "C" int qg_ctx_destroy(qg_ctx* c) {
-  if (!c) return QG_OK;
-  (void)hipSetDevice(c->device);
-  if (c->stream) (void)hipStreamSynchronize(c->stream);
-  if (c->ev0) (void)hipEventDestroy(c->ev0);
-  if (c->ev1) (void)hipEventDestroy(c->ev1);
-  if (c->own_stream && c->stream) (void)hipStreamDestroy(c->stream);
-  if (c->noalloc_host) (void)hipHostFree(c->noalloc_host);
-  delete c;
+  if (c) ctx_release(c);
   return QG_OK;
 }
 
@@ -755,6 +768,7 @@ extern "C" int qg_plan_destroy(qg_plan* p) {
   drop_graph(p);
   for (auto& set : p->prof_ev)
     for (hipEvent_t e : set) (void)hipEventDestroy(e);
+  ctx_release(p->ctx);
   delete p;
   return QG_OK;
 }
@@ -1637,7 +1651,7 @@ extern "C" int qg_mcclean_plan(qg_ctx* ctx, int n, int L, int dtype, int entangl
   if (ckpt_every < QG_HISTORY) return fail(QG_ERR_INVALID, "ckpt_every must be >= 0 or QG_HISTORY");
   HIPCHK(hipSetDevice(ctx->device));
   qg_plan* p = new qg_plan();
-  p->ctx = ctx;
+  p->ctx = ctx_retain(ctx);
   p->kind = PK_MCCLEAN;
   p->n = n;
   p->L = L;
@@ -2571,7 +2585,7 @@ extern "C" int qg_mcclean_batch_plan(qg_ctx* ctx, int n, int L, int dtype, int e
   if (batch < 1) return fail(QG_ERR_INVALID, "batch must be >= 1");
   HIPCHK(hipSetDevice(ctx->device));
   qg_plan* p = new qg_plan();
-  p->ctx = ctx;
+  p->ctx = ctx_retain(ctx);
   p->kind = PK_MCCLEAN;
   p->n = n;
   p->L = L;
@@ -3260,7 +3274,7 @@ extern "C" int qg_qaoa_plan(qg_ctx* ctx, int n, int p_layers, int dtype, int bat
   if (batch < 1) return fail(QG_ERR_INVALID, "batch must be >= 1");
   HIPCHK(hipSetDevice(ctx->device));
   qg_plan* p = new qg_plan();
-  p->ctx = ctx;
+  p->ctx = ctx_retain(ctx);
   p->kind = PK_QAOA;
   p->n = n;
   p->L = p_layers;
@@ -4096,6 +4110,7 @@ extern "C" int qg_state_destroy(qg_state* s) {
   (void)hipFree(s->d_xy);
   (void)hipFree(s->d_tab);
   (void)hipFree(s->d_dot);
+  ctx_release(s->ctx);
   delete s;
   return QG_OK;
 }
@@ -4107,7 +4122,7 @@ extern "C" int qg_state_create(qg_ctx* ctx, int n, int dtype, char ini, qg_state
   if (ini != '0' && ini != '+') return fail(QG_ERR_INVALID, std::string("Invalid initialization format ") + ini + ".");
   HIPCHK(hipSetDevice(ctx->device));
   qg_state* s = new qg_state();
-  s->ctx = ctx;
+  s->ctx = ctx_retain(ctx);
   s->n = n;
   s->dtype = dtype;
   s->max_terms = std::max(64, n * n);
