@@ -20,9 +20,19 @@
 // phase.  The circuit's last pass forms lambda = D psi itself.  psi is never
 // stored.
 //
+// A complex64 forward pass moves FP64 real parts through its 8-byte slots and
+// then the imaginary parts (see qg_sweep.hpp), so psi is rounded where it is
+// stored and nowhere else.  With FP32 exchanges E and the gradients of 15 qubits
+// and 2 or 3 layers were less accurate than one layer at a time.  Error against
+// complex128, 16 graphs, root mean square, one layer at a time | FP32 exchanges |
+// now: E of 15 qubits, 2 layers, 6.4e-9 | 8.0e-9 | 4.1e-9, its gradient 1.14e-8 |
+// 2.81e-8 | 1.38e-8; gradient of 20 qubits, 8 layers 9.1e-9 | 7.7e-9 | 6.7e-9, of
+// 20 qubits, 30 layers 2.8e-7 | 1.9e-7 | 1.6e-7.  It costs 1 to 3% of a gradient
+// run (256 circuits of 20 qubits, 8 layers 32.1 -> 32.5 ms).
+//
 // Bound: the vector ALU (gates, reductions, and the FP64 <-> FP32 conversions
 // of the exchanges), then HBM: 84 GB of states would take 18 ms at the copy
-// rate.  256 circuits of 20 qubits, 8 layers, complex64: 46.5 -> 32.0 ms (9 + 9
+// rate.  256 circuits of 20 qubits, 8 layers, complex64: 46.5 -> 32.5 ms (9 + 9
 // passes instead of 16 + 16); one circuit of 17 qubits, 6 layers, complex128,
 // real weights: 541 -> 251 us.
 #pragma once
@@ -45,6 +55,7 @@ __device__ __forceinline__ void run_turn(const TurnDesc* __restrict__ d, void* l
   constexpr int GSH = sizeof(G) == 4 ? 3 : 4;
   constexpr int SH = sizeof(LT) == 4 ? 3 : 4;
   constexpr bool PF = !TWO;  // the next tile's loads in flight while this one is worked on
+  constexpr bool HALVES = SH == 3 && !TWO;  // FP64 halves of an amplitude through its 8-byte slot (see above)
   warm_lines<(int)sizeof(TurnDesc)>(d);
   const int n = d->n, K = d->K, t = d->t, c = d->c, p = d->p;
   const uint32_t flags = d->flags;
@@ -164,7 +175,20 @@ __device__ __forceinline__ void run_turn(const TurnDesc* __restrict__ d, void* l
       uint32_t bw = lds_addr(lds) + (swz<LT>(lidx<R>(tid, 0, lo)) << SH);
       uint32_t br = lds_addr(lds) + (swz<LT>(lidx<R>(tid, 0, ldc(&rd->lo, 0))) << SH);
       asm volatile("" : "+v"(bw), "+v"(br));  // opaque (see lds_transpose)
-      if constexpr (decltype(with_a)::value) {
+      if constexpr (HALVES) {
+        // real parts, then imaginary parts, unrounded, through the same slots
+        auto half = [&](double Cd::*part) __attribute__((always_inline)) {
+#pragma unroll
+          for (int a = 0; a < A; ++a) lds_st_d(bw ^ wo[a], xa[a].*part);
+          barrier();
+#pragma unroll
+          for (int a = 0; a < A; ++a) xa[a].*part = lds_ld_d(br ^ ro[a]);
+        };
+        half(&Cd::re);
+        barrier();
+        asm volatile("" : "+v"(bw), "+v"(br));  // opaque again: shared addresses would all stay live
+        half(&Cd::im);
+      } else if constexpr (decltype(with_a)::value) {
 #pragma unroll
         for (int a = 0; a < A; ++a) Stor<LT>::lds_st_a(bw ^ wo[a], xa[a]);
         barrier();
