@@ -298,7 +298,7 @@ int qg_plan_pass_times(const qg_plan* plan, int cap, float* ms, int* kinds, int*
  * smallest kmax (>= 11 for QG_C64, >= 12 for QG_C128) that keeps it, 13 for
  * QG_C64 states of 4 GiB and more (n >= 29). */
 int qg_plan_tune(qg_plan* plan, int kmax, int cmin, int r_fwd, int r_rev);
-/* on = 1 (default): circuits with n <= kmax run whole in one workgroup each
+/* on = 1 (default): circuits with n <= 13 run whole in one workgroup each
  * (one launch per call, FP64 throughout); on = 0 uses the pass kernels. */
 int qg_plan_set_fused(qg_plan* plan, int on);
 /* on = 1: a run's pass launches are captured once as a HIP graph and
@@ -315,7 +315,8 @@ int qg_plan_set_graph(qg_plan* plan, int on);
  * FP64 in the forward passes and FP32 in the adjoint passes, -1 (default)
  * picks 2 when the circuit has more than 200 passes of one layer, else 0.
  * Forward passes of several layers (qg_plan_tune) round only when they store,
- * except in mode 0 when it is asked for.  The plan is laid out again.  qg_plan_lds64 returns the mode in effect (0, 1 or 2).
+ * except in mode 0 when it is asked for.  The plan is laid out again.
+ * qg_plan_lds64 returns the mode in effect (0, 1 or 2).
  * No counterpart in the reference (complex128 only). */
 int qg_plan_set_lds64(qg_plan* plan, int mode);
 int qg_plan_lds64(const qg_plan* plan, int* out);

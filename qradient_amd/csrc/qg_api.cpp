@@ -799,10 +799,6 @@ extern "C" int qg_plan_last_ms(const qg_plan* p, double* ms) {
   return QG_OK;
 }
 
-// prob[k] = <v|(I + P_k)/2|v> = |P_k^+ v|^2 for each term, in the given order
-// (weights ignored): the probability of the +1 outcome that the projectors of
-// observable.py:126-177 give in base.py:22-46, also for a state whose norm is
-// not exactly 1.  One pass over v per 32 diagonal or 16 other terms.
 // The term table of the term-expectation kernel: terms[0, nterms) in order,
 // then the identity (|v|^2).
 static int pterm_table(int n, const qg_term* terms, int nterms, std::vector<PTerm>& h) {
@@ -834,7 +830,7 @@ static int pterm_table(int n, const qg_term* terms, int nterms, std::vector<PTer
 }
 
 // e[k] = <v|P_k|v> for the terms in order, e[nterms] = |v|^2 (weights
-// ignored).  One pass over v per 32 diagonal or 16 other terms.
+// ignored).  One pass over v per 24 diagonal or 16 other terms.
 static int term_expec(qg_ctx* c, int dtype, const void* v, int n, const qg_term* terms, int nterms, double* e) {
   std::vector<PTerm> h;
   CHK(pterm_table(n, terms, nterms, h));
@@ -1457,9 +1453,9 @@ constexpr double kPlanMemFraction = 0.75;
 
 // Whether the automatic FP64-tile rule (circuits of more than 200 passes)
 // covers the adjoint passes as well as the forward passes.  Measured at 30
-// qubits, 100 layers, checkpoints every 5 layers: FP64 tiles everywhere 5.78 s
-// and 6.2e-7 gradient error against complex128, forward only 5.44 s and 7.9e-7,
-// none 5.42 s and 1.1e-6.  The forward roundings dominate the error.
+// qubits, 100 layers, checkpoints every 5 layers: FP64 tiles everywhere 2.85 s
+// and 3.7e-7 gradient error against complex128, forward only 2.61 s and 6.6e-7,
+// none 2.54 s and 1.1e-6.  The forward roundings dominate the error.
 constexpr bool kLds64Adjoint = false;
 
 static int plan_budget(qg_plan* p, size_t* budget) {
@@ -4340,7 +4336,6 @@ extern "C" int qg_state_scale(qg_state* s, double re, double im) {
   return QG_OK;
 }
 
-// Lays a McClean plan out again after a change of its shape parameters.
 // Lays a McClean plan out again (new shape or tile options).  An owned
 // workspace too small for the new layout is freed (the next run allocates);
 // a supplied one is detached when detach_small is set, else it is an error.
